@@ -616,6 +616,15 @@ void to_caller(const sc_system *h, const std::vector<int64_t> &map, const T *src
 // one stress slot, whatever launch shape is set while the sum accumulates.
 int64_t stress_slots(int64_t nb) { return nb / 64 + 2; }
 
+// Scratch between steps: the rebuild's run slabs (kRunSlab * 8 bytes per
+// bond), which only the launches between the degree and the list pass of one
+// rebuild use.  Every filament has at least two bonds, so it holds three
+// FP64 components of every site, or six of every filament.
+double *idle_scratch(const sc_system *h) { return reinterpret_cast<double *>(h->d.nrun); }
+size_t idle_scratch_bytes(const sc_system *h) {
+  return sizeof(int2) * sc::kRunSlab * (size_t)h->g.nb;
+}
+
 int fetch_mapped(sc_system *h, const double *dev, double *out, int64_t n, int comp,
                  bool sites) {
   std::vector<double> tmp((size_t)comp * n);
@@ -963,7 +972,7 @@ size_t system_estimate_bytes(const sc_params *params, int32_t nf, int64_t ns, in
   const int64_t n_cells = n1d * n1d * n1d;
   const int64_t nb = ns - nf;
   auto R = [](int64_t n) { return Arena::round((size_t)(n > 0 ? n : 1)); };
-  size_t b = R(sizeof(Ctl)) + R(8 * sc::kDrSlots) + R(4 * (nf + 1)) + R(4 * (int64_t)nf) +
+  size_t b = R(sizeof(Ctl)) + R(8 * sc::kDrSlots) + R(4 * (nf + 1)) + 2 * R(4 * (int64_t)nf) +
              R(64 * (int64_t)nf) +
              R(8 * (int64_t)nf) + R(4 * nb);
   b += 4 * R(24 * ns) + 2 * R(8 * ns);                    // r, rp, fr, dr0, acc, acc_prev
@@ -1150,6 +1159,7 @@ int sc_load_filaments(sc_handle h, int32_t nf, const int32_t *site_off,
                            h->stream));
   if ((rc = dalloc(h, &d.site_off, nf + 1, false))) return rc;
   if ((rc = dalloc(h, &d.noise_off, nf, false))) return rc;
+  if ((rc = dalloc(h, &d.fil_caller, nf, false))) return rc;
   if ((rc = dalloc(h, &d.fpar, 8 * (size_t)nf, false))) return rc;
   if ((rc = dalloc(h, &d.norm, 2 * (size_t)nf, false))) return rc;
   if ((rc = dalloc(h, &d.bond_fil, nb, false))) return rc;
@@ -1215,6 +1225,9 @@ int sc_load_filaments(sc_handle h, int32_t nf, const int32_t *site_off,
   }
   HIPCHK(h, hipMemcpyAsync(d.site_off, site_off, sizeof(int32_t) * (nf + 1), hipMemcpyHostToDevice, h->stream));
   HIPCHK(h, hipMemcpyAsync(d.noise_off, noise_off.data(), sizeof(int32_t) * nf, hipMemcpyHostToDevice, h->stream));
+  std::vector<int32_t> fil_caller(nf);
+  for (int f = 0; f < nf; ++f) fil_caller[f] = h->reordered ? h->perm[f] : f;
+  HIPCHK(h, hipMemcpyAsync(d.fil_caller, fil_caller.data(), sizeof(int32_t) * nf, hipMemcpyHostToDevice, h->stream));
   HIPCHK(h, hipMemcpyAsync(d.fpar, fpar.data(), sizeof(double) * fpar.size(), hipMemcpyHostToDevice, h->stream));
   HIPCHK(h, hipMemcpyAsync(d.norm, norm.data(), sizeof(int32_t) * norm.size(), hipMemcpyHostToDevice, h->stream));
   HIPCHK(h, hipMemcpyAsync(d.bond_fil, bond_fil.data(), sizeof(int32_t) * nb, hipMemcpyHostToDevice, h->stream));
@@ -1826,25 +1839,19 @@ int sc_filament_stats(sc_handle h, double *e2e, double *com) {
   if (rc) return rc;
   if (!e2e && !com) return SC_OK;
   const int64_t n = 3 * (int64_t)h->g.nf;
-  double *buf = nullptr;
-  HIPCHK(h, hipMalloc(&buf, sizeof(double) * 2 * n));
+  double *buf = idle_scratch(h);
+  if (sizeof(double) * 2 * n > idle_scratch_bytes(h))
+    return fail(h, SC_ERR_STATE, "statistics scratch too small");
   HIPCHK(h, hipStreamSynchronize(h->stream));
   refresh_records(h);
-  sc::launch_filament_stats(h->d, h->g, buf, buf + n, h->stream);
-  std::vector<double> tmp(2 * (size_t)n);
-  hipError_t e = hipMemcpyAsync(tmp.data(), buf, sizeof(double) * 2 * n, hipMemcpyDeviceToHost,
-                                h->stream);
-  if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
-  (void)hipFree(buf);
-  if (e != hipSuccess) return fail(h, SC_ERR_HIP, std::string("sc_filament_stats: ") +
-                                                      hipGetErrorString(e));
-  const int64_t nf = h->g.nf;
-  for (int k = 0; k < 3; ++k)
-    for (int64_t f = 0; f < nf; ++f) {
-      const int64_t u = h->reordered ? h->perm[f] : f;
-      if (e2e) e2e[k * nf + u] = tmp[k * nf + f];
-      if (com) com[k * nf + u] = tmp[n + k * nf + f];
-    }
+  // results in the caller's filament order, copied into the caller's memory
+  sc::launch_filament_stats(h->d, h->g, e2e ? buf : nullptr, com ? buf + n : nullptr, h->stream);
+  HIPCHK(h, hipGetLastError());
+  if (e2e)
+    HIPCHK(h, hipMemcpyAsync(e2e, buf, sizeof(double) * n, hipMemcpyDeviceToHost, h->stream));
+  if (com)
+    HIPCHK(h, hipMemcpyAsync(com, buf + n, sizeof(double) * n, hipMemcpyDeviceToHost, h->stream));
+  HIPCHK(h, hipStreamSynchronize(h->stream));
   return SC_OK;
 }
 
@@ -1853,19 +1860,22 @@ int sc_theta_histogram(sc_handle h, int32_t n_bins, int32_t n_rows, int64_t *his
   if (rc) return rc;
   if (n_bins <= 0 || n_rows <= 0 || !hist) return fail(h, SC_ERR_ARG, "bad histogram shape");
   const size_t n = (size_t)n_bins * (size_t)n_rows;
-  unsigned long long *buf = nullptr;
-  HIPCHK(h, hipMalloc(&buf, sizeof(unsigned long long) * n));
+  HIPCHK(h, hipStreamSynchronize(h->stream));
+  refresh_records(h);
+  // counters in the idle rebuild scratch; shapes beyond it take a buffer of
+  // their own (allocated and freed here, which waits for the whole device)
+  const bool own = sizeof(unsigned long long) * n > idle_scratch_bytes(h);
+  unsigned long long *buf = reinterpret_cast<unsigned long long *>(idle_scratch(h));
+  if (own) HIPCHK(h, hipMalloc(&buf, sizeof(unsigned long long) * n));
   std::vector<unsigned long long> host(n);
-  hipError_t e = hipMemsetAsync(buf, 0, sizeof(unsigned long long) * n, h->stream);
-  if (e == hipSuccess) {
-    HIPCHK(h, hipStreamSynchronize(h->stream));
-    refresh_records(h);
-    sc::launch_theta_hist(h->d, h->g, n_bins, n_rows, buf, h->stream);
+  sc::launch_zero_i32(reinterpret_cast<int32_t *>(buf), 2 * (int64_t)n, h->stream);
+  sc::launch_theta_hist(h->d, h->g, n_bins, n_rows, buf, h->stream);
+  hipError_t e = hipGetLastError();
+  if (e == hipSuccess)
     e = hipMemcpyAsync(host.data(), buf, sizeof(unsigned long long) * n, hipMemcpyDeviceToHost,
                        h->stream);
-  }
   if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
-  (void)hipFree(buf);
+  if (own) (void)hipFree(buf);
   if (e != hipSuccess) return fail(h, SC_ERR_HIP, std::string("sc_theta_histogram: ") +
                                                       hipGetErrorString(e));
   for (size_t k = 0; k < n; ++k) hist[k] += (int64_t)host[k];

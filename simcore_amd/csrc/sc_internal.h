@@ -87,6 +87,7 @@ struct Dev {
   // filaments
   int32_t *site_off;       // nf+1
   int32_t *noise_off;      // nf: site index the noise stream is keyed by
+  int32_t *fil_caller;     // nf: the caller's index of the filament
   double *fpar;            // nf*8: bl, kappa, gpar, gperp, sig_par, sig_perp, diam, 0
   int32_t *norm;           // nf*2: normalize_switch_, n_normalize_
   int32_t *bond_fil;       // nb
