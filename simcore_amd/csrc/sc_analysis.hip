@@ -100,6 +100,23 @@ __global__ __launch_bounds__(256) void k_theta_hist_lds(Dev d, Geo g, int n_bins
     if (cnt[i]) atomicAdd(&hist[i], (unsigned long long)cnt[i]);
 }
 
+// Storage-order array (n entries per component, sites or bonds of every
+// filament) to the caller's order in FP64: kFilLanes lanes per filament, both
+// sides in coalesced runs.  Bound: one read and one write of the array.
+template <typename T>
+__global__ __launch_bounds__(256) void k_caller_order(Dev d, Geo g, const T *__restrict__ src,
+                                                      double *__restrict__ dst, int64_t n,
+                                                      int comp, int bonds) {
+  const int f = blockIdx.x * (256 / kFilLanes) + (int)threadIdx.x / kFilLanes;
+  const int gl = threadIdx.x % kFilLanes;
+  if (f >= g.nf) return;
+  const int64_t s0 = d.site_off[f] - (bonds ? f : 0);
+  const int64_t len = d.site_off[f + 1] - d.site_off[f] - bonds;
+  const int64_t t0 = d.noise_off[f] - (bonds ? d.fil_caller[f] : 0);
+  for (int k = 0; k < comp; ++k)
+    for (int64_t i = gl; i < len; i += kFilLanes) dst[k * n + t0 + i] = (double)src[k * n + s0 + i];
+}
+
 inline dim3 fil_grid(int nf) {
   const int per = 256 / kFilLanes, b = (nf + per - 1) / per;
   return dim3((unsigned)(b > 0 ? b : 1));
@@ -122,6 +139,16 @@ void launch_theta_hist(const Dev &d, const Geo &g, int n_bins, int n_rows,
   else
     hipLaunchKernelGGL(k_theta_hist, dim3((unsigned)blocks), dim3(256), 0, st, d, g, n_bins,
                        n_rows, hist);
+}
+
+void launch_caller_order(const Dev &d, const Geo &g, const void *src, bool f32, double *dst,
+                         int64_t n, int comp, bool bonds, hipStream_t st) {
+  if (f32)
+    hipLaunchKernelGGL(k_caller_order<float>, fil_grid(g.nf), dim3(256), 0, st, d, g,
+                       static_cast<const float *>(src), dst, n, comp, bonds ? 1 : 0);
+  else
+    hipLaunchKernelGGL(k_caller_order<double>, fil_grid(g.nf), dim3(256), 0, st, d, g,
+                       static_cast<const double *>(src), dst, n, comp, bonds ? 1 : 0);
 }
 
 }  // namespace sc

@@ -611,7 +611,6 @@ void to_caller(const sc_system *h, const std::vector<int64_t> &map, const T *src
     for (int64_t i = 0; i < n; ++i) dst[k * n + map[i]] = src[k * n + i];
 }
 
-// device SoA site/bond array -> caller-order host array
 // Blocks of the pair pass at its smallest block size (64 bonds): each owns
 // one stress slot, whatever launch shape is set while the sum accumulates.
 int64_t stress_slots(int64_t nb) { return nb / 64 + 2; }
@@ -625,11 +624,40 @@ size_t idle_scratch_bytes(const sc_system *h) {
   return sizeof(int2) * sc::kRunSlab * (size_t)h->g.nb;
 }
 
-int fetch_mapped(sc_system *h, const double *dev, double *out, int64_t n, int comp,
+// Reordered or FP32 arrays of at least this many values are put into the
+// caller's order and precision by a kernel, whose launch costs a few
+// microseconds; below it the host's loop is cheaper (992 sites: 21 us on the
+// host; 1.66M sites: 13.5 ms on the host against the copy alone).
+constexpr int64_t kDeviceOrderMin = 16384;
+
+// device SoA site/bond array (storage order) -> caller-order FP64 host array,
+// the stream idle.  Arrays already in the caller's order and precision are
+// copied straight into the caller's memory.
+int fetch_mapped(sc_system *h, const void *dev, bool f32, double *out, int64_t n, int comp,
                  bool sites) {
-  std::vector<double> tmp((size_t)comp * n);
-  HIPCHK(h, hipMemcpy(tmp.data(), dev, sizeof(double) * tmp.size(), hipMemcpyDeviceToHost));
-  to_caller(h, sites ? h->site_map : h->bond_map, tmp.data(), out, n, comp);
+  const size_t count = (size_t)comp * n;
+  if (h->reordered || f32) {
+    if ((int64_t)count < kDeviceOrderMin) {
+      std::vector<double> wide(count);
+      if (f32) {
+        std::vector<float> v32(count);
+        HIPCHK(h, hipMemcpy(v32.data(), dev, sizeof(float) * count, hipMemcpyDeviceToHost));
+        wide.assign(v32.begin(), v32.end());
+      } else {
+        HIPCHK(h, hipMemcpy(wide.data(), dev, sizeof(double) * count, hipMemcpyDeviceToHost));
+      }
+      to_caller(h, sites ? h->site_map : h->bond_map, wide.data(), out, n, comp);
+      return SC_OK;
+    }
+    double *tmp = idle_scratch(h);
+    if (sizeof(double) * count > idle_scratch_bytes(h))
+      return fail(h, SC_ERR_STATE, "getter scratch too small");
+    sc::launch_caller_order(h->d, h->g, dev, f32, tmp, n, comp, !sites, h->stream);
+    HIPCHK(h, hipGetLastError());
+    dev = tmp;
+  }
+  HIPCHK(h, hipMemcpyAsync(out, dev, sizeof(double) * count, hipMemcpyDeviceToHost, h->stream));
+  HIPCHK(h, hipStreamSynchronize(h->stream));
   return SC_OK;
 }
 
@@ -1505,19 +1533,11 @@ int sc_get_sites(sc_handle h, double *r, double *r_prev, double *f_rand) {
   int rc = check_handle(h, true);
   if (rc) return rc;
   HIPCHK(h, hipStreamSynchronize(h->stream));
-  if (r && (rc = fetch_mapped(h, h->d.r, r, h->g.ns, 3, true))) return rc;
-  if (r_prev && (rc = fetch_mapped(h, h->d.rp, r_prev, h->g.ns, 3, true))) return rc;
-  if (f_rand) {
-    if (h->g.compact) {  // mixed precision: FP32 random forces
-      const int64_t ns = h->g.ns;
-      std::vector<float> tmp(3 * (size_t)ns);
-      HIPCHK(h, hipMemcpy(tmp.data(), h->d.fr, sizeof(float) * tmp.size(), hipMemcpyDeviceToHost));
-      std::vector<double> wide(tmp.begin(), tmp.end());
-      to_caller(h, h->site_map, wide.data(), f_rand, ns, 3);
-    } else if ((rc = fetch_mapped(h, h->d.fr, f_rand, h->g.ns, 3, true))) {
-      return rc;
-    }
-  }
+  if (r && (rc = fetch_mapped(h, h->d.r, false, r, h->g.ns, 3, true))) return rc;
+  if (r_prev && (rc = fetch_mapped(h, h->d.rp, false, r_prev, h->g.ns, 3, true))) return rc;
+  // (mixed precision: FP32 random forces)
+  if (f_rand && (rc = fetch_mapped(h, h->d.fr, h->g.compact != 0, f_rand, h->g.ns, 3, true)))
+    return rc;
   return SC_OK;
 }
 
@@ -1592,15 +1612,10 @@ int sc_get_bond_forces(sc_handle h, double *f, double *t) {
   for (int which = 0; which < 2; ++which) {
     double *out = which == 0 ? f : t;
     if (!out) continue;
-    if (d.bf) {
-      if ((rc = fetch_mapped(h, which == 0 ? d.bf : d.bt, out, nb, 3, false))) return rc;
-    } else {  // mixed precision: FP32 sums widened to FP64
-      std::vector<float> v32(3 * (size_t)nb);
-      HIPCHK(h, hipMemcpy(v32.data(), which == 0 ? d.bf32 : d.bt32, sizeof(float) * v32.size(),
-                          hipMemcpyDeviceToHost));
-      std::vector<double> v(v32.begin(), v32.end());
-      to_caller(h, h->bond_map, v.data(), out, nb, 3);
-    }
+    // (mixed precision: FP32 sums widened to FP64)
+    const void *src = d.bf ? (const void *)(which == 0 ? d.bf : d.bt)
+                           : (const void *)(which == 0 ? d.bf32 : d.bt32);
+    if ((rc = fetch_mapped(h, src, !d.bf, out, nb, 3, false))) return rc;
   }
   return SC_OK;
 }
@@ -1610,7 +1625,7 @@ int sc_get_tensions(sc_handle h, double *tension) {
   if (rc) return rc;
   if (!tension) return fail(h, SC_ERR_ARG, "null output");
   HIPCHK(h, hipStreamSynchronize(h->stream));
-  return fetch_mapped(h, h->d.tension, tension, h->g.nb, 1, false);
+  return fetch_mapped(h, h->d.tension, false, tension, h->g.nb, 1, false);
 }
 
 int sc_thermo_enable(sc_handle h, int on) {
@@ -1676,7 +1691,7 @@ int sc_get_bond_energies(sc_handle h, double *pote) {
   if (!pote) return fail(h, SC_ERR_ARG, "null output");
   if (!h->g.thermo) return fail(h, SC_ERR_STATE, "thermodynamics not enabled");
   HIPCHK(h, hipStreamSynchronize(h->stream));
-  return fetch_mapped(h, h->d.bpote, pote, h->g.nb, 1, false);
+  return fetch_mapped(h, h->d.bpote, false, pote, h->g.nb, 1, false);
 }
 
 int sc_get_cell_keys(sc_handle h, int32_t *keys) {
@@ -1753,7 +1768,7 @@ int sc_get_dr_state(sc_handle h, double *acc) {
   if (rc) return rc;
   if (!acc) return fail(h, SC_ERR_ARG, "null output");
   HIPCHK(h, hipStreamSynchronize(h->stream));
-  return fetch_mapped(h, h->d.acc, acc, h->g.ns, 1, true);
+  return fetch_mapped(h, h->d.acc, false, acc, h->g.ns, 1, true);
 }
 
 int sc_get_counters(sc_handle h, int64_t *i_step, int64_t *n_rebuilds,

@@ -301,6 +301,10 @@ void launch_filament_stats(const Dev &d, const Geo &g, double *e2e, double *com,
                            hipStream_t st);
 void launch_theta_hist(const Dev &d, const Geo &g, int n_bins, int n_rows,
                        unsigned long long *hist, hipStream_t st);
+// `comp` components of n sites or bonds each, storage order (FP64 or FP32)
+// into FP64 caller order
+void launch_caller_order(const Dev &d, const Geo &g, const void *src, bool f32, double *dst,
+                         int64_t n, int comp, bool bonds, hipStream_t st);
 void launch_zero_i32(int32_t *p, int64_t n, hipStream_t st);
 void launch_redo_dr(const Dev &d, const Geo &g, hipStream_t st);
 void launch_copy_probe(const void *src, void *dst, int64_t n32, hipStream_t st);

@@ -22,6 +22,47 @@ def _straight(lengths, seed, box):
     return out
 
 
+# 3 values per site, 16384 the size from which the device reorders
+@pytest.mark.parametrize("ns_min", [30, 5300, 5600, 40000])
+@pytest.mark.parametrize("spatial", [False, True])
+def test_read_back_is_in_the_callers_order(ns_min, spatial):
+    rng = np.random.default_rng(ns_min)
+    lengths = [3, 256, 17, 16, 15, 129, 128]
+    while sum(lengths) < ns_min:
+        lengths.append(int(rng.integers(3, 60)))
+    rng.shuffle(lengths)
+    box = 400.0
+    p = sc.params_init(box / 2, delta=1e-5, min_cell_length=4.0, seed=5)
+    fil = make_filaments(_straight(lengths, ns_min, box))
+    s = sc.FilamentSystem(p, fil, precision="mixed", spatial_order=spatial)
+    r, rp, fr = s.sites()
+    np.testing.assert_array_equal(r, fil.r)
+    np.testing.assert_array_equal(rp, fil.r)
+    assert not fr.any()
+    # the end-to-end vectors are differences of positions, the centres sums
+    # of at most 256 of them: 256 roundings of the largest
+    e2e, com = s.filament_stats()
+    x = fil.r.reshape(3, -1)
+    off = fil.site_off
+    np.testing.assert_array_equal(e2e, x[:, off[1:] - 1] - x[:, off[:-1]])
+    want = np.add.reduceat(x, off[:-1], axis=1) / np.diff(off)
+    np.testing.assert_allclose(com, want, rtol=0, atol=256 * 2.0 ** -52 * np.abs(x).max())
+    # moved positions, per-bond values and random forces against the same
+    # system in the caller's storage order
+    ref = sc.FilamentSystem(p, fil, precision="mixed", spatial_order=False)
+    for q in (s, ref):
+        q.step(1)
+    for a, b in zip(s.sites(), ref.sites()):
+        # the packed lanes round alike in either order: no pair interacts
+        np.testing.assert_array_equal(a, b)
+    np.testing.assert_array_equal(s.tensions(), ref.tensions())
+    np.testing.assert_array_equal(s.dr_state(), ref.dr_state())
+    for a, b in zip(s.bond_forces(), ref.bond_forces()):
+        np.testing.assert_allclose(a, b, rtol=0, atol=1e-5 * max(1.0, np.abs(b).max()))
+    s.close()
+    ref.close()
+
+
 # 8192 counters fit a block's local memory
 @pytest.mark.parametrize("precision", ["fp64", "mixed"])
 def test_theta_histogram_paths_agree(precision):
