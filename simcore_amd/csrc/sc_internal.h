@@ -249,6 +249,7 @@ constexpr int kScanItems = 8;
 // grid cap of streaming and scan passes (they loop over their range)
 constexpr int kStreamBlocks = 1024;
 constexpr int kScanTile = kScanBlock * kScanItems;
+constexpr int kPullGroup = 256;  // bonds whose lists a block of the list pass writes at a time
 
 enum Guard { kGuardStep = 0, kGuardRebuild = 1, kGuardXlink = 2 };
 
@@ -315,6 +316,6 @@ void launch_redo_dr(const Dev &d, const Geo &g, hipStream_t st);
 void launch_copy_probe(const void *src, void *dst, int64_t n32, hipStream_t st);
 void launch_scan(const int32_t *in, int32_t *out, int64_t n, int32_t *tmp,
                  const Ctl *ctl, int guard, hipStream_t st);
-int64_t scan_tmp_elems(int64_t n);
+int64_t scan_tmp_elems(int64_t ncol, int64_t nb);
 
 }  // namespace sc

@@ -9,8 +9,8 @@
 // One step, in stream order (all guarded by the device control block,
 // which holds the decision for the step about to run):
 //   [rebuild: keys (+ column populations), column scan, column scatter,
-//    column rank sort (+ cell runs, occupancy), degrees, degree scan,
-//    incidence lists (+ capacity, zero dr)]
+//    column rank sort (+ cell runs, occupancy), degrees, degree sums,
+//    incidence lists (+ incidence starts, capacity, zero dr)]
 //   -> pair+scatter -> integrate (per length class)
 //   -> commit (and decide the next step)
 #include <hip/hip_runtime.h>
@@ -254,7 +254,15 @@ __global__ __launch_bounds__(kScanBlock) void k_scan_down(const int32_t *in,
   scan_down_body(in, n, bsum, out, blockIdx.x, gridDim.x);
 }
 
-int64_t scan_tmp_elems(int64_t n) { return (n + kScanTile - 1) / kScanTile + 1; }
+// entries of Dev::scan_tmp: tile sums of a two-launch scan over the columns
+// or the bonds, or the degree sums of the list pass
+int64_t scan_tmp_elems(int64_t ncol, int64_t nb) {
+  const int64_t n = ncol > nb ? ncol : nb;
+  const int64_t tiles = (n + kScanTile - 1) / kScanTile + 1;
+  const int64_t groups = (nb + kPullGroup - 1) / kPullGroup;
+  const int64_t sums = 2 * groups;  // block sums, then group sums
+  return tiles > sums ? tiles : sums;
+}
 
 void launch_scan(const int32_t *in, int32_t *out, int64_t n, int32_t *tmp,
                  const Ctl *ctl, int guard, hipStream_t st) {
@@ -265,6 +273,100 @@ void launch_scan(const int32_t *in, int32_t *out, int64_t n, int32_t *tmp,
                      st, in, n, tmp, ctl, guard);
   hipLaunchKernelGGL(k_scan_down, dim3((unsigned)nblk), dim3(kScanBlock), 0,
                      st, in, n, tmp, out, ctl, guard);
+}
+
+// ---------------------------------------------------------------------------
+// Column starts in one launch.  A tile's block adds up the populations of all
+// columns before it itself (at most half a megabyte, in L2, 16 bytes a load)
+// instead of waiting for a launch of tile sums: launches cost 1.55 us each
+// also on the steps that do not rebuild, and the extra reads take less than
+// that up to kColScanMax columns (measured active: 225^2 columns 4.4 us
+// against 4.6 + 4.5 for the two launches).  Larger grids of columns keep the
+// two-launch scan, whose reads grow linearly.
+// ---------------------------------------------------------------------------
+constexpr int kColScanBlock = 1024;
+constexpr int kColScanTile = 4 * kColScanBlock;
+constexpr int64_t kColScanMax = (int64_t)1 << 17;
+
+// sum of v over the block; `ws` holds one int per wavefront
+template <int BLOCK>
+__device__ __forceinline__ int block_sum(int v, int *ws) {
+  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+  if ((threadIdx.x & 63) == 0) ws[threadIdx.x >> 6] = v;
+  __syncthreads();
+  int t = 0;
+#pragma unroll
+  for (int i = 0; i < BLOCK / 64; ++i) t += ws[i];
+  __syncthreads();
+  return t;
+}
+
+// exclusive scan of v over the block
+template <int BLOCK>
+__device__ __forceinline__ int block_excl(int v, int *total, int *ws) {
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  int x = v;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const int y = __shfl_up(x, o, 64);
+    if (lane >= o) x += y;
+  }
+  if (lane == 63) ws[w] = x;
+  __syncthreads();
+  int base = 0, tot = 0;
+#pragma unroll
+  for (int i = 0; i < BLOCK / 64; ++i) {
+    const int t = ws[i];
+    if (i < w) base += t;
+    tot += t;
+  }
+  __syncthreads();
+  *total = tot;
+  return base + x - v;
+}
+
+__device__ __forceinline__ void colscan_body(const Dev &d, int64_t ncol, int64_t tile) {
+  __shared__ int ws[kColScanBlock / 64];
+  const int64_t base = tile * kColScanTile;
+  const int4 *in4 = reinterpret_cast<const int4 *>(d.col_count);
+  int part = 0;
+  for (int64_t i = threadIdx.x; i < base / 4; i += kColScanBlock) {
+    const int4 v = in4[i];
+    part += v.x + v.y + v.z + v.w;
+  }
+  const int carry = block_sum<kColScanBlock>(part, ws);
+  const int64_t i0 = base + 4 * (int64_t)threadIdx.x;
+  int v[4], s = 0;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    v[k] = i0 + k < ncol ? d.col_count[i0 + k] : 0;
+    s += v[k];
+  }
+  int tot;
+  int ex = carry + block_excl<kColScanBlock>(s, &tot, ws);
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    if (i0 + k < ncol) d.col_start[i0 + k] = ex;
+    ex += v[k];
+  }
+  if (base + kColScanTile >= ncol && threadIdx.x == 0) d.col_start[ncol] = carry + tot;
+}
+
+__global__ __launch_bounds__(kColScanBlock) void k_colscan(Dev d, int64_t ncol, int guard) {
+  if (guard_off(d.ctl, guard)) return;
+  colscan_body(d, ncol, blockIdx.x);
+}
+
+static inline unsigned colscan_tiles(int64_t ncol) {
+  return (unsigned)((ncol + kColScanTile - 1) / kColScanTile);
+}
+
+static void launch_colscan(const Dev &d, int64_t ncol, int guard, hipStream_t st) {
+  if (ncol <= kColScanMax)
+    hipLaunchKernelGGL(k_colscan, dim3(colscan_tiles(ncol)), dim3(kColScanBlock), 0, st, d, ncol,
+                       guard);
+  else
+    launch_scan(d.col_count, d.col_start, ncol, d.scan_tmp, guard ? d.ctl : nullptr, guard, st);
 }
 
 // ---------------------------------------------------------------------------
@@ -640,6 +742,54 @@ __global__ __launch_bounds__(256) void k_deg(Dev d, Geo g) {
   deg_body(d, g, blockIdx.x, gridDim.x);
 }
 
+// Degree sums of the groups of kPullGroup bonds and of blocks of kSuper such
+// groups, one 256-thread block per kSuper groups.  The list pass scans its own
+// group and adds up the blocks and groups before it, so the degrees need no
+// scan of their own (one launch instead of two, and the incidence starts are
+// written by the pass that uses them).  With group sums alone every block of
+// the list pass read all of them, which cost the uneven 1.6M-bond system 1 us
+// per step more than the two-launch scan; two levels read one block sum per
+// thread there.  Layout in Dev::scan_tmp: the block sums, then the group sums.
+constexpr int kSuper = 32;
+
+__device__ __forceinline__ int64_t n_groups(int64_t nb) { return (nb + kPullGroup - 1) / kPullGroup; }
+__device__ __forceinline__ int64_t n_supers(int64_t nb) {
+  return (nb + kPullGroup * kSuper - 1) / (kPullGroup * kSuper);
+}
+
+__device__ __forceinline__ void degsum_body(const Dev &d, const Geo &g, int64_t sup) {
+  __shared__ int ws[4];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  int32_t *gsum = d.scan_tmp + n_supers(g.nb);
+  const int64_t ngrp = n_groups(g.nb);
+  int all = 0;
+#pragma unroll
+  for (int j = 0; j < kSuper / 4; ++j) {
+    const int64_t grp = sup * kSuper + wv * (kSuper / 4) + j;
+    int s = 0;
+#pragma unroll
+    for (int k = 0; k < kPullGroup / 64; ++k) {
+      const int64_t b = grp * kPullGroup + lane + 64 * k;
+      if (b < g.nb) s += d.deg[b];
+    }
+    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+    if (lane == 0 && grp < ngrp) gsum[grp] = s;
+    all += s;
+  }
+  if (lane == 0) ws[wv] = all;
+  __syncthreads();
+  if (threadIdx.x == 0) d.scan_tmp[sup] = ws[0] + ws[1] + ws[2] + ws[3];
+}
+
+__global__ __launch_bounds__(256) void k_degsum(Dev d, Geo g) {
+  if (guard_off(d.ctl, kGuardRebuild)) return;
+  degsum_body(d, g, blockIdx.x);
+}
+
+static inline unsigned degsum_blocks(int64_t nb) {
+  return (unsigned)std::max<int64_t>(1, (nb + kPullGroup * kSuper - 1) / (kPullGroup * kSuper));
+}
+
 // Incidence lists in candidate order, one thread per bond, no atomics and
 // no sort.  The list order of CellList::MakePairs (src/cell_list.cpp:
 // 127-137, src/cell.cpp:14-70) is: home cells in key order; inside a home
@@ -660,14 +810,8 @@ __global__ __launch_bounds__(256) void k_deg(Dev d, Geo g) {
 // displacement bookkeeping (InteractionManager::ZeroDrTot -> Mesh/Object::
 // ZeroDrTot, src/interaction_manager.cpp:316-321, src/mesh.cpp:546-551).
 __device__ __forceinline__ void pull_one(const Dev &d, const Geo &g, int32_t b,
-                                         int64_t total, int2 *stage, int32_t base) {
-  int32_t w = d.inc_start[b];
-  const int32_t wend = d.inc_start[b + 1];
-  if (w < 0 || wend < w || wend > total) {  // a wrapped count: refuse, never write
-    d.ctl->abort = 1;
-    d.ctl->overflow = 1;
-    return;
-  }
+                                         int32_t w, int32_t wend, int2 *stage,
+                                         int32_t base) {
   const int32_t k = d.keys[b];
   const Excl x = excl_of(d, g, b);
   const int32_t tag = (b & 63) << 2;
@@ -736,16 +880,31 @@ __device__ __forceinline__ void pull_one(const Dev &d, const Geo &g, int32_t b,
 
 constexpr int kPullStage = 512;
 
+// Each block takes every nblk-th group of kPullGroup bonds; the list range of
+// a group starts at the sum of the groups before it.  The total is 64-bit, so
+// a count that does not fit the lists is seen before anything is written.
 __device__ __forceinline__ void pull_body(const Dev &d, const Geo &g, int64_t bid, int64_t nblk) {
-  const int64_t i0 = bid * blockDim.x + threadIdx.x;
-  const int64_t stride = nblk * blockDim.x;
-  const int64_t total = d.inc_start[g.nb];  // two incidences per candidate
-  const bool fits = total >= 0 && total <= 2 * g.cap;
+  static_assert(kPullGroup == 256, "one bond per thread of a block");
+  __shared__ int64_t red[4];
+  __shared__ int ws[4];
+  __shared__ int2 stage[4][kPullStage];
+  const int t = threadIdx.x, wv = t >> 6, lane = t & 63;
+  const int64_t i0 = bid * 256 + t;
+  const int64_t stride = nblk * 256;
+  const int64_t ngrp = n_groups(g.nb), nsup = n_supers(g.nb);
+  int64_t part = 0;
+  for (int64_t i = t; i < nsup; i += 256) part += d.scan_tmp[i];
+  for (int o = 32; o > 0; o >>= 1) part += __shfl_xor(part, o, 64);
+  if (lane == 0) red[wv] = part;
+  __syncthreads();
+  const int64_t total = red[0] + red[1] + red[2] + red[3];  // two per candidate
+  const bool fits = total <= 2 * g.cap;
   if (i0 == 0) {
-    d.ctl->nc_need = total >= 0 ? total / 2 : 2 * g.cap + 1;
+    d.ctl->nc_need = total / 2;
     if (fits) {
       d.ctl->nc = total / 2;
       d.ctl->n_rebuilds += 1;
+      d.inc_start[g.nb] = (int32_t)total;
     } else {
       d.ctl->abort = 1;
       d.ctl->overflow = 1;
@@ -756,21 +915,31 @@ __device__ __forceinline__ void pull_body(const Dev &d, const Geo &g, int64_t bi
     for (int q = 0; q < 3; ++q) d.dr0[q * g.ns + i] = d.r[q * g.ns + i];
     d.acc[i] = 0.0;
   }
-  // each wavefront takes 64 consecutive bonds, whose lists are one
-  // contiguous range: written to LDS entry by entry, then copied out in
-  // coalesced stores (ranges longer than the stage are written directly)
-  __shared__ int2 stage[4][kPullStage];
-  const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int64_t ngrp = (g.nb + 255) / 256;
+  // the incidence starts of the block's groups, before the walk over them (in
+  // one loop with it they cost the walk 22 registers, two waves per SIMD)
+  for (int grp = (int)bid; grp < (int)ngrp; grp += (int)nblk) {
+    const int64_t b = (int64_t)grp * kPullGroup + t;
+    const int sup = grp / kSuper;
+    int32_t before = sup * kSuper + t < grp ? d.scan_tmp[nsup + sup * kSuper + t] : 0;
+    for (int i = t; i < sup; i += 256) before += d.scan_tmp[i];
+    const int32_t base = block_sum<256>(before, ws);
+    int gtot;
+    const int32_t w = base + block_excl<256>(b < g.nb ? d.deg[b] : 0, &gtot, ws);
+    if (b < g.nb) d.inc_start[b] = w;  // read back by the same thread below
+  }
+  // each wavefront's 64 consecutive bonds have one contiguous list range:
+  // written to LDS entry by entry, then copied out in coalesced stores
+  // (ranges longer than the stage are written directly)
   for (int64_t grp = bid; grp < ngrp; grp += nblk) {
-    const int64_t b0 = grp * 256 + wv * 64, b = b0 + lane;
-    int32_t base = 0, cnt = 0;
-    if (b0 < g.nb) {
-      base = d.inc_start[b0];
-      cnt = d.inc_start[b0 + 64 < g.nb ? b0 + 64 : g.nb] - base;
+    const int64_t b = grp * kPullGroup + t;
+    int32_t w = (int32_t)total, wend = w;
+    if (b < g.nb) {
+      w = d.inc_start[b];
+      wend = w + d.deg[b];
     }
-    const bool staged = cnt >= 0 && cnt <= kPullStage;
-    if (b < g.nb) pull_one(d, g, (int32_t)b, total, staged ? stage[wv] : nullptr, base);
+    const int32_t base = __shfl(w, 0, 64), cnt = __shfl(wend, 63, 64) - base;
+    const bool staged = cnt <= kPullStage;
+    if (b < g.nb) pull_one(d, g, (int32_t)b, w, wend, staged ? stage[wv] : nullptr, base);
     __syncthreads();
     if (staged)
       for (int i = lane; i < cnt; i += 64) d.inc[base + i] = stage[wv][i];
@@ -793,9 +962,9 @@ static inline unsigned sgrid(int64_t n) {
   return b < (unsigned)kStreamBlocks ? b : (unsigned)kStreamBlocks;
 }
 
-// keys (+ column populations) -> column scan (2) -> column scatter ->
-// column sort (+ runs, occupancy) -> degrees -> degree scan (2) ->
-// incidence lists (+ capacity check, displacement restart): 9 launches,
+// keys (+ column populations) -> column scan -> column scatter -> column
+// sort (+ runs, occupancy) -> degrees -> degree sums -> incidence lists
+// (+ incidence starts, capacity check, displacement restart): 7 launches,
 // none over the n1d^3 cells.  Every launch's grid is capped (the kernels
 // loop over their range), so on the odd steps that do not rebuild each
 // launch only reads the guard.  The two per-bond list passes are
@@ -806,13 +975,13 @@ void launch_rebuild(const Dev &d, const Geo &g, hipStream_t st) {
   const unsigned gs = sgrid(g.nb);
   const int64_t ncol = (int64_t)g.n1d * g.n1d;
   hipLaunchKernelGGL(k_keys, dim3(gs), dim3(kScanBlock), 0, st, d, g);
-  launch_scan(d.col_count, d.col_start, ncol, d.scan_tmp, d.ctl, kGuardRebuild, st);
+  launch_colscan(d, ncol, kGuardRebuild, st);
   hipLaunchKernelGGL(k_scatter, dim3(gs), dim3(kScanBlock), 0, st, d, g, (int)kGuardRebuild);
   hipLaunchKernelGGL(k_colsort, dim3(colsort_grid(ncol)), dim3(64 * kColWaves), 0, st, d, g,
                      (int)kGuardRebuild);
   const unsigned gl = std::min(nblocks(g.nb, 256), kListBlocks);
   hipLaunchKernelGGL(k_deg, dim3(gl), dim3(256), 0, st, d, g);
-  launch_scan(d.deg, d.inc_start, g.nb, d.scan_tmp, d.ctl, kGuardRebuild, st);
+  hipLaunchKernelGGL(k_degsum, dim3(degsum_blocks(g.nb)), dim3(256), 0, st, d, g);
   hipLaunchKernelGGL(k_pull, dim3(std::min(nblocks(g.ns > g.nb ? g.ns : g.nb, 256), kListBlocks)),
                      dim3(256), 0, st, d, g);
 }
@@ -857,27 +1026,41 @@ __global__ __launch_bounds__(256) void k_group_pull(const Member *__restrict__ m
   pull_body(M.d[0], M.g, blockIdx.x - b0, nblk);
 }
 
-// which 0: the column populations into column starts; 1: the degrees into
-// the incidence starts
+// the two-launch column scan, for batches with a member of more than
+// kColScanMax columns
 __global__ __launch_bounds__(kScanBlock) void k_group_scan_reduce(const Member *__restrict__ ms,
-                                                                  GroupGrid gg, int which) {
+                                                                  GroupGrid gg) {
   int b0, nblk;
   const Member &M = ms[group_member(gg, blockIdx.x, &b0, &nblk)];
   const Dev &d = M.d[0];
   if (guard_off(d.ctl, kGuardRebuild)) return;
-  const int64_t n = which ? M.g.nb : (int64_t)M.g.n1d * M.g.n1d;
-  scan_reduce_body(which ? d.deg : d.col_count, n, d.scan_tmp, blockIdx.x - b0, nblk);
+  scan_reduce_body(d.col_count, (int64_t)M.g.n1d * M.g.n1d, d.scan_tmp, blockIdx.x - b0, nblk);
 }
 
 __global__ __launch_bounds__(kScanBlock) void k_group_scan_down(const Member *__restrict__ ms,
-                                                                GroupGrid gg, int which) {
+                                                                GroupGrid gg) {
   int b0, nblk;
   const Member &M = ms[group_member(gg, blockIdx.x, &b0, &nblk)];
   const Dev &d = M.d[0];
   if (guard_off(d.ctl, kGuardRebuild)) return;
-  const int64_t n = which ? M.g.nb : (int64_t)M.g.n1d * M.g.n1d;
-  scan_down_body(which ? d.deg : d.col_count, n, d.scan_tmp, which ? d.inc_start : d.col_start,
+  scan_down_body(d.col_count, (int64_t)M.g.n1d * M.g.n1d, d.scan_tmp, d.col_start,
                  blockIdx.x - b0, nblk);
+}
+
+__global__ __launch_bounds__(kColScanBlock) void k_group_colscan(const Member *__restrict__ ms,
+                                                                 GroupGrid gg) {
+  int b0, nblk;
+  const Member &M = ms[group_member(gg, blockIdx.x, &b0, &nblk)];
+  if (guard_off(M.d[0].ctl, kGuardRebuild)) return;
+  colscan_body(M.d[0], (int64_t)M.g.n1d * M.g.n1d, blockIdx.x - b0);
+}
+
+__global__ __launch_bounds__(256) void k_group_degsum(const Member *__restrict__ ms,
+                                                      GroupGrid gg) {
+  int b0, nblk;
+  const Member &M = ms[group_member(gg, blockIdx.x, &b0, &nblk)];
+  if (guard_off(M.d[0].ctl, kGuardRebuild)) return;
+  degsum_body(M.d[0], M.g, blockIdx.x - b0);
 }
 
 namespace {
@@ -894,9 +1077,8 @@ int32_t group_grid(GroupGrid &gg, const Member *hm, int n, F blocks) {
 }
 
 unsigned scan_blocks(int64_t n) {
-  int64_t nblk = (n + kScanTile - 1) / kScanTile;
-  if (nblk == 0) nblk = 1;
-  return (unsigned)(nblk > kStreamBlocks ? kStreamBlocks : nblk);
+  const int64_t nblk = std::max<int64_t>(1, (n + kScanTile - 1) / kScanTile);
+  return (unsigned)std::min<int64_t>(nblk, kStreamBlocks);
 }
 }  // namespace
 
@@ -904,8 +1086,11 @@ void launch_group_rebuild(const Member *dm, const Member *hm, int n, hipStream_t
   if (n <= 0) return;
   GroupGrid gk, gcs, gsrt, gdeg, gds, gpl;
   const int32_t tk = group_grid(gk, hm, n, [](const Geo &g) { return sgrid(g.nb); });
-  const int32_t tcs = group_grid(gcs, hm, n, [](const Geo &g) {
-    return scan_blocks((int64_t)g.n1d * g.n1d);
+  bool wide = false;
+  for (int m = 0; m < n; ++m) wide = wide || (int64_t)hm[m].g.n1d * hm[m].g.n1d > kColScanMax;
+  const int32_t tcs = group_grid(gcs, hm, n, [wide](const Geo &g) {
+    const int64_t ncol = (int64_t)g.n1d * g.n1d;
+    return wide ? scan_blocks(ncol) : colscan_tiles(ncol);
   });
   const int32_t tsrt = group_grid(gsrt, hm, n, [](const Geo &g) {
     return (unsigned)std::min<int64_t>((int64_t)g.n1d * g.n1d, 8192);
@@ -913,18 +1098,21 @@ void launch_group_rebuild(const Member *dm, const Member *hm, int n, hipStream_t
   const int32_t tdeg = group_grid(gdeg, hm, n, [](const Geo &g) {
     return std::min(nblocks(g.nb, 256), kListBlocks);
   });
-  const int32_t tds = group_grid(gds, hm, n, [](const Geo &g) { return scan_blocks(g.nb); });
+  const int32_t tds = group_grid(gds, hm, n, [](const Geo &g) { return degsum_blocks(g.nb); });
   const int32_t tpl = group_grid(gpl, hm, n, [](const Geo &g) {
     return std::min(nblocks(g.ns > g.nb ? g.ns : g.nb, 256), kListBlocks);
   });
   hipLaunchKernelGGL(k_group_keys, dim3(tk), dim3(kScanBlock), 0, st, dm, gk);
-  hipLaunchKernelGGL(k_group_scan_reduce, dim3(tcs), dim3(kScanBlock), 0, st, dm, gcs, 0);
-  hipLaunchKernelGGL(k_group_scan_down, dim3(tcs), dim3(kScanBlock), 0, st, dm, gcs, 0);
+  if (wide) {
+    hipLaunchKernelGGL(k_group_scan_reduce, dim3(tcs), dim3(kScanBlock), 0, st, dm, gcs);
+    hipLaunchKernelGGL(k_group_scan_down, dim3(tcs), dim3(kScanBlock), 0, st, dm, gcs);
+  } else {
+    hipLaunchKernelGGL(k_group_colscan, dim3(tcs), dim3(kColScanBlock), 0, st, dm, gcs);
+  }
   hipLaunchKernelGGL(k_group_scatter, dim3(tk), dim3(kScanBlock), 0, st, dm, gk);
   hipLaunchKernelGGL(k_group_colsort, dim3(tsrt), dim3(64), 0, st, dm, gsrt);
   hipLaunchKernelGGL(k_group_deg, dim3(tdeg), dim3(256), 0, st, dm, gdeg);
-  hipLaunchKernelGGL(k_group_scan_reduce, dim3(tds), dim3(kScanBlock), 0, st, dm, gds, 1);
-  hipLaunchKernelGGL(k_group_scan_down, dim3(tds), dim3(kScanBlock), 0, st, dm, gds, 1);
+  hipLaunchKernelGGL(k_group_degsum, dim3(tds), dim3(256), 0, st, dm, gds);
   hipLaunchKernelGGL(k_group_pull, dim3(tpl), dim3(256), 0, st, dm, gpl);
 }
 
@@ -942,7 +1130,7 @@ void launch_group_ctl(const Member *dm, int n, Ctl *out, hipStream_t st) {
 void launch_cells_from_keys(const Dev &d, const Geo &g, hipStream_t st) {
   const int64_t ncol = (int64_t)g.n1d * g.n1d;
   hipLaunchKernelGGL(k_key_count, dim3(sgrid(g.nb)), dim3(256), 0, st, d, g);
-  launch_scan(d.col_count, d.col_start, ncol, d.scan_tmp, nullptr, 0, st);
+  launch_colscan(d, ncol, 0, st);
   hipLaunchKernelGGL(k_scatter, dim3(sgrid(g.nb)), dim3(256), 0, st, d, g, 0);
   hipLaunchKernelGGL(k_colsort, dim3(colsort_grid(ncol)), dim3(64 * kColWaves), 0, st, d, g, 0);
 }

@@ -1,0 +1,79 @@
+"""Candidate lists where the rebuild's launches change shape: numbers of cell
+columns at the edges of a scan tile (4096) and of the one-launch scan (2^17),
+numbers of bonds at the edges of the list pass's groups (256) and blocks of
+groups (8192).  Checked against a brute-force walk over all pairs."""
+import numpy as np
+import pytest
+
+import simcore_amd as sc
+from tests.scenarios import make_filaments
+
+pytestmark = pytest.mark.gpu
+
+
+def _system(n1d, nb, seed):
+    """Straight filaments with nb bonds in all in a box of n1d cells of side 2,
+    in a few clumps so that lists are not empty."""
+    rng = np.random.default_rng(seed)
+    box = 2.0 * n1d
+    lengths = []
+    left = nb
+    while left > 0:
+        k = min(left, int(rng.integers(2, 40)))
+        if left - k == 1:
+            k += 1
+        lengths.append(k + 1)
+        left -= k
+    sites = []
+    for n in lengths:
+        u = rng.normal(size=3)
+        u /= np.linalg.norm(u)
+        start = (rng.integers(0, 3, 3) / 3.0 - 0.5) * box + rng.normal(size=3) * 6.0
+        sites.append(start + np.arange(n)[:, None] * u)
+    p = sc.params_init(box / 2, delta=1e-6, min_cell_length=2.0, seed=3)
+    return p, make_filaments(sites)
+
+
+def _brute(keys, n, site_off):
+    c = np.stack([keys // (n * n), keys // n % n, keys % n])
+    near = np.ones((len(keys), len(keys)), bool)
+    for x in c:
+        d = (x[:, None] - x[None, :]) % n
+        near &= (d <= 1) | (d == n - 1)
+    i, j = np.nonzero(np.triu(near, 1))
+    fil = np.repeat(np.arange(len(site_off) - 1), np.diff(site_off) - 1)
+    keep = ~((j - i == 1) & (fil[i] == fil[j]))
+    return set(zip(i[keep].tolist(), j[keep].tolist()))
+
+
+@pytest.mark.parametrize("n1d, nb", [(63, 255), (64, 256), (65, 257), (90, 511), (91, 513),
+                                     (362, 300), (363, 300), (40, 8191), (40, 8192), (40, 8193)])
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+def test_lists_at_launch_edges(n1d, nb, precision):
+    p, fil = _system(n1d, nb, n1d + nb)
+    assert fil.nb == nb
+    s = sc.FilamentSystem(p, fil, precision=precision, use_graph=True)
+    assert s.counters()["n_cells_1d"] == n1d
+    a, b = s.candidates()
+    got = set(zip(np.minimum(a, b).tolist(), np.maximum(a, b).tolist()))
+    assert len(got) == len(a)
+    assert got == _brute(s.cell_keys().astype(np.int64), n1d, np.asarray(fil.site_off))
+    s.step(4)
+    s.close()
+
+
+def test_batch_with_a_wide_member():
+    """A batch member with more columns than the one-launch scan takes, beside
+    a small one: each as when stepped alone."""
+    cases = [_system(363, 300, 5), _system(40, 600, 6)]
+    for p, _ in cases:
+        p.delta = 1e-4
+    ens = sc.Ensemble(hbm_budget=4 << 30, max_active=4, steps_per_launch=16, batch_size=4)
+    ids = [ens.submit(p, f, 40, precision="mixed") for p, f in cases]
+    ens.drain(60)
+    for i, (p, f) in zip(ids, cases):
+        s = sc.FilamentSystem(p, f, precision="mixed", use_graph=True)
+        s.step(40)
+        np.testing.assert_array_equal(ens.result(i), s.sites()[0])
+        s.close()
+    ens.close()
