@@ -347,18 +347,26 @@ bool midsteps_in_buffer(const sc_system *h, int64_t from, int64_t n) {
   return (k0 - 1) / 2 >= h->g.xi_m0 && (k1 - 1) / 2 < h->g.xi_m0 + h->g.xi_nm;
 }
 
+// How a step is committed: by a launch at its end (Alone), or as part of a
+// run of odd+even pairs, where an odd step is committed with the even step
+// after it and that pair by the first launch of the next pair; only the last
+// even step of the run has a commit launch.
+enum class Commit { kAlone, kFirstOdd, kOdd, kEven, kLastEven };
+
 // One step.  `odd` says whether the step index is odd: only odd steps can
 // rebuild, so even steps skip the rebuild stage's launches.
-void enqueue_step(sc_system *h, bool odd) {
+void enqueue_step(sc_system *h, bool odd, Commit how) {
+  const bool commit = how == Commit::kAlone || how == Commit::kLastEven;
   // an odd step k starts from the state after k - 1 (even) steps
   Dev d = h->d;
+  d.ahead = how == Commit::kEven || how == Commit::kLastEven ? 1 : 0;
   d.br = h->rec[odd ? 0 : 1];
   d.br_out = h->rec[odd ? 1 : 0];
   const Geo &g = h->g;
   hipStream_t st = h->stream;
   const bool pf = h->prof;
   if (pf) (void)hipEventRecord(h->ev[6], st);
-  if (odd) sc::launch_rebuild(d, g, st);
+  if (odd) sc::launch_rebuild(d, g, how == Commit::kOdd, st);
   if (pf) {
     (void)hipEventRecord(h->ev[7], st);
     (void)hipEventRecord(h->ev[0], st);
@@ -404,7 +412,7 @@ void enqueue_step(sc_system *h, bool odd) {
       if (b.maxn <= 128 && !packed)
         sc::launch_integrate(d, g, b.list, b.count, b.maxn, h->p.precision, h->tune, odd, st);
     (void)hipStreamWaitEvent(st, h->join_ev[1], 0);
-    sc::launch_commit(d, g, st);
+    if (commit) sc::launch_commit(d, g, st);
     return;
   }
   const int P = std::min(h->tune.parts, sc::kMaxParts);
@@ -457,7 +465,7 @@ void enqueue_step(sc_system *h, bool odd) {
       (void)hipEventRecord(h->join_ev[k], h->side[k]);
       (void)hipStreamWaitEvent(st, h->join_ev[k], 0);
     }
-    sc::launch_commit(d, g, st);
+    if (commit) sc::launch_commit(d, g, st);
     return;
   }
   if (!odd) sc::launch_xlink_forces(d, g, st);
@@ -543,19 +551,26 @@ void enqueue_step(sc_system *h, bool odd) {
     (void)hipEventRecord(h->ev[5], st);
     (void)hipEventRecord(h->ev[2], st);
   }
-  sc::launch_commit(d, g, st);
+  if (commit) sc::launch_commit(d, g, st);
   if (pf) (void)hipEventRecord(h->ev[3], st);
+}
+
+// `pairs` odd+even pairs of steps, starting at an odd step
+void enqueue_pairs(sc_system *h, int64_t pairs) {
+  for (int64_t q = 0; q < pairs; ++q) {
+    enqueue_step(h, true, q == 0 ? Commit::kFirstOdd : Commit::kOdd);
+    enqueue_step(h, false, q + 1 == pairs ? Commit::kLastEven : Commit::kEven);
+  }
 }
 
 int capture_graphs(sc_system *h) {
   drop_graph(h);
   for (int k = 0; k < sc_system::kGraphs; ++k) {
     HIPCHK(h, hipStreamBeginCapture(h->stream, hipStreamCaptureModeThreadLocal));
-    const int pairs = k == 3 ? sc_system::kGraphPairs : 1;
-    for (int q = 0; q < pairs; ++q) {
-      if (k == 0 || k >= 2) enqueue_step(h, true);
-      if (k >= 1) enqueue_step(h, false);
-    }
+    if (k < 2)
+      enqueue_step(h, k == 0, Commit::kAlone);
+    else
+      enqueue_pairs(h, k == 3 ? sc_system::kGraphPairs : 1);
     hipGraph_t gr = nullptr;
     HIPCHK(h, hipStreamEndCapture(h->stream, &gr));
     h->graph[k] = gr;
@@ -574,7 +589,7 @@ int initial_rebuild(sc_system *h) {
     c.overflow = 0;
     int rc = write_ctl(h, c);
     if (rc) return rc;
-    sc::launch_rebuild(h->d, h->g, h->stream);
+    sc::launch_rebuild(h->d, h->g, false, h->stream);
     HIPCHK(h, hipStreamSynchronize(h->stream));
     HIPCHK(h, hipGetLastError());
     c = read_ctl(h);
@@ -841,8 +856,14 @@ int enqueue_range(sc_system *h, int64_t from, int64_t count) {
         continue;
       }
       HIPCHK(h, hipGraphLaunch(h->gexec[odd ? 0 : 1], h->stream));
+    } else if (odd && count - s >= 2 && !h->prof) {
+      const int64_t pairs = (count - s) / 2;
+      enqueue_pairs(h, pairs);
+      s += 2 * pairs;
+      next += 2 * pairs;
+      continue;
     } else {
-      enqueue_step(h, odd);
+      enqueue_step(h, odd, Commit::kAlone);
       if (h->prof) {
         HIPCHK(h, hipEventSynchronize(h->ev[3]));
         float ms = 0.f;
@@ -970,6 +991,8 @@ void system_member(sc_handle h, Member *m) {
   m->d[1] = h->d;
   m->d[1].br = h->rec[1];
   m->d[1].br_out = h->rec[0];
+  m->d[0].ahead = 0;
+  m->d[1].ahead = 1;
   m->g = h->g;
   m->pack_tab = h->pack_tab;
   m->pack_waves = h->pack_waves;

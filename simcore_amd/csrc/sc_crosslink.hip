@@ -125,7 +125,7 @@ __global__ __launch_bounds__(256) void k_xl_events(Dev d, Geo g) {
   if (ctl->abort) return;
   const int64_t x = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (x >= g.nx) return;
-  const int64_t m = ctl->cur_step / 2;
+  const int64_t m = step_index(d) / 2;
   uint32_t o[4] = {(uint32_t)x, (uint32_t)((uint64_t)x >> 32), (uint32_t)m, 1u};
   const uint32_t k0 = (uint32_t)g.xseed, k1 = (uint32_t)(g.xseed >> 32);
   philox4x32(o, k0, k1);

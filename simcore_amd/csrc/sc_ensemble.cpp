@@ -253,15 +253,15 @@ int enqueue_batch(sc_ensemble e, Batch &B) {
       if (hipStreamBeginCapture(B.st, hipStreamCaptureModeThreadLocal) != hipSuccess)
         return SC_ERR_HIP;
       for (int q = 0; q < (v ? kBatchGraphPairs : 1); ++q) {
-        // odd step (the rebuild stage, then the midstep), even step
-        sc::launch_group_rebuild(B.dm, B.hm, n, B.st);
+        // odd step (the rebuild stage, whose first launch commits the pair
+        // before, then the midstep), even step
+        sc::launch_group_rebuild(B.dm, B.hm, n, q > 0, B.st);
         sc::launch_group_pair(B.dm, B.hm, n, true, B.st);
         sc::launch_group_integrate(B.dm, B.hm, n, true, B.st);
-        sc::launch_group_commit(B.dm, n, B.st);
         sc::launch_group_pair(B.dm, B.hm, n, false, B.st);
         sc::launch_group_integrate(B.dm, B.hm, n, false, B.st);
-        sc::launch_group_commit(B.dm, n, B.st);
       }
+      sc::launch_group_commit(B.dm, n, B.st);
       hipGraph_t gr = nullptr;
       if (hipStreamEndCapture(B.st, &gr) != hipSuccess) return SC_ERR_HIP;
       const hipError_t ie = hipGraphInstantiate(&B.gx[v], gr, nullptr, nullptr, 0);

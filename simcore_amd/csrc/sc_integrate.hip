@@ -83,8 +83,8 @@ __global__ __launch_bounds__(64) void k_integrate(Dev d, Geo g,
   const int n = active ? (int)(d.site_off[f + 1] - s0) : 0;
   const int64_t b0 = s0 - f;
   const int64_t ns = g.ns, nb = g.nb;
-  const bool mid = ctl->midstep != 0;
-  const int64_t step = ctl->cur_step;
+  const bool mid = step_is_mid(d);
+  const int64_t step = step_index(d);
   double bl = 1.0, kappa = 0.0, gpar = 1.0, gperp = 1.0, sgpar = 0.0, sgperp = 0.0;
   if (active) {
     const double *fp = d.fpar + 8 * f;

@@ -268,14 +268,13 @@ __device__ __forceinline__ void det_backward(const double (&N)[S][4], double (&o
 template <int W, int S, bool MID>
 __device__ __forceinline__ void long_body(const Dev &d, const Geo &g, bool factive, int f,
                                           int gl, int Gf, int slot) {
-  const Ctl *ctl = d.ctl;
   const int lane = threadIdx.x & 63;
   const int64_t s0 = factive ? d.site_off[f] : 0;
   const int n = factive ? (int)(d.site_off[f + 1] - s0) : 0;
   const int64_t b0 = s0 - f;
   const int64_t ns = g.ns;
   constexpr bool mid = MID;
-  const int64_t step = ctl->cur_step;
+  const int64_t step = step_index(d);
   const int m = n - 1;
   double bl = 1.0, kappa = 0.0, gpar = 1.0, gperp = 1.0, sgpar = 0.0, sgperp = 0.0;
   int64_t noise0 = 0;
@@ -710,7 +709,7 @@ void k_integrate_long(Dev d, Geo g, const int32_t *list,
                                                         int count) {
   Ctl *ctl = d.ctl;
   if (ctl->abort) return;
-  if ((ctl->midstep != 0) != MID) {  // launched for the wrong kind of step
+  if (step_is_mid(d) != MID) {  // launched for the wrong kind of step
     if (blockIdx.x == 0 && threadIdx.x == 0) {
       ctl->err = SC_ERR_STATE;
       ctl->abort = 1;
@@ -738,7 +737,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(W == 64 ? 3
 void k_integrate_packed(Dev d, Geo g, const int32_t *lane_tab, int n_waves) {
   Ctl *ctl = d.ctl;
   if (ctl->abort) return;
-  if ((ctl->midstep != 0) != MID) {
+  if (step_is_mid(d) != MID) {
     if (blockIdx.x == 0 && threadIdx.x == 0) {
       ctl->err = SC_ERR_STATE;
       ctl->abort = 1;
@@ -769,7 +768,7 @@ __device__ __forceinline__ void packed_any_body(const Dev &d, const Geo &g,
                                                 int cs2, int bid) {
   Ctl *ctl = d.ctl;
   if (ctl->abort) return;
-  if ((ctl->midstep != 0) != MID) {
+  if (step_is_mid(d) != MID) {
     if (bid == 0 && threadIdx.x == 0) {
       ctl->err = SC_ERR_STATE;
       ctl->abort = 1;
@@ -813,7 +812,7 @@ __device__ __forceinline__ void all_body(const Dev &d, const Geo &g, const int32
   if (wave < n_long) {
     Ctl *ctl = d.ctl;
     if (ctl->abort) return;
-    if ((ctl->midstep != 0) != MID) {
+    if (step_is_mid(d) != MID) {
       if (wave == 0 && (threadIdx.x & 63) == 0) {
         ctl->err = SC_ERR_STATE;
         ctl->abort = 1;
@@ -828,7 +827,7 @@ __device__ __forceinline__ void all_body(const Dev &d, const Geo &g, const int32
   const int pw = wave - n_long;
   Ctl *ctl = d.ctl;
   if (ctl->abort) return;
-  if ((ctl->midstep != 0) != MID) {
+  if (step_is_mid(d) != MID) {
     if (wave == 0 && (threadIdx.x & 63) == 0) {
       ctl->err = SC_ERR_STATE;
       ctl->abort = 1;

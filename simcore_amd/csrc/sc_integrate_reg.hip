@@ -39,8 +39,8 @@ __global__ __launch_bounds__(256) void k_integrate_reg(Dev d, Geo g, const int32
   const int n = factive ? (int)(d.site_off[f + 1] - s0) : 0;
   const int64_t b0 = s0 - f;
   const int64_t ns = g.ns;
-  const bool mid = ctl->midstep != 0;
-  const int64_t step = ctl->cur_step;
+  const bool mid = step_is_mid(d);
+  const int64_t step = step_index(d);
   const int i = gl;
   const bool act = i < n;
   const int m = n - 1;  // bonds / tension unknowns

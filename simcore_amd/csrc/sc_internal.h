@@ -83,6 +83,9 @@ constexpr int kDrSlots = 256;
 
 struct Dev {
   Ctl *ctl;
+  int ahead;               // steps taken since the last commit of Ctl: 1 on an
+                           // even step that follows its odd step without a
+                           // commit between them, else 0
   unsigned long long *dr_slots;  // kDrSlots, zero between steps
   // filaments
   int32_t *site_off;       // nf+1
@@ -151,6 +154,12 @@ struct Dev {
   // per bond, its pair potential energy of the last step
   double *stress_acc, *bpote;
 };
+
+// Index of the step being executed, and whether it is a midstep.
+__device__ __forceinline__ int64_t step_index(const Dev &d) { return d.ctl->cur_step + d.ahead; }
+__device__ __forceinline__ bool step_is_mid(const Dev &d) {
+  return (d.ctl->midstep != 0) != (d.ahead != 0);
+}
 
 // Launch shapes the autotuner chooses among; none changes a result.
 struct Tune {
@@ -227,9 +236,11 @@ __device__ __forceinline__ int group_member(const GroupGrid &gg, int bid, int *b
 // Grouped launchers (sc_kernels.hip, sc_pair.hip, sc_integrate_long.hip):
 // `dm` the device copy of the members, `hm` the host copy (sizes), n
 // members, `odd` the parity of the step all of them take.
-void launch_group_rebuild(const Member *dm, const Member *hm, int n, hipStream_t st);
+// (`fold`: see launch_rebuild)
+void launch_group_rebuild(const Member *dm, const Member *hm, int n, bool fold, hipStream_t st);
 void launch_group_pair(const Member *dm, const Member *hm, int n, bool odd, hipStream_t st);
 void launch_group_integrate(const Member *dm, const Member *hm, int n, bool odd, hipStream_t st);
+// after an even step that followed its odd step without a commit
 void launch_group_commit(const Member *dm, int n, hipStream_t st);
 // each member's control block into out[m]
 void launch_group_ctl(const Member *dm, int n, Ctl *out, hipStream_t st);
@@ -263,7 +274,9 @@ __device__ __forceinline__ bool cell_occupied(const Dev &d, const Geo &g, int x,
 // Launchers (sc_kernels.hip).  All are asynchronous on `st`.
 void launch_decide(const Dev &d, const Geo &g, hipStream_t st);
 void launch_commit(const Dev &d, const Geo &g, hipStream_t st);
-void launch_rebuild(const Dev &d, const Geo &g, hipStream_t st);
+// `fold`: the odd step follows an even step that was not committed; the first
+// launch commits it and decides the rebuild
+void launch_rebuild(const Dev &d, const Geo &g, bool fold, hipStream_t st);
 void launch_cells_from_keys(const Dev &d, const Geo &g, hipStream_t st);
 // `thermo`: also sum the pair stress and the bond energies (Geo::thermo)
 void launch_pair(const Dev &d, const Geo &g, int precision, const Tune &t,

@@ -13,6 +13,9 @@
 //    incidence lists (+ incidence starts, capacity, zero dr)]
 //   -> pair+scatter -> integrate (per length class)
 //   -> commit (and decide the next step)
+// Runs of odd+even pairs commit less often: an odd step is committed with the
+// even step after it, and that pair by the first launch of the next pair
+// (fold_commit), so only the last pair of a run needs the commit launch.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -76,16 +79,19 @@ __global__ void k_decide(Ctl *c, unsigned long long *slots, double thr) {
 
 // end of a step: commit it and decide the next one (one launch for both).
 // Every value it needs is loaded up front, so the kernel costs one memory
-// round trip; the decision is decide_next's on those values.
-__device__ __forceinline__ void commit_body(Ctl *c, unsigned long long *slots, double thr) {
+// round trip; the decision is decide_next's on those values.  `ahead`: the
+// odd step before was not committed either (its commit would only have moved
+// the counters and cleared dr_bits), so both are committed here.
+__device__ __forceinline__ void commit_body(Ctl *c, unsigned long long *slots, double thr,
+                                            int ahead) {
   static_assert(kDrSlots == 4 * 64, "four slots per lane");
   const int lane = threadIdx.x;
   unsigned long long v[4];
 #pragma unroll
   for (int i = 0; i < 4; ++i) v[i] = slots[lane + 64 * i];
   const int32_t abort = c->abort;
-  const int64_t cur = c->cur_step;
-  const unsigned long long drb = c->dr_bits;
+  const int64_t cur = c->cur_step + ahead;
+  const unsigned long long drb = ahead ? 0ull : c->dr_bits;
   if (abort) return;
   unsigned long long m = drb;
 #pragma unroll
@@ -117,15 +123,15 @@ __device__ __forceinline__ void commit_body(Ctl *c, unsigned long long *slots, d
   c->rebuild = rb;
 }
 
-__global__ void k_commit(Ctl *c, unsigned long long *slots, double thr) {
+__global__ void k_commit(Ctl *c, unsigned long long *slots, double thr, int ahead) {
   if (blockIdx.x != 0) return;
-  commit_body(c, slots, thr);
+  commit_body(c, slots, thr, ahead);
 }
 
 // one block per member
 __global__ void k_group_commit(const Member *__restrict__ ms) {
   const Member &M = ms[blockIdx.x];
-  commit_body(M.d[0].ctl, M.d[0].dr_slots, M.g.thr);
+  commit_body(M.d[1].ctl, M.d[1].dr_slots, M.g.thr, M.d[1].ahead);
 }
 
 __global__ void k_group_ctl(const Member *__restrict__ ms, int n, Ctl *out) {
@@ -423,8 +429,54 @@ __device__ __forceinline__ void keys_body(const Dev &d, const Geo &g, int64_t bi
   }
 }
 
-__global__ void k_keys(Dev d, Geo g) {
-  if (guard_off(d.ctl, kGuardRebuild)) return;
+// Commit of the full step before an odd step, inside the odd step's first
+// launch, in place of a launch of its own (2-3 us, mostly waiting: it is one
+// block that loads and stores a few words).  Every block folds the
+// displacement slots and takes the decision for itself from values that no
+// block of this launch changes; block 0 also stores it in Ctl for the
+// launches that follow.  The slots are cleared by the column scatter, after
+// every block has read them and before a full step fills them again.  Returns
+// whether the odd step rebuilds.
+__device__ __forceinline__ bool fold_commit(const Dev &d, double thr, bool first) {
+  static_assert(kDrSlots == kScanBlock, "one slot per thread");
+  __shared__ unsigned long long wmax[kScanBlock / 64];
+  __shared__ int off;
+  Ctl *c = d.ctl;
+  unsigned long long m = d.dr_slots[threadIdx.x];
+  if (threadIdx.x == 0) off = c->abort;
+  for (int o = 32; o > 0; o >>= 1) {
+    const unsigned long long y = __shfl_xor(m, o, 64);
+    m = y > m ? y : m;
+  }
+  if ((threadIdx.x & 63) == 0) wmax[threadIdx.x >> 6] = m;
+  __syncthreads();
+  if (off) return false;
+#pragma unroll
+  for (int i = 0; i < kScanBlock / 64; ++i) m = wmax[i] > m ? wmax[i] : m;
+  const double drm = __longlong_as_double((long long)m);
+  const bool lost = drm > 10000;  // include/simcore/species.hpp:114-118
+  const bool rb = !lost && drm > thr;
+  if (first && threadIdx.x == 0) {
+    const int64_t cur = c->cur_step;  // the odd step before the full step
+    c->i_step = cur + 1;
+    c->cur_step = cur + 2;
+    c->dr_bits = m;
+    c->rebuild = rb ? 1 : 0;
+    if (lost) {
+      c->abort = 1;
+      c->err = SC_ERR_UNPHYSICAL;
+    }
+  }
+  return rb;
+}
+
+template <bool FOLD>
+__global__ __launch_bounds__(kScanBlock) void k_keys(Dev d, Geo g) {
+  if (FOLD) {
+    if (!fold_commit(d, g.thr, blockIdx.x == 0)) return;
+  } else {
+    if (guard_off(d.ctl, kGuardRebuild)) return;
+  }
   keys_body(d, g, blockIdx.x, gridDim.x);
 }
 
@@ -447,7 +499,14 @@ __device__ __forceinline__ void scatter_body(const Dev &d, const Geo &g, int64_t
   }
 }
 
+// (the displacement slots of the step before are done with here, see
+// fold_commit; between steps they are zero anyway)
+__device__ __forceinline__ void clear_dr_slots(const Dev &d) {
+  for (int i = threadIdx.x; i < kDrSlots; i += blockDim.x) d.dr_slots[i] = 0ull;
+}
+
 __global__ void k_scatter(Dev d, Geo g, int guard) {
+  if (blockIdx.x == 0) clear_dr_slots(d);
   if (guard_off(d.ctl, guard)) return;
   scatter_body(d, g, blockIdx.x, gridDim.x);
 }
@@ -971,10 +1030,13 @@ static inline unsigned sgrid(int64_t n) {
 // latency-bound and get 8 waves per SIMD.
 constexpr unsigned kListBlocks = 2048;
 
-void launch_rebuild(const Dev &d, const Geo &g, hipStream_t st) {
+void launch_rebuild(const Dev &d, const Geo &g, bool fold, hipStream_t st) {
   const unsigned gs = sgrid(g.nb);
   const int64_t ncol = (int64_t)g.n1d * g.n1d;
-  hipLaunchKernelGGL(k_keys, dim3(gs), dim3(kScanBlock), 0, st, d, g);
+  if (fold)
+    hipLaunchKernelGGL(k_keys<true>, dim3(gs), dim3(kScanBlock), 0, st, d, g);
+  else
+    hipLaunchKernelGGL(k_keys<false>, dim3(gs), dim3(kScanBlock), 0, st, d, g);
   launch_colscan(d, ncol, kGuardRebuild, st);
   hipLaunchKernelGGL(k_scatter, dim3(gs), dim3(kScanBlock), 0, st, d, g, (int)kGuardRebuild);
   hipLaunchKernelGGL(k_colsort, dim3(colsort_grid(ncol)), dim3(64 * kColWaves), 0, st, d, g,
@@ -990,16 +1052,23 @@ void launch_rebuild(const Dev &d, const Geo &g, hipStream_t st) {
 // (odd-step pointers: a rebuild only ever starts an odd step); a member
 // that does not rebuild returns at its guard.  Per member, the same grid as
 // its own launch.
-__global__ void k_group_keys(const Member *__restrict__ ms, GroupGrid gg) {
+template <bool FOLD>
+__global__ __launch_bounds__(kScanBlock) void k_group_keys(const Member *__restrict__ ms,
+                                                           GroupGrid gg) {
   int b0, nblk;
   const Member &M = ms[group_member(gg, blockIdx.x, &b0, &nblk)];
-  if (guard_off(M.d[0].ctl, kGuardRebuild)) return;
+  if (FOLD) {
+    if (!fold_commit(M.d[0], M.g.thr, (int)blockIdx.x == b0)) return;
+  } else {
+    if (guard_off(M.d[0].ctl, kGuardRebuild)) return;
+  }
   keys_body(M.d[0], M.g, blockIdx.x - b0, nblk);
 }
 
 __global__ void k_group_scatter(const Member *__restrict__ ms, GroupGrid gg) {
   int b0, nblk;
   const Member &M = ms[group_member(gg, blockIdx.x, &b0, &nblk)];
+  if ((int)blockIdx.x == b0) clear_dr_slots(M.d[0]);
   if (guard_off(M.d[0].ctl, kGuardRebuild)) return;
   scatter_body(M.d[0], M.g, blockIdx.x - b0, nblk);
 }
@@ -1082,7 +1151,7 @@ unsigned scan_blocks(int64_t n) {
 }
 }  // namespace
 
-void launch_group_rebuild(const Member *dm, const Member *hm, int n, hipStream_t st) {
+void launch_group_rebuild(const Member *dm, const Member *hm, int n, bool fold, hipStream_t st) {
   if (n <= 0) return;
   GroupGrid gk, gcs, gsrt, gdeg, gds, gpl;
   const int32_t tk = group_grid(gk, hm, n, [](const Geo &g) { return sgrid(g.nb); });
@@ -1102,7 +1171,10 @@ void launch_group_rebuild(const Member *dm, const Member *hm, int n, hipStream_t
   const int32_t tpl = group_grid(gpl, hm, n, [](const Geo &g) {
     return std::min(nblocks(g.ns > g.nb ? g.ns : g.nb, 256), kListBlocks);
   });
-  hipLaunchKernelGGL(k_group_keys, dim3(tk), dim3(kScanBlock), 0, st, dm, gk);
+  if (fold)
+    hipLaunchKernelGGL(k_group_keys<true>, dim3(tk), dim3(kScanBlock), 0, st, dm, gk);
+  else
+    hipLaunchKernelGGL(k_group_keys<false>, dim3(tk), dim3(kScanBlock), 0, st, dm, gk);
   if (wide) {
     hipLaunchKernelGGL(k_group_scan_reduce, dim3(tcs), dim3(kScanBlock), 0, st, dm, gcs);
     hipLaunchKernelGGL(k_group_scan_down, dim3(tcs), dim3(kScanBlock), 0, st, dm, gcs);
@@ -1182,7 +1254,7 @@ void launch_decide(const Dev &d, const Geo &g, hipStream_t st) {
 }
 
 void launch_commit(const Dev &d, const Geo &g, hipStream_t st) {
-  hipLaunchKernelGGL(k_commit, dim3(1), dim3(64), 0, st, d.ctl, d.dr_slots, g.thr);
+  hipLaunchKernelGGL(k_commit, dim3(1), dim3(64), 0, st, d.ctl, d.dr_slots, g.thr, d.ahead);
 }
 
 void launch_zero_i32(int32_t *p, int64_t n, hipStream_t st) {
