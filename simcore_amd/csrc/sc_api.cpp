@@ -22,6 +22,7 @@ namespace {
 
 struct Bin {
   int maxn = 0;
+  int longest = 0;  // sites of its longest filament
   int count = 0;
   int32_t *list = nullptr;
   std::vector<int64_t> last;  // last bond of each listed filament (ascending)
@@ -497,7 +498,9 @@ void enqueue_step(sc_system *h, bool odd, Commit how) {
                          h->pack_cs[c + 1] - h->pack_cs[c], 0, 16 << c};
   }
   for (const Bin &b : h->bins)
-    if ((!packed || b.maxn > 128) && &b != merged) bins[nbins++] = {b.list, b.count, b.maxn, 0};
+    if ((!packed || b.maxn > 128) && &b != merged)
+      bins[nbins++] = {b.list, b.count, b.maxn,
+                       h->p.precision == SC_PREC_FP64 ? b.longest : 0};
   auto load_of = [&](int k) -> int64_t {
     if (bins[k].maxn) return (int64_t)bins[k].count * bins[k].maxn;
     const int64_t l = (int64_t)bins[k].count * 120;
@@ -517,7 +520,9 @@ void enqueue_step(sc_system *h, bool odd, Commit how) {
       sc::launch_integrate(d, g, bins[k].list, bins[k].count, bins[k].maxn, h->p.precision,
                            h->tune, odd, sk);
   };
-  if (h->tune.int_streams && nbins > 1 && h->side[0]) {
+  if (h->p.precision == SC_PREC_FP64 && !h->tune.int_streams) {
+    sc::launch_integrate_exact(d, g, bins, nbins, st);
+  } else if (h->tune.int_streams && nbins > 1 && h->side[0]) {
     // bins are independent (disjoint filaments; the displacement maxima
     // combine by max): deal them to the main and side streams, largest
     // first onto the least loaded, then join
@@ -1321,7 +1326,10 @@ int sc_load_filaments(sc_handle h, int32_t nf, const int32_t *site_off,
     Bin b;
     b.maxn = bin_max[k];
     b.count = (int)lists[k].size();
-    for (int32_t f : lists[k]) b.last.push_back((int64_t)site_off[f + 1] - f - 2);
+    for (int32_t f : lists[k]) {
+      b.last.push_back((int64_t)site_off[f + 1] - f - 2);
+      b.longest = std::max(b.longest, (int)(site_off[f + 1] - site_off[f]));
+    }
     if (b.maxn > 128) h->long_last = std::max(h->long_last, b.last.back());
     if ((rc = dalloc(h, &b.list, lists[k].size(), false))) return rc;
     HIPCHK(h, hipMemcpyAsync(b.list, lists[k].data(), sizeof(int32_t) * lists[k].size(),

@@ -1,19 +1,29 @@
-// sc_integrate.hip -- Filament::UpdatePosition (src/filament.cpp:394-428)
-// for all filaments of one length bin.
+// sc_integrate.hip -- Filament::UpdatePosition (src/filament.cpp:394-428) on
+// the FP64 path: every operation in the reference's order, so the results are
+// those of the CPU path bit for bit.
 //
-// Mapping: a wavefront holds 64/G filaments, G lanes each; lane gl of a
-// group owns sites gl, gl+G, ..., gl+(S-1)G, so a bin serves filaments of up
-// to G*S sites.  Per-site values live in LDS, one slice per group.
+// Mapping: one site per lane.  A block of 256 lanes holds as many filaments
+// of one length bin as fit (the bin's longest filament sets the slice), and
+// one launch serves every bin, the longest first, so that their chains run
+// beside the short filaments' instead of after them.  Per-site values live in
+// LDS, one slice per filament, odd strides between slices.
 //
 // The reference's sequential pieces -- the two Thomas solves
 // (src/linear_algebra.cpp:164-197), the metric-determinant recursions
-// (src/filament.cpp:613-623) and bond renormalisation (:904-924) -- run on
-// each group's first lane with the recursion carried in registers, so the
-// groups of a wave advance their chains together.  In FAST mode the
-// tridiagonal solves instead use parallel cyclic reduction over the
-// group's lanes (log2 n rounds); EXACT mode keeps Thomas, operation for
-// operation, and reproduces the CPU path bit for bit.
+// (src/filament.cpp:613-623) and bond renormalisation (:904-924) -- run one
+// filament per lane of one wavefront, the recursion in registers and the
+// coefficients of the next rows loaded from LDS while the current ones are
+// worked on; a midstep's determinant recursions run in a second wavefront
+// beside its random-force solve.
+//
+// Bound: the latency of those chains (about 100 clocks a Thomas row, most of
+// it the division) and, for large systems, instruction issue.  Measured, full
+// step and midstep: 925 x 8 filaments of 8-256 sites (229k bonds) 58 and 69 us
+// where the six launches, one per bin, with chains branching and loading row
+// by row took 190 and 260; 5000 filaments of 32 sites 28 and 31 us (31, 40).
 #include <hip/hip_runtime.h>
+
+#include <algorithm>
 
 #include "sc_internal.h"
 #include "sc_math.h"
@@ -22,62 +32,214 @@ namespace sc {
 
 namespace {
 
-// Thomas on m unknowns with the reference's operation order; lower[i]
-// couples row i+1 to x[i], upper[i] couples row i to x[i+1].
-__device__ __forceinline__ void thomas_reg(int m, const double *__restrict__ lo,
-                                           const double *__restrict__ di,
-                                           double *__restrict__ up,
-                                           double *__restrict__ rh) {
-  const int nn = m - 1;
-  double cp = up[0] / di[0];
-  double dp = rh[0] / di[0];
-  up[0] = cp;
-  rh[0] = dp;
-  for (int i = 1; i < nn; ++i) {
-    const double a = lo[i - 1];
-    const double den = di[i] - a * cp;
-    cp = up[i] / den;
-    dp = (rh[i] - a * dp) / den;
-    up[i] = cp;
-    rh[i] = dp;
+constexpr int kExactBlock = 256;
+constexpr int kSlots = 288;    // site slots of a block: slices of odd stride
+constexpr int kMaxChains = 64;  // filaments of a block: one lane each in a chain
+constexpr int kAhead = 2;       // rows loaded ahead of a chain (120 registers, four
+                                // wavefronts per SIMD; 4 rows take 144)
+
+// Slice layout of filaments of at most w sites: the stride between slices
+// (odd, so that the chains' lanes, one per slice, hit different banks) and
+// how many fit a block.
+__host__ __device__ __forceinline__ int exact_stride(int w) { return w | 1; }
+__host__ __device__ __forceinline__ int exact_per_block(int w) {
+  const int a = kExactBlock / w, b = kSlots / exact_stride(w);
+  const int n = a < b ? a : b;
+  return n < kMaxChains ? (n < 1 ? 1 : n) : kMaxChains;
+}
+
+// IEEE division of several numerators by one denominator: the refined
+// reciprocal is shared and each quotient rounds once more, which gives the
+// correctly rounded quotient (the steps of the hardware division sequence
+// without its operand scaling).  Valid for 2^-200 <= |den| <= 2^200 or 0 and
+// |num| = 0 or >= 2^-900; v_div_fixup supplies zeros, infinities and NaNs.
+// 81 clocks for two dependent quotients in a chain, against 138 for two IEEE
+// divisions as the compiler expands them (one wavefront, measured).
+__device__ __forceinline__ double shared_rcp(double den) {
+  double y = __builtin_amdgcn_rcp(den);
+  y = fma(y, fma(-den, y, 1.0), y);
+  return fma(y, fma(-den, y, 1.0), y);
+}
+__device__ __forceinline__ double shared_quot(double num, double den, double y) {
+  const double m = num * y;
+  return __builtin_amdgcn_div_fixup(fma(fma(-den, m, num), y, m), den, num);
+}
+// (the high word of |x|, doubled) - 1: zero is the largest value, so a
+// minimum over numerators ignores zeros
+__device__ __forceinline__ uint32_t magnitude(double x) {
+  return ((uint32_t)(__double_as_longlong(x) >> 32) << 1) - 1u;
+}
+constexpr uint32_t kTiny = (1023u - 900u) << 21;  // magnitude of 2^-900
+
+// Thomas with the reference's operation order on symmetric rows {diagonal,
+// right-hand side} and off-diagonals off[i] (rows i, i+1); the solution
+// replaces the right-hand side.  `rows` is the same for every lane: rows
+// past a filament's last are {1, 0} with off-diagonal 0, which solve to 0
+// and leave the others as they are, so no lane needs a branch.  The last row's
+// solution is the forward recursion's value there.  FAST: quotients by
+// shared_quot; returns false when a numerator was too small for it (the
+// caller then sets the rows up again and takes the plain divisions).
+template <bool FAST>
+__device__ __forceinline__ bool thomas_chain(int rows, double2 *row, const double *off) {
+  uint32_t least = ~0u;
+  double cp = 0.0, dp = 0.0, lo = 0.0;
+  double2 v[kAhead];
+  double c[kAhead];
+  auto load = [&](int i0) {
+#pragma unroll
+    for (int k = 0; k < kAhead; ++k) {
+      const int i = i0 + k < rows ? i0 + k : rows - 1;
+      v[k] = row[i];
+      c[k] = off[i];
+    }
+  };
+  auto step = [&](int i, const double2 &w, double o) {
+    const double den = w.x - lo * cp;  // (row 0: lo, cp and dp are 0)
+    const double num = w.y - lo * dp;
+    if (FAST) {
+      const double y = shared_rcp(den);
+      least = min(least, magnitude(num));
+      cp = shared_quot(o, den, y);
+      dp = shared_quot(num, den, y);
+    } else {
+      cp = o / den;
+      dp = num / den;
+    }
+    lo = o;
+    row[i] = make_double2(cp, dp);
+  };
+  load(0);
+  int i0 = 0;
+  for (; i0 + kAhead <= rows; i0 += kAhead) {
+    double2 w[kAhead];
+    double o[kAhead];
+#pragma unroll
+    for (int k = 0; k < kAhead; ++k) {
+      w[k] = v[k];
+      o[k] = c[k];
+    }
+    load(i0 + kAhead);
+#pragma unroll
+    for (int k = 0; k < kAhead; ++k) step(i0 + k, w[k], o[k]);
   }
-  const double a = lo[nn - 1];
-  double x = (rh[nn] - a * dp) / (di[nn] - a * cp);
-  rh[nn] = x;
-  for (int i = nn; i-- > 0;) {
-    x = rh[i] - up[i] * x;
-    rh[i] = x;
+#pragma unroll
+  for (int k = 0; k < kAhead; ++k)
+    if (i0 + k < rows) step(i0 + k, v[k], c[k]);
+  // back substitution, rows rows-2 .. 0
+  double x = dp;
+  auto loadb = [&](int j0) {
+#pragma unroll
+    for (int k = 0; k < kAhead; ++k) v[k] = row[j0 - k > 0 ? j0 - k : 0];
+  };
+  int j0 = rows - 2;
+  loadb(j0);
+  for (; j0 - kAhead + 1 >= 0; j0 -= kAhead) {
+    double2 w[kAhead];
+#pragma unroll
+    for (int k = 0; k < kAhead; ++k) w[k] = v[k];
+    loadb(j0 - kAhead);
+#pragma unroll
+    for (int k = 0; k < kAhead; ++k) {
+      x = w[k].y - w[k].x * x;
+      row[j0 - k].y = x;
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < kAhead; ++k)
+    if (j0 - k >= 0) {
+      x = v[k].y - v[k].x * x;
+      row[j0 - k].y = x;
+    }
+  return !FAST || least >= kTiny;
+}
+
+// Metric determinants (src/filament.cpp:613-623) from the cosines cs[0..n-3]
+// of n sites: det_t[0..rows-1] forward from the tail (entries past n-1 are
+// not used)
+__device__ __forceinline__ void det_tail(int rows, const double *cs, double *dt) {
+  double t2 = 1.0, t1 = 2.0;
+  dt[0] = 1;
+  dt[1] = 2;
+  double f[kAhead];
+  auto load = [&](int i0) {
+#pragma unroll
+    for (int k = 0; k < kAhead; ++k) f[k] = cs[(i0 + k < rows ? i0 + k : rows - 1) - 2];
+  };
+  load(2);
+  for (int i0 = 2; i0 < rows; i0 += kAhead) {
+    double w[kAhead];
+#pragma unroll
+    for (int k = 0; k < kAhead; ++k) w[k] = f[k];
+    load(i0 + kAhead);
+#pragma unroll
+    for (int k = 0; k < kAhead; ++k)
+      if (i0 + k < rows) {
+        const double v = 2 * t1 - (-w[k]) * (-w[k]) * t2;
+        dt[i0 + k] = v;
+        t2 = t1;
+        t1 = v;
+      }
   }
 }
 
-// (I - b b^T) a = a - b (a.b): the metric-corrected bending term in three
-// multiply-adds per component (FAST path).
-__device__ __forceinline__ void proj_perp(const double *a, const double *b, double *out) {
-  const double ab = a[0] * b[0] + a[1] * b[1] + a[2] * b[2];
-  for (int q = 0; q < 3; ++q) out[q] = a[q] - b[q] * ab;
-}
-
-// Site mobility applied to f: f/gperp + (1/gpar - 1/gperp) t (t.f).
-__device__ __forceinline__ void mobility(double igperp, double dg, const double *t,
-                                         const double *f, double *out) {
-  const double tf = t[0] * f[0] + t[1] * f[1] + t[2] * f[2];
-  for (int q = 0; q < 3; ++q) out[q] = igperp * f[q] + dg * t[q] * tf;
+// det_b[j], kept at db[j-1] for j = 1..n, backward from the head; `rows` is
+// the block's, lanes of shorter filaments run out of entries and write to
+// their slice's spare slot db[spare]
+__device__ __forceinline__ void det_head(int rows, int n, const double *cs, double *db,
+                                         int spare) {
+  double b2 = 1.0, b1 = 2.0;
+  db[n - 1] = 1;
+  db[n - 2] = 2;
+  double f[kAhead];
+  auto load = [&](int i0) {
+#pragma unroll
+    for (int k = 0; k < kAhead; ++k) {
+      const int j = n - 1 - (i0 + k);
+      f[k] = cs[j >= 0 ? j : 0];
+    }
+  };
+  load(2);
+  for (int i0 = 2; i0 < rows; i0 += kAhead) {
+    double w[kAhead];
+#pragma unroll
+    for (int k = 0; k < kAhead; ++k) w[k] = f[k];
+    load(i0 + kAhead);
+#pragma unroll
+    for (int k = 0; k < kAhead; ++k)
+      if (i0 + k < rows) {
+        const double v = 2 * b1 - (-w[k]) * (-w[k]) * b2;
+        const int j = n - 1 - (i0 + k);
+        db[j >= 0 ? j : spare] = v;
+        b2 = b1;
+        b1 = v;
+      }
+  }
 }
 
 }  // namespace
 
-template <int G, int S, bool EXACT>
-__global__ __launch_bounds__(64) void k_integrate(Dev d, Geo g,
-                                                  const int32_t *list,
-                                                  int count, int prec) {
-  constexpr int NG = 64 / G;
-  constexpr int MAXN = G * S;
-  const Ctl *ctl = d.ctl;
-  if (ctl->abort) return;
-  const int lane = threadIdx.x;
-  const int grp = lane / G, gl = lane % G;
-  const int fidx = blockIdx.x * NG + grp;
-  const bool active = fidx < count;
+__global__ __launch_bounds__(kExactBlock) void k_integrate_exact(Dev d, Geo g, ExactBins eb) {
+  if (d.ctl->abort) return;
+  // the block's bin (uniform)
+  int bin = 0;
+#pragma unroll
+  for (int k = 1; k < kMaxBins; ++k)
+    if (k < eb.n && (int)blockIdx.x >= eb.blk0[k]) bin = k;
+  const int32_t *list = eb.list[0];
+  int count = eb.count[0], w = eb.width[0], blk0 = eb.blk0[0];
+#pragma unroll
+  for (int k = 1; k < kMaxBins; ++k)
+    if (k == bin) {
+      list = eb.list[k];
+      count = eb.count[k];
+      w = eb.width[k];
+      blk0 = eb.blk0[k];
+    }
+  const int per = exact_per_block(w), stride = exact_stride(w);
+  const int t = threadIdx.x;
+  const int grp = t / w, i = t - grp * w;  // the lane's filament and site
+  const int fidx = ((int)blockIdx.x - blk0) * per + grp;
+  const bool active = grp < per && fidx < count;
   const int f = active ? list[fidx] : 0;
   const int64_t s0 = active ? d.site_off[f] : 0;
   const int n = active ? (int)(d.site_off[f + 1] - s0) : 0;
@@ -96,543 +258,323 @@ __global__ __launch_bounds__(64) void k_integrate(Dev d, Geo g,
     sgperp = fp[5];
   }
 
-  __shared__ double U_[3][NG][MAXN], F_[3][NG][MAXN], T_[3][NG][MAXN];
-  __shared__ double R_[3][NG][MAXN], X_[3][NG][MAXN];
-  __shared__ double A_[NG][MAXN], B_[NG][MAXN], C_[NG][MAXN], D_[NG][MAXN];
-  __shared__ double CS_[NG][MAXN];
-  double *U[3] = {U_[0][grp], U_[1][grp], U_[2][grp]};
-  double *FS[3] = {F_[0][grp], F_[1][grp], F_[2][grp]};
-  double *TN[3] = {T_[0][grp], T_[1][grp], T_[2][grp]};
-  double *RR[3] = {R_[0][grp], R_[1][grp], R_[2][grp]};  // f_rand, then r_new
-  double *XX[3] = {X_[0][grp], X_[1][grp], X_[2][grp]};  // scratch
-  double *A = A_[grp], *B = B_[grp], *C = C_[grp], *Dd = D_[grp], *CS = CS_[grp];
+  __shared__ double U_[3][kSlots], F_[3][kSlots], T_[3][kSlots], R_[3][kSlots];
+  __shared__ double2 P_[kSlots];  // rows of a solve: {diagonal, right-hand side}
+  __shared__ double C_[kSlots], CS_[kSlots];
+  __shared__ double sbl[kMaxChains];
+  __shared__ int sn[kMaxChains], sfil[kMaxChains], sbad[kMaxChains], slow;
+  const int at = active ? grp * stride : 0;  // the filament's slice
+  double *U[3] = {U_[0] + at, U_[1] + at, U_[2] + at};
+  double *FS[3] = {F_[0] + at, F_[1] + at, F_[2] + at};  // site forces, then new orientations
+  double *TN[3] = {T_[0] + at, T_[1] + at, T_[2] + at};  // bond torque terms, then tangents
+  // bond force halves; random forces; determinants and K_eff; new positions
+  double *RR[3] = {R_[0] + at, R_[1] + at, R_[2] + at};
+  double2 *P = P_ + at;
+  double *CS = CS_ + at;
+  const bool site = i < n, bond = i < n - 1;
+  // the lane's row of a solve: row, unit row past the last, or none
+  const bool slot = grp < per;
+  const int row = grp * stride + i;
+  const bool sane = gpar > 0x1p-50 && gpar < 0x1p50 && gperp > 0x1p-50 && gperp < 0x1p50;
 
-  // ---- loads (issued up front; per-lane registers) ----------------------
-  double rp_reg[S][3];
-  double Fb[S][3], Tb[S][3];
-#pragma unroll
-  for (int k = 0; k < S; ++k) {
-    const int i = gl + G * k;
-    if (i < n) {
-#pragma unroll
-      for (int q = 0; q < 3; ++q) rp_reg[k][q] = mid ? d.r[q * ns + s0 + i] : d.rp[q * ns + s0 + i];
-    }
-    if (i < n - 1) {
-      const int64_t j = b0 + i;
-      double rs[3], ru[3], rl;
-      rec_read(d.br, g, j, rs, ru, &rl);
-#pragma unroll
-      for (int q = 0; q < 3; ++q) {
-        Fb[k][q] = bond_force(d, nb, q, j);
-        Tb[k][q] = bond_torque(d, nb, q, j);
-        U[q][i] = ru[q];
-      }
-    } else if (i == n - 1) {
-      double rs[3], ru[3], rl;
-      rec_read(d.br, g, b0 + n - 2, rs, ru, &rl);
-#pragma unroll
-      for (int q = 0; q < 3; ++q) U[q][i] = ru[q];
-    }
-    if (i < n && !mid && g.stoch) {
-#pragma unroll
-      for (int q = 0; q < 3; ++q)
-        RR[q][i] = g.compact ? (double)reinterpret_cast<const float *>(d.fr)[q * ns + s0 + i]
-                             : d.fr[q * ns + s0 + i];
-    }
+  // ---- loads -------------------------------------------------------------
+  double rp_reg[3], fr[3] = {0.0, 0.0, 0.0}, u[3] = {0.0, 0.0, 0.0};
+  double Fb[3], Tb[3];
+  if (i == 0 && grp < per && grp < kMaxChains) {
+    sn[grp] = n;
+    sfil[grp] = f;
+    sbl[grp] = bl;
+    sbad[grp] = 0;
   }
-  __syncthreads();
-
+  if (t == 0) slow = 0;
+  if (site) {
+    for (int q = 0; q < 3; ++q) rp_reg[q] = mid ? d.r[q * ns + s0 + i] : d.rp[q * ns + s0 + i];
+    // the last site takes the last bond's orientation
+    double rs[3], rl;
+    rec_read_full(d.br, b0 + (bond ? i : n - 2), rs, u, &rl);
+    if (bond)
+      for (int q = 0; q < 3; ++q) {
+        Fb[q] = d.bf[q * nb + b0 + i];
+        Tb[q] = d.bt[q * nb + b0 + i];
+      }
+    for (int q = 0; q < 3; ++q) U[q][i] = u[q];
+    if (!mid && g.stoch)
+      for (int q = 0; q < 3; ++q) fr[q] = d.fr[q * ns + s0 + i];
+  }
   // ---- ApplyInteractionForces (src/filament.cpp:992-1048) ----------------
-  // per bond: sf = F/2 into XX, pt = (u x T)/l into TN (TN is rebuilt below)
+  // per bond: F/2 into RR, (u x T)/l into TN (TN is rebuilt below)
   const double linv = 1.0 / bl;
-#pragma unroll
-  for (int k = 0; k < S; ++k) {
-    const int i = gl + G * k;
-    if (i < n - 1) {
-      double uj[3] = {U[0][i], U[1][i], U[2][i]};
-      double pt[3];
-      cross3(uj, Tb[k], pt);
-#pragma unroll
-      for (int q = 0; q < 3; ++q) {
-        TN[q][i] = pt[q] * linv;
-        XX[q][i] = 0.5 * Fb[k][q];
-      }
+  if (bond) {
+    double pt[3];
+    cross3(u, Tb, pt);
+    for (int q = 0; q < 3; ++q) {
+      TN[q][i] = pt[q] * linv;
+      RR[q][i] = 0.5 * Fb[q];
     }
   }
   __syncthreads();
-  double fsum[S][3];
-#pragma unroll
-  for (int k = 0; k < S; ++k) {
-    const int i = gl + G * k;
-#pragma unroll
-    for (int q = 0; q < 3; ++q) fsum[k][q] = 0.0;
-    if (i < n) {
-      if (i >= 1) {
-#pragma unroll
-        for (int q = 0; q < 3; ++q) fsum[k][q] += XX[q][i - 1];
-#pragma unroll
-        for (int q = 0; q < 3; ++q) fsum[k][q] += -TN[q][i - 1];
-      }
-      if (i <= n - 2) {
-#pragma unroll
-        for (int q = 0; q < 3; ++q) fsum[k][q] += XX[q][i];
-#pragma unroll
-        for (int q = 0; q < 3; ++q) fsum[k][q] += TN[q][i];
-      }
+  double fs[3] = {0.0, 0.0, 0.0}, um[3] = {0.0, 0.0, 0.0}, up[3] = {0.0, 0.0, 0.0};
+  double tg[3] = {0.0, 0.0, 0.0};
+  if (site) {
+    if (i >= 1) {
+      for (int q = 0; q < 3; ++q) um[q] = U[q][i - 1];
+      for (int q = 0; q < 3; ++q) fs[q] += RR[q][i - 1];
+      for (int q = 0; q < 3; ++q) fs[q] += -TN[q][i - 1];
     }
-  }
-  __syncthreads();
-  // ---- CalculateAngles / CalculateTangents ------------------------------
-#pragma unroll
-  for (int k = 0; k < S; ++k) {
-    const int i = gl + G * k;
-    if (i >= n) continue;
-#pragma unroll
-    for (int q = 0; q < 3; ++q) FS[q][i] = fsum[k][q];
-    if (i < n - 2) {
-      double a[3] = {U[0][i], U[1][i], U[2][i]};
-      double b[3] = {U[0][i + 1], U[1][i + 1], U[2][i + 1]};
-      CS[i] = dot3(a, b);
+    if (i <= n - 2) {
+      for (int q = 0; q < 3; ++q) up[q] = U[q][i + 1];
+      for (int q = 0; q < 3; ++q) fs[q] += RR[q][i];
+      for (int q = 0; q < 3; ++q) fs[q] += TN[q][i];
     }
+    // ---- CalculateAngles / CalculateTangents -----------------------------
+    if (i < n - 2) CS[i] = dot3(u, up);
     if (i == 0 || i == n - 1) {
-      const int bb = (i == 0 ? 0 : n - 2);
-#pragma unroll
-      for (int q = 0; q < 3; ++q) TN[q][i] = U[q][bb];
+      for (int q = 0; q < 3; ++q) tg[q] = u[q];  // the end bond's (see the loads)
     } else {
-      double t[3];
-#pragma unroll
-      for (int q = 0; q < 3; ++q) t[q] = U[q][i - 1] + U[q][i];
-      if (EXACT) {
-        normalize3(t);
-      } else {
-        const double inv = 1.0 / sqrt(t[0] * t[0] + t[1] * t[1] + t[2] * t[2]);
-#pragma unroll
-        for (int q = 0; q < 3; ++q) t[q] *= inv;
-      }
-#pragma unroll
-      for (int q = 0; q < 3; ++q) TN[q][i] = t[q];
+      for (int q = 0; q < 3; ++q) tg[q] = um[q] + u[q];
+      normalize3(tg);
     }
   }
   __syncthreads();
+  if (site)
+    for (int q = 0; q < 3; ++q) TN[q][i] = tg[q];
 
-  // ---- tridiagonal solve helper (EXACT: Thomas on the leader; FAST: PCR) --
-  // System rows i < m: lower coefficient in A[i] (x[i-1]), diagonal B[i],
-  // upper C[i] (x[i+1]), right-hand side D[i]; EXACT keeps the reference's
-  // layout lower[i] = A[i] coupling row i+1.
-  auto solve = [&](int m) {
-    if (EXACT) {
-      if (gl == 0 && m > 0) thomas_reg(m, A, B, C, Dd);
-      __syncthreads();
-    } else {
-      // the round count is the bin's, the same for every group of the
-      // block (barriers inside); rounds with s >= m leave a row unchanged.
-      // Each round shares 1/B through RB so a row divides once.
-      double *RB = XX[2];
-      for (int s = 1; s < MAXN; s <<= 1) {
-#pragma unroll
-        for (int k = 0; k < S; ++k) {
-          const int i = gl + G * k;
-          if (i < m) RB[i] = 1.0 / B[i];
-        }
-        __syncthreads();
-        double na[S], nbv[S], nc[S], nd[S];
-#pragma unroll
-        for (int k = 0; k < S; ++k) {
-          const int i = gl + G * k;
-          if (i >= m) continue;
-          const double ai = A[i], bi = B[i], ci = C[i], di = Dd[i];
-          double A2 = 0.0, C2 = 0.0, B2 = bi, D2 = di;
-          if (i - s >= 0) {
-            const double al = -ai * RB[i - s];
-            A2 = al * A[i - s];
-            B2 += al * C[i - s];
-            D2 += al * Dd[i - s];
-          }
-          if (i + s < m) {
-            const double ga = -ci * RB[i + s];
-            C2 = ga * C[i + s];
-            B2 += ga * A[i + s];
-            D2 += ga * Dd[i + s];
-          }
-          na[k] = A2;
-          nbv[k] = B2;
-          nc[k] = C2;
-          nd[k] = D2;
-        }
-        __syncthreads();
-#pragma unroll
-        for (int k = 0; k < S; ++k) {
-          const int i = gl + G * k;
-          if (i >= m) continue;
-          A[i] = na[k];
-          B[i] = nbv[k];
-          C[i] = nc[k];
-          Dd[i] = nd[k];
-        }
-        __syncthreads();
-      }
-#pragma unroll
-      for (int k = 0; k < S; ++k) {
-        const int i = gl + G * k;
-        if (i < m) Dd[i] = Dd[i] / B[i];
-      }
-      __syncthreads();
+  // ---- random forces (midstep) -------------------------------------------
+  const bool draws = mid && g.stoch;
+  if (draws && site) {
+    // ConstructUnprojectedRandomForces (src/filament.cpp:518-548)
+    double xi[3], xt[3];
+    draw_xi(g, (int64_t)d.noise_off[f] + i, (step - 1) >> 1, xi);
+    const double t0 = tg[0], t1 = tg[1], t2 = tg[2];
+    xt[0] = t0 * t0 * xi[0] + t0 * t1 * xi[1] + t0 * t2 * xi[2];
+    xt[1] = t1 * t1 * xi[1] + t0 * t1 * xi[0] + t1 * t2 * xi[2];
+    xt[2] = t2 * t2 * xi[2] + t0 * t2 * xi[0] + t1 * t2 * xi[1];
+    for (int q = 0; q < 3; ++q) {
+      fr[q] = sgperp * xi[q] + (sgpar - sgperp) * xt[q];
+      RR[q][i] = fr[q];
     }
+  }
+  __syncthreads();
+  // GeometricallyProjectRandomForces (src/filament.cpp:550-599)
+  auto set_row = [&](double diag, double rhs, double off) {
+    P_[row] = make_double2(diag, rhs);
+    C_[row] = off;
+    if (!sane || (off != 0.0 && dabs(off) < 0x1p-900)) slow = 1;
   };
-  // coefficients of row i of a symmetric tridiagonal system with
-  // off-diagonal o coupling rows i and i+1
-  auto put_offdiag = [&](int i, double o, int m) {
-    if (EXACT) {
-      A[i] = o;  // lower[i]: row i+1, column i
-      C[i] = o;  // upper[i]: row i, column i+1
-    } else {
-      C[i] = o;       // row i, column i+1
-      A[i + 1] = o;   // row i+1, column i
-      if (i == 0) A[0] = 0.0;
-      if (i + 1 == m - 1) C[m - 1] = 0.0;
+  double rhs = 0.0;
+  if (draws && slot) {
+    double tmp[3] = {0.0, 0.0, 0.0}, off = 0.0;
+    if (bond) {
+      for (int q = 0; q < 3; ++q) tmp[q] = RR[q][i + 1] - fr[q];
+      rhs = dot3(tmp, u);
+      if (i < n - 2) off = -CS[i];
     }
-  };
-
-  if (mid) {
-    if (g.stoch) {
-      // ConstructUnprojectedRandomForces (src/filament.cpp:518-548)
-      const int64_t mstep = (step - 1) >> 1;
-#pragma unroll
-      for (int k = 0; k < S; ++k) {
-        const int i = gl + G * k;
-        if (i >= n) continue;
-        double xi[3];
-        draw_xi(g, (int64_t)d.noise_off[f] + i, mstep, xi);
-        const double t0 = TN[0][i], t1 = TN[1][i], t2 = TN[2][i];
-        double xt[3];
-        if (EXACT) {
-          xt[0] = t0 * t0 * xi[0] + t0 * t1 * xi[1] + t0 * t2 * xi[2];
-          xt[1] = t1 * t1 * xi[1] + t0 * t1 * xi[0] + t1 * t2 * xi[2];
-          xt[2] = t2 * t2 * xi[2] + t0 * t2 * xi[0] + t1 * t2 * xi[1];
-        } else {
-          const double txi = t0 * xi[0] + t1 * xi[1] + t2 * xi[2];
-          xt[0] = t0 * txi;
-          xt[1] = t1 * txi;
-          xt[2] = t2 * txi;
-        }
-#pragma unroll
-        for (int q = 0; q < 3; ++q) RR[q][i] = sgperp * xi[q] + (sgpar - sgperp) * xt[q];
+    set_row(bond ? 2.0 : 1.0, rhs, off);
+  }
+  __syncthreads();
+  // one filament per lane: the random-force solve in the first wavefront, the
+  // determinants (into R_[0], R_[1], whose random forces are in registers by
+  // now) in the second and third
+  const int chain = t & 63, cw = t >> 6;
+  const bool runs = chain < per, fils = runs && sn[chain] > 0;
+  const int o = chain * stride;
+  if (cw == 0 && draws && runs && !thomas_chain<true>(w, P_ + o, C_ + o)) slow = 1;
+  if (cw == 1 && runs) det_tail(w, CS_ + o, R_[0] + o);
+  if (cw == 2 && fils) det_head(w, sn[chain], CS_ + o, R_[1] + o, stride - 1);
+  __syncthreads();
+  if (draws && slow) {  // numbers shared_quot does not serve
+    if (slot) {
+      P_[row] = make_double2(bond ? 2.0 : 1.0, rhs);
+      C_[row] = i < n - 2 ? -CS[i] : 0.0;
+    }
+    __syncthreads();
+    if (t == 0) slow = 0;
+    if (cw == 0 && runs) thomas_chain<false>(w, P_ + o, C_ + o);
+    __syncthreads();
+  }
+  if (mid && site) {
+    if (draws) {
+      double p[3];
+      if (i == 0) {
+        for (int q = 0; q < 3; ++q) p[q] = fr[q] + P[0].y * u[q];
+      } else if (i == n - 1) {
+        for (int q = 0; q < 3; ++q) p[q] = fr[q] - P[n - 2].y * u[q];
+      } else {
+        for (int q = 0; q < 3; ++q) p[q] = fr[q] + P[i].y * u[q] - P[i - 1].y * um[q];
       }
-      __syncthreads();
-      // GeometricallyProjectRandomForces (src/filament.cpp:550-599)
-      const int m = n - 1;
-#pragma unroll
-      for (int k = 0; k < S; ++k) {
-        const int i = gl + G * k;
-        if (i >= m) continue;
-        double tmp[3], ui[3] = {U[0][i], U[1][i], U[2][i]};
-#pragma unroll
-        for (int q = 0; q < 3; ++q) tmp[q] = RR[q][i + 1] - RR[q][i];
-        Dd[i] = dot3(tmp, ui);
-        B[i] = 2;
-        if (i < m - 1) put_offdiag(i, -CS[i], m);
-      }
-      __syncthreads();
-      solve(m);
-      // the projection of each site reads only its own unprojected force
-#pragma unroll
-      for (int k = 0; k < S; ++k) {
-        const int i = gl + G * k;
-        if (i >= n) continue;
-        double p[3];
-        if (i == 0) {
-#pragma unroll
-          for (int q = 0; q < 3; ++q) p[q] = RR[q][0] + Dd[0] * U[q][0];
-        } else if (i == n - 1) {
-#pragma unroll
-          for (int q = 0; q < 3; ++q) p[q] = RR[q][i] - Dd[n - 2] * U[q][n - 2];
-        } else {
-#pragma unroll
-          for (int q = 0; q < 3; ++q)
-            p[q] = RR[q][i] + Dd[i] * U[q][i] - Dd[i - 1] * U[q][i - 1];
-        }
-#pragma unroll
-        for (int q = 0; q < 3; ++q) {
-          if (g.compact) {  // mixed precision keeps the random force in FP32
-            p[q] = (double)(float)p[q];
-            reinterpret_cast<float *>(d.fr)[q * ns + s0 + i] = (float)p[q];
-          } else {
-            d.fr[q * ns + s0 + i] = p[q];
-          }
-          RR[q][i] = p[q];
-        }
+      for (int q = 0; q < 3; ++q) {
+        d.fr[q * ns + s0 + i] = p[q];
+        fr[q] = p[q];
       }
     }
     // Mesh::UpdatePrevPositions (src/mesh.cpp:175-182)
-#pragma unroll
-    for (int k = 0; k < S; ++k) {
-      const int i = gl + G * k;
-      if (i < n)
-#pragma unroll
-        for (int q = 0; q < 3; ++q) d.rp[q * ns + s0 + i] = rp_reg[k][q];
-    }
+    for (int q = 0; q < 3; ++q) d.rp[q * ns + s0 + i] = rp_reg[q];
   }
   // AddRandomForces (src/filament.cpp:601-606)
-  if (g.stoch) {
-#pragma unroll
-    for (int k = 0; k < S; ++k) {
-      const int i = gl + G * k;
-      if (i < n)
-#pragma unroll
-        for (int q = 0; q < 3; ++q) FS[q][i] += RR[q][i];
-    }
-  }
-  __syncthreads();
+  if (g.stoch && site)
+    for (int q = 0; q < 3; ++q) fs[q] += fr[q];
 
-  // ---- CalculateBendingForces, 3D (src/filament.cpp:608-776) ------------
-  // det_t in A[0..n-1], det_b[j] in C[j-1] for j = 1..n, k_eff in XX[0]
-  if (gl == 0 && n > 0) {
-    double t2 = 1.0, t1 = 2.0;
-    A[0] = 1;
-    A[1] = 2;
-    double b2 = 1.0, b1 = 2.0;
-    C[n - 1] = 1;
-    C[n - 2] = 2;
-    for (int i = 2; i < n; ++i) {
-      const double ca = CS[i - 2];
-      const double v = 2 * t1 - (-ca) * (-ca) * t2;
-      A[i] = v;
-      t2 = t1;
-      t1 = v;
-      const double cb = CS[n - i - 1];
-      const double w = 2 * b1 - (-cb) * (-cb) * b2;
-      C[n - i - 1] = w;
-      b2 = b1;
-      b1 = w;
-    }
+  // ---- CalculateBendingForces, 3D (src/filament.cpp:608-776) -------------
+  double *KE = RR[2];
+  if (i < n - 2) {
+    const double ginv = CS[i] * RR[0][i] * RR[1][i + 2] / RR[0][n - 1];
+    KE[i] = (kappa + bl * ginv) / (bl * bl);
   }
   __syncthreads();
-  double *KE = XX[0];
-#pragma unroll
-  for (int k = 0; k < S; ++k) {
-    const int i = gl + G * k;
-    if (i < n - 2) {
-      if (EXACT) {
-        const double ginv = CS[i] * A[i] * C[i + 2] / A[n - 1];
-        KE[i] = (kappa + bl * ginv) / (bl * bl);
-      } else {
-        const double ginv = CS[i] * A[i] * C[i + 2] * (1.0 / A[n - 1]);
-        KE[i] = (kappa + bl * ginv) * (linv * linv);
-      }
-    }
-  }
-  __syncthreads();
-#pragma unroll
-  for (int k = 0; k < S; ++k) {
-    const int kk = gl + G * k;
-    if (kk >= n) continue;
+  if (site) {
     double f3[3] = {0.0, 0.0, 0.0};
-    if (EXACT) {
-      if (kk > 1) {
-        double u1[3] = {U[0][kk - 2], U[1][kk - 2], U[2][kk - 2]};
-        double u2[3] = {U[0][kk - 1], U[1][kk - 1], U[2][kk - 1]};
-        bend_add(f3, KE[kk - 2], u1, u2);
-      }
-      if (kk > 0 && kk < n - 1) {
-        double u1[3] = {U[0][kk - 1], U[1][kk - 1], U[2][kk - 1]};
-        double u2[3] = {U[0][kk], U[1][kk], U[2][kk]};
-        bend_mid(f3, KE[kk - 1], u1, u2);
-      }
-      if (kk < n - 2) {
-        double u1[3] = {U[0][kk], U[1][kk], U[2][kk]};
-        double u2[3] = {U[0][kk + 1], U[1][kk + 1], U[2][kk + 1]};
-        bend_sub(f3, KE[kk], u1, u2);
-      }
-    } else {
-      // bond k-1 couples with k-2 and k: f_k = K_{k-2} P(u_{k-1}) u_{k-2}
-      //   + K_{k-1} [P(u_{k-1}) u_k - P(u_k) u_{k-1}] - K_k P(u_k) u_{k+1},
-      // P(b) a = (I - b b^T) a
-      double um2[3], um1[3], u0[3], up1[3], pa[3], pb[3];
-      if (kk > 1)
-        for (int q = 0; q < 3; ++q) um2[q] = U[q][kk - 2];
-      if (kk > 0)
-        for (int q = 0; q < 3; ++q) um1[q] = U[q][kk - 1];
-      for (int q = 0; q < 3; ++q) u0[q] = U[q][kk];
-      if (kk < n - 2)
-        for (int q = 0; q < 3; ++q) up1[q] = U[q][kk + 1];
-      if (kk > 1) {
-        proj_perp(um2, um1, pa);
-        const double ke = KE[kk - 2];
-        for (int q = 0; q < 3; ++q) f3[q] += ke * pa[q];
-      }
-      if (kk > 0 && kk < n - 1) {
-        proj_perp(u0, um1, pa);
-        proj_perp(um1, u0, pb);
-        const double ke = KE[kk - 1];
-        for (int q = 0; q < 3; ++q) f3[q] += ke * (pa[q] - pb[q]);
-      }
-      if (kk < n - 2) {
-        proj_perp(up1, u0, pa);
-        const double ke = KE[kk];
-        for (int q = 0; q < 3; ++q) f3[q] -= ke * pa[q];
-      }
+    if (i > 1) {
+      double u1[3] = {U[0][i - 2], U[1][i - 2], U[2][i - 2]};
+      bend_add(f3, KE[i - 2], u1, um);
     }
-#pragma unroll
-    for (int q = 0; q < 3; ++q) FS[q][kk] += f3[q];
+    if (i > 0 && i < n - 1) bend_mid(f3, KE[i - 1], um, u);
+    if (i < n - 2) bend_sub(f3, KE[i], u, up);
+    for (int q = 0; q < 3; ++q) {
+      fs[q] += f3[q];
+      FS[q][i] = fs[q];
+    }
   }
   __syncthreads();
 
-  // ---- CalculateTensions (src/filament.cpp:778-838) ---------------------
+  // ---- CalculateTensions (src/filament.cpp:778-838) ----------------------
   const double igpar = 1.0 / gpar, igperp = 1.0 / gperp;
-  {
-    const int m = n - 1;
-#pragma unroll
-    for (int k = 0; k < S; ++k) {
-      const int i = gl + G * k;
-      if (i >= m) continue;
-      double t1[3] = {TN[0][i], TN[1][i], TN[2][i]};
-      double t2[3] = {TN[0][i + 1], TN[1][i + 1], TN[2][i + 1]};
-      double f1[3] = {FS[0][i], FS[1][i], FS[2][i]};
-      double f2[3] = {FS[0][i + 1], FS[1][i + 1], FS[2][i + 1]};
-      double fd[3];
-      if (EXACT) {
-#pragma unroll
-        for (int a = 0; a < 3; ++a) {
-          double ta_ = gam(igpar, igperp, t1, a, 0) * f1[0] + gam(igpar, igperp, t1, a, 1) * f1[1];
-          ta_ += gam(igpar, igperp, t1, a, 2) * f1[2];
-          double tb_ = gam(igpar, igperp, t2, a, 0) * f2[0] + gam(igpar, igperp, t2, a, 1) * f2[1];
-          tb_ += gam(igpar, igperp, t2, a, 2) * f2[2];
-          fd[a] = tb_ - ta_;
-        }
-      } else {
-        double m1[3], m2[3];
-        mobility(igperp, igpar - igperp, t1, f1, m1);
-        mobility(igperp, igpar - igperp, t2, f2, m2);
-        for (int a = 0; a < 3; ++a) fd[a] = m2[a] - m1[a];
-      }
-      double u2[3] = {U[0][i], U[1][i], U[2][i]};
-      Dd[i] = dot3(u2, fd);
-      const double a1 = dot3(t1, u2), a2 = dot3(t2, u2);
-      B[i] = 2.0 / gperp + (1.0 / gpar - 1.0 / gperp) * (a1 * a1 + a2 * a2);
-      if (i > 0) {
-        double u1[3] = {U[0][i - 1], U[1][i - 1], U[2][i - 1]};
-        const double hu = -1.0 / gperp * dot3(u2, u1) -
-                          (1.0 / gpar - 1.0 / gperp) * (dot3(t1, u1) * dot3(t1, u2));
-        put_offdiag(i - 1, hu, m);
-      }
+  double diag = 1.0, off = 0.0;
+  rhs = 0.0;
+  if (bond) {
+    double t2[3] = {TN[0][i + 1], TN[1][i + 1], TN[2][i + 1]};
+    double f2[3] = {FS[0][i + 1], FS[1][i + 1], FS[2][i + 1]};
+    double fd[3];
+    for (int a = 0; a < 3; ++a) {
+      double ta_ = gam(igpar, igperp, tg, a, 0) * fs[0] + gam(igpar, igperp, tg, a, 1) * fs[1];
+      ta_ += gam(igpar, igperp, tg, a, 2) * fs[2];
+      double tb_ = gam(igpar, igperp, t2, a, 0) * f2[0] + gam(igpar, igperp, t2, a, 1) * f2[1];
+      tb_ += gam(igpar, igperp, t2, a, 2) * f2[2];
+      fd[a] = tb_ - ta_;
+    }
+    rhs = dot3(u, fd);
+    const double a1 = dot3(tg, u), a2 = dot3(t2, u);
+    // 2 / gperp is 2 (1 / gperp), -1 / gperp is -(1 / gperp): the same bits
+    diag = 2.0 * igperp + (igpar - igperp) * (a1 * a1 + a2 * a2);
+    // the coupling of bonds i and i+1, row i+1's (src/filament.cpp:811-818)
+    if (i < n - 2) off = -igperp * dot3(up, u) - (igpar - igperp) * (dot3(t2, u) * dot3(t2, up));
+  }
+  if (slot) set_row(diag, rhs, off);
+  __syncthreads();
+  if (cw == 0 && runs && !thomas_chain<true>(w, P_ + o, C_ + o)) slow = 1;
+  __syncthreads();
+  if (slow) {
+    if (slot) {
+      P_[row] = make_double2(diag, rhs);
+      C_[row] = off;
     }
     __syncthreads();
-    solve(m);
+    if (cw == 0 && runs) thomas_chain<false>(w, P_ + o, C_ + o);
+    __syncthreads();
   }
-#pragma unroll
-  for (int k = 0; k < S; ++k) {
-    const int i = gl + G * k;
-    if (i < n - 1) d.tension[b0 + i] = Dd[i];
-  }
+  const double ti = bond ? P[i].y : 0.0, tl = i >= 1 && site ? P[i - 1].y : 0.0;
+  if (bond) d.tension[b0 + i] = ti;
 
-  // ---- UpdateSitePositions (src/filament.cpp:840-927) -------------------
+  // ---- UpdateSitePositions (src/filament.cpp:840-927) --------------------
   const double delta = mid ? 0.5 * g.delta : g.delta;
-#pragma unroll
-  for (int k = 0; k < S; ++k) {
-    const int i = gl + G * k;
-    if (i >= n) continue;
-    double f3[3] = {FS[0][i], FS[1][i], FS[2][i]};
+  double rn[3] = {0.0, 0.0, 0.0};
+  if (site) {
+    double f3[3] = {fs[0], fs[1], fs[2]};
     if (i == 0) {
-#pragma unroll
-      for (int q = 0; q < 3; ++q) f3[q] += Dd[0] * U[q][0];
+      for (int q = 0; q < 3; ++q) f3[q] += ti * u[q];
     } else if (i == n - 1) {
-#pragma unroll
-      for (int q = 0; q < 3; ++q) f3[q] += -Dd[n - 2] * U[q][n - 2];
+      for (int q = 0; q < 3; ++q) f3[q] += -tl * u[q];
     } else {
-#pragma unroll
-      for (int q = 0; q < 3; ++q) f3[q] += Dd[i] * U[q][i] - Dd[i - 1] * U[q][i - 1];
+      for (int q = 0; q < 3; ++q) f3[q] += ti * u[q] - tl * um[q];
     }
-    double t3[3] = {TN[0][i], TN[1][i], TN[2][i]};
-    if (EXACT) {
-#pragma unroll
-      for (int a = 0; a < 3; ++a) {
-        double ft = gam(igpar, igperp, t3, a, 0) * f3[0] + gam(igpar, igperp, t3, a, 1) * f3[1];
-        ft += gam(igpar, igperp, t3, a, 2) * f3[2];
-        RR[a][i] = rp_reg[k][a] + delta * ft;
-      }
-    } else {
-      double mv[3];
-      mobility(igperp, igpar - igperp, t3, f3, mv);
-#pragma unroll
-      for (int a = 0; a < 3; ++a) RR[a][i] = rp_reg[k][a] + delta * mv[a];
+    for (int a = 0; a < 3; ++a) {
+      double ft = gam(igpar, igperp, tg, a, 0) * f3[0] + gam(igpar, igperp, tg, a, 1) * f3[1];
+      ft += gam(igpar, igperp, tg, a, 2) * f3[2];
+      rn[a] = rp_reg[a] + delta * ft;
+      RR[a][i] = rn[a];
     }
   }
   __syncthreads();
-  // new orientations in XX, CheckBondLengths (src/filament.cpp:934-951)
-  int bad = 0;
-#pragma unroll
-  for (int k = 0; k < S; ++k) {
-    const int i = gl + G * k;
-    if (i >= n - 1) continue;
-    double rd[3], mm = 0.0;
-#pragma unroll
+  // new lengths and orientations, CheckBondLengths (src/filament.cpp:934-951)
+  double rd[3] = {0.0, 0.0, 0.0}, mm = 0.0;
+  if (bond) {
     for (int q = 0; q < 3; ++q) {
-      rd[q] = RR[q][i + 1] - RR[q][i];
+      rd[q] = RR[q][i + 1] - rn[q];
       mm += rd[q] * rd[q];
     }
     mm = sqrt(mm);
-    if (EXACT) {
-#pragma unroll
-      for (int q = 0; q < 3; ++q) XX[q][i] = rd[q] / mm;
-    } else {
-      const double inv = 1.0 / mm;
-#pragma unroll
-      for (int q = 0; q < 3; ++q) XX[q][i] = rd[q] * inv;
+    for (int q = 0; q < 3; ++q) {
+      u[q] = rd[q] / mm;
+      FS[q][i] = u[q];
     }
     const double diff = bl - mm;
     const double err = (diff < 0 ? -diff : diff) / bl;
-    if (err > 1e-3) bad = 1;
+    if (err > 1e-3) sbad[grp] = 1;
   }
-  // per-group OR of the renormalisation flag
-  const unsigned long long bal = __ballot(bad);
-  const unsigned long long gmask = (G == 64) ? ~0ull : (((1ull << G) - 1ull) << (grp * G));
-  const bool renorm = (bal & gmask) != 0;
   __syncthreads();
-  if (gl == 0 && n > 0) {
-    int32_t sw = d.norm[2 * f], nn = d.norm[2 * f + 1];
-    if (renorm) {
+  if (cw == 0 && fils) {
+    const int cf = sfil[chain], cn = sn[chain];
+    int32_t sw = d.norm[2 * cf], nn = d.norm[2 * cf + 1];
+    if (sbad[chain]) {
       sw = !sw;
       nn = 0;
+      const double cbl = sbl[chain];
+      double *X = R_[0] + o, *Y = R_[1] + o, *Z = R_[2] + o;
+      const double *ux = F_[0] + o, *uy = F_[1] + o, *uz = F_[2] + o;
       if (sw) {
-        double x = RR[0][0], y = RR[1][0], z = RR[2][0];
-        for (int i = 1; i < n; ++i) {
-          x = x + bl * XX[0][i - 1];
-          y = y + bl * XX[1][i - 1];
-          z = z + bl * XX[2][i - 1];
-          RR[0][i] = x;
-          RR[1][i] = y;
-          RR[2][i] = z;
+        double x = X[0], y = Y[0], z = Z[0];
+#pragma unroll 4
+        for (int k = 1; k < cn; ++k) {
+          x = x + cbl * ux[k - 1];
+          y = y + cbl * uy[k - 1];
+          z = z + cbl * uz[k - 1];
+          X[k] = x;
+          Y[k] = y;
+          Z[k] = z;
         }
       } else {
-        double x = RR[0][n - 1], y = RR[1][n - 1], z = RR[2][n - 1];
-        for (int i = n - 1; i > 0; --i) {
-          x = x - bl * XX[0][i - 1];
-          y = y - bl * XX[1][i - 1];
-          z = z - bl * XX[2][i - 1];
-          RR[0][i - 1] = x;
-          RR[1][i - 1] = y;
-          RR[2][i - 1] = z;
+        double x = X[cn - 1], y = Y[cn - 1], z = Z[cn - 1];
+#pragma unroll 4
+        for (int k = cn - 1; k > 0; --k) {
+          x = x - cbl * ux[k - 1];
+          y = y - cbl * uy[k - 1];
+          z = z - cbl * uz[k - 1];
+          X[k - 1] = x;
+          Y[k - 1] = y;
+          Z[k - 1] = z;
         }
       }
     }
     nn++;
-    d.norm[2 * f] = sw;
-    d.norm[2 * f + 1] = nn;
+    d.norm[2 * cf] = sw;
+    d.norm[2 * cf + 1] = nn;
   }
   __syncthreads();
 
   // ---- write back sites, Mesh::UpdateBondPositions, rebuild bookkeeping --
   double lmax = 0.0;
-#pragma unroll
-  for (int k = 0; k < S; ++k) {
-    const int i = gl + G * k;
-    if (i >= n) continue;
-    double rn[3] = {RR[0][i], RR[1][i], RR[2][i]};
-#pragma unroll
+  if (site) {
+    const bool moved = sbad[grp] != 0;
+    if (moved)
+      for (int q = 0; q < 3; ++q) rn[q] = RR[q][i];
     for (int q = 0; q < 3; ++q) d.r[q * ns + s0 + i] = rn[q];
-    if (i < n - 1) {
-      double r2[3] = {RR[0][i + 1], RR[1][i + 1], RR[2][i + 1]};
-      bond_reinit(d, g, b0 + i, rn, r2, prec);
+    if (bond) {
+      if (moved) {
+        double r2[3] = {RR[0][i + 1], RR[1][i + 1], RR[2][i + 1]};
+        bond_reinit(d, g, b0 + i, rn, r2, SC_PREC_FP64);
+      } else {
+        // the length and orientation bond_reinit would compute again
+        double pos[3], sp[3];
+        for (int q = 0; q < 3; ++q) pos[q] = rn[q] + 0.5 * rd[q];
+        for (int k = 0; k < 3; ++k) {
+          double si = 0.0;
+          for (int j = 0; j < 3; ++j) si += g.hinv[3 * k + j] * pos[j];
+          si -= (double)nint(si);
+          sp[k] = si;
+        }
+        double4 *rec = reinterpret_cast<double4 *>(d.br_out + 8 * (b0 + i));
+        rec[0] = make_double4(sp[0], sp[1], sp[2], u[0]);
+        rec[1] = make_double4(u[1], u[2], mm, 0.0);
+      }
     }
     if (!mid) {
       // Mesh::UpdateDrTot for the next step's rebuild test, two
@@ -641,66 +583,62 @@ __global__ __launch_bounds__(64) void k_integrate(Dev d, Geo g,
       double a = d.acc[s0 + i];
       d.acc_prev[s0 + i] = a;
       for (int rep = 0; rep < 2; ++rep)
-#pragma unroll
         for (int q = 0; q < 3; ++q) {
           const double dd = rn[q] - d.dr0[q * ns + s0 + i];
           a += dd * dd;
         }
       d.acc[s0 + i] = a;
-      lmax = a > lmax ? a : lmax;
+      lmax = a;
     }
   }
   if (!mid) {
-#pragma unroll
     for (int o = 32; o > 0; o >>= 1) {
       const double y = __shfl_xor(lmax, o, 64);
       lmax = y > lmax ? y : lmax;
     }
-    if (lane == 0)
-      atomicMax(&d.dr_slots[(blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)) &
-                            (kDrSlots - 1)],
+    if ((t & 63) == 0)
+      atomicMax(&d.dr_slots[((int)blockIdx.x * (kExactBlock / 64) + (t >> 6)) & (kDrSlots - 1)],
                 (unsigned long long)__double_as_longlong(lmax));
   }
 }
 
-static int integrate_bin_lanes(int maxn) {
-  // lanes per filament: the bin size up to 64, then 64 with 2 or 4 sites
-  // per lane
-  return maxn <= 64 ? maxn : 64;
+void launch_integrate_exact(const Dev &d, const Geo &g, const BinDesc *bins, int n,
+                            hipStream_t st) {
+  // longest bin first
+  int order[kMaxBins];
+  ExactBins eb{};
+  for (int k = 0; k < n && eb.n < kMaxBins; ++k)
+    if (bins[k].count > 0) order[eb.n++] = k;
+  std::sort(order, order + eb.n, [&](int a, int b) { return bins[a].maxn > bins[b].maxn; });
+  int blocks = 0;
+  for (int k = 0; k < eb.n; ++k) {
+    const BinDesc &b = bins[order[k]];
+    eb.list[k] = b.list;
+    eb.count[k] = b.count;
+    eb.width[k] = b.width > 0 ? b.width : b.maxn;
+    eb.blk0[k] = blocks;
+    const int per = exact_per_block(eb.width[k]);
+    blocks += (b.count + per - 1) / per;
+  }
+  if (blocks > 0)
+    hipLaunchKernelGGL(k_integrate_exact, dim3((unsigned)blocks), dim3(kExactBlock), 0, st, d, g,
+                       eb);
 }
 
 void launch_integrate(const Dev &d, const Geo &g, const int32_t *bin_list,
                       int bin_count, int bin_maxn, int precision, const Tune &t, bool mid,
                       hipStream_t st) {
   if (bin_count <= 0) return;
-  // fast path: register-resident variants
+  if (precision == SC_PREC_FP64) {
+    const BinDesc b = {bin_list, bin_count, bin_maxn, 0};
+    launch_integrate_exact(d, g, &b, 1, st);
+    return;
+  }
+  // mixed precision: register-resident variants
   if (launch_integrate_long(d, g, bin_list, bin_count, bin_maxn, precision, t.int_waves,
                             t.int_layout, mid, st))
     return;
-  if (launch_integrate_reg(d, g, bin_list, bin_count, bin_maxn, precision, t.int_waves, st))
-    return;
-  const bool exact = precision == SC_PREC_FP64;
-  const int G = integrate_bin_lanes(bin_maxn);
-  const int per_wave = 64 / G;
-  dim3 grid((bin_count + per_wave - 1) / per_wave), block(64);
-#define SC_LAUNCH(GG, SS)                                                          \
-  do {                                                                             \
-    if (exact)                                                                     \
-      hipLaunchKernelGGL((k_integrate<GG, SS, true>), grid, block, 0, st, d, g,    \
-                         bin_list, bin_count, precision);                          \
-    else                                                                           \
-      hipLaunchKernelGGL((k_integrate<GG, SS, false>), grid, block, 0, st, d, g,   \
-                         bin_list, bin_count, precision);                          \
-  } while (0)
-  switch (bin_maxn) {
-    case 8: SC_LAUNCH(8, 1); break;
-    case 16: SC_LAUNCH(16, 1); break;
-    case 32: SC_LAUNCH(32, 1); break;
-    case 64: SC_LAUNCH(64, 1); break;
-    case 128: SC_LAUNCH(64, 2); break;
-    default: SC_LAUNCH(64, 4); break;
-  }
-#undef SC_LAUNCH
+  (void)launch_integrate_reg(d, g, bin_list, bin_count, bin_maxn, precision, t.int_waves, st);
 }
 
 }  // namespace sc

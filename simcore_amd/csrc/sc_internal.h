@@ -195,7 +195,15 @@ struct BinDesc {
   const int32_t *list;  // filament indices of the bin (packed: lane table)
   int count;            // filaments (packed: wavefronts)
   int maxn;             // 8, 16, 32, 64, 128 or 256 sites; 0: packed waves
-  int width;            // packed: lane-group width of the waves (16/32/64)
+  int width;            // packed: lane-group width of the waves (16/32/64);
+                        // else the sites of the longest filament (0: maxn)
+};
+
+// Bins of one FP64 integrator launch: bin k takes blocks [blk0[k], ...).
+struct ExactBins {
+  int n;
+  int32_t blk0[kMaxBins], count[kMaxBins], width[kMaxBins];
+  const int32_t *list[kMaxBins];
 };
 
 // Grouped launches: one launch steps several independent systems (a batch
@@ -288,6 +296,9 @@ void launch_pair_range(const Dev &d, const Geo &g, int precision, const Tune &t,
 void launch_integrate(const Dev &d, const Geo &g, const int32_t *bin_list,
                       int bin_count, int bin_maxn, int precision, const Tune &t, bool mid,
                       hipStream_t st);
+// FP64: every bin in one launch
+void launch_integrate_exact(const Dev &d, const Geo &g, const BinDesc *bins, int n,
+                            hipStream_t st);
 // register-resident fast-path integrator; false when the bin is not one it
 // serves (FP64 precision or more than 64 sites), nothing launched then
 bool launch_integrate_reg(const Dev &d, const Geo &g, const int32_t *bin_list,
