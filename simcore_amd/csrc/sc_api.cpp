@@ -25,6 +25,7 @@ struct Bin {
   int longest = 0;  // sites of its longest filament
   int count = 0;
   int32_t *list = nullptr;
+  int4 *entries = nullptr;  // FP64 (see BinDesc)
   std::vector<int64_t> last;  // last bond of each listed filament (ascending)
 };
 
@@ -396,7 +397,8 @@ void enqueue_step(sc_system *h, bool odd, Commit how) {
     const bool packed = h->tune.int_layout >= 2 && h->pack_waves > 0;
     for (const Bin &b : h->bins)
       if (b.maxn > 128)
-        sc::launch_integrate(d, g, b.list, b.count, b.maxn, h->p.precision, h->tune, odd, sl);
+        sc::launch_integrate(d, g, {b.list, b.entries, b.count, b.maxn, b.longest},
+                             h->p.precision, h->tune, odd, sl);
     (void)hipEventRecord(h->join_ev[1], sl);
     sc::launch_pair_range(d, g, h->p.precision, h->tune, st, g.thermo != 0, cut, nb);
     if (packed && h->tune.int_layout == 2) {
@@ -411,7 +413,8 @@ void enqueue_step(sc_system *h, bool odd, Commit how) {
     }
     for (const Bin &b : h->bins)
       if (b.maxn <= 128 && !packed)
-        sc::launch_integrate(d, g, b.list, b.count, b.maxn, h->p.precision, h->tune, odd, st);
+        sc::launch_integrate(d, g, {b.list, b.entries, b.count, b.maxn, b.longest},
+                             h->p.precision, h->tune, odd, st);
     (void)hipStreamWaitEvent(st, h->join_ev[1], 0);
     if (commit) sc::launch_commit(d, g, st);
     return;
@@ -458,8 +461,10 @@ void enqueue_step(sc_system *h, bool odd, Commit how) {
         const int i0 = p == 0 ? 0 : first_at(b.last, lo);
         const int i1 = p + 1 < P ? first_at(b.last, hi) : b.count;
         if (i1 > i0)
-          sc::launch_integrate(d, g, b.list + i0, i1 - i0, b.maxn, h->p.precision, h->tune,
-                               odd, packed ? sl : si);
+          sc::launch_integrate(d, g,
+                               {b.list + i0, b.entries ? b.entries + i0 : nullptr, i1 - i0,
+                                b.maxn, b.longest},
+                               h->p.precision, h->tune, odd, packed ? sl : si);
       }
     }
     for (int k = 0; k < 2; ++k) {
@@ -490,16 +495,16 @@ void enqueue_step(sc_system *h, bool odd, Commit how) {
   if (packed && h->tune.int_layout == 2) {
     for (const Bin &b : h->bins)
       if (b.maxn == 256) merged = &b;
-    bins[nbins++] = {h->pack_tab, h->pack_waves, 0, 0};
+    bins[nbins++] = {h->pack_tab, nullptr, h->pack_waves, 0, 0};
   } else if (packed) {
     for (int c = 0; c < 3; ++c)
       if (h->pack_cs[c + 1] > h->pack_cs[c])
-        bins[nbins++] = {h->pack_tab + (int64_t)64 * h->pack_cs[c],
+        bins[nbins++] = {h->pack_tab + (int64_t)64 * h->pack_cs[c], nullptr,
                          h->pack_cs[c + 1] - h->pack_cs[c], 0, 16 << c};
   }
   for (const Bin &b : h->bins)
     if ((!packed || b.maxn > 128) && &b != merged)
-      bins[nbins++] = {b.list, b.count, b.maxn,
+      bins[nbins++] = {b.list, b.entries, b.count, b.maxn,
                        h->p.precision == SC_PREC_FP64 ? b.longest : 0};
   auto load_of = [&](int k) -> int64_t {
     if (bins[k].maxn) return (int64_t)bins[k].count * bins[k].maxn;
@@ -517,8 +522,7 @@ void enqueue_step(sc_system *h, bool odd, Commit how) {
       sc::launch_integrate_packed(d, g, bins[k].list, bins[k].count, bins[k].width,
                                   h->tune.int_waves, odd, sk);
     else
-      sc::launch_integrate(d, g, bins[k].list, bins[k].count, bins[k].maxn, h->p.precision,
-                           h->tune, odd, sk);
+      sc::launch_integrate(d, g, bins[k], h->p.precision, h->tune, odd, sk);
   };
   if (h->p.precision == SC_PREC_FP64 && !h->tune.int_streams) {
     sc::launch_integrate_exact(d, g, bins, nbins, st);
@@ -1043,6 +1047,8 @@ size_t system_estimate_bytes(const sc_params *params, int32_t nf, int64_t ns, in
   const int64_t tmp = scan_tmp_elems(ncol, nb);
   b += R(4 * tmp);
   b += R(4 * (int64_t)nf) + (size_t)n_bins * Arena::kAlign;  // bin lists
+  if (params->precision == SC_PREC_FP64)
+    b += R(16 * (int64_t)nf) + (size_t)n_bins * Arena::kAlign;
   if (params->precision == SC_PREC_MIXED)  // packed layout: at most one wave per filament
     b += R(4 * 64 * (int64_t)nf) + R(4 * (int64_t)nf);
   const int64_t cap = initial_capacity(*params, nb);
@@ -1313,6 +1319,7 @@ int sc_load_filaments(sc_handle h, int32_t nf, const int32_t *site_off,
   const int bin_max[] = {8, 16, 32, 64, 128, 256};
   constexpr int kBins = 6;
   std::vector<std::vector<int32_t>> lists(kBins);
+  std::vector<std::vector<int4>> entries(kBins);  // alive until the copies have run
   for (int f = 0; f < nf; ++f) {
     int n = site_off[f + 1] - site_off[f];
     for (int k = 0; k < kBins; ++k)
@@ -1334,6 +1341,13 @@ int sc_load_filaments(sc_handle h, int32_t nf, const int32_t *site_off,
     if ((rc = dalloc(h, &b.list, lists[k].size(), false))) return rc;
     HIPCHK(h, hipMemcpyAsync(b.list, lists[k].data(), sizeof(int32_t) * lists[k].size(),
                              hipMemcpyHostToDevice, h->stream));
+    if (h->p.precision == SC_PREC_FP64) {
+      for (int32_t f : lists[k])
+        entries[k].push_back(make_int4(f, site_off[f], site_off[f + 1] - site_off[f], 0));
+      if ((rc = dalloc(h, &b.entries, entries[k].size(), false))) return rc;
+      HIPCHK(h, hipMemcpyAsync(b.entries, entries[k].data(), sizeof(int4) * entries[k].size(),
+                               hipMemcpyHostToDevice, h->stream));
+    }
     h->bins.push_back(b);
   }
   // (host arrays of the packed layout live until the copies below have run)

@@ -219,13 +219,15 @@ __device__ __forceinline__ void det_head(int rows, int n, const double *cs, doub
 }  // namespace
 
 __global__ __launch_bounds__(kExactBlock) void k_integrate_exact(Dev d, Geo g, ExactBins eb) {
-  if (d.ctl->abort) return;
+  // (an aborted step leaves every lane inactive rather than returning: the
+  // list and site loads then need not wait for the control block)
+  const bool live = d.ctl->abort == 0;
   // the block's bin (uniform)
   int bin = 0;
 #pragma unroll
   for (int k = 1; k < kMaxBins; ++k)
     if (k < eb.n && (int)blockIdx.x >= eb.blk0[k]) bin = k;
-  const int32_t *list = eb.list[0];
+  const int4 *list = eb.list[0];
   int count = eb.count[0], w = eb.width[0], blk0 = eb.blk0[0];
 #pragma unroll
   for (int k = 1; k < kMaxBins; ++k)
@@ -239,10 +241,10 @@ __global__ __launch_bounds__(kExactBlock) void k_integrate_exact(Dev d, Geo g, E
   const int t = threadIdx.x;
   const int grp = t / w, i = t - grp * w;  // the lane's filament and site
   const int fidx = ((int)blockIdx.x - blk0) * per + grp;
-  const bool active = grp < per && fidx < count;
-  const int f = active ? list[fidx] : 0;
-  const int64_t s0 = active ? d.site_off[f] : 0;
-  const int n = active ? (int)(d.site_off[f + 1] - s0) : 0;
+  const bool listed = grp < per && fidx < count, active = listed && live;
+  const int4 ent = listed ? list[fidx] : make_int4(0, 0, 0, 0);
+  const int f = ent.x, n = live ? ent.z : 0;
+  const int64_t s0 = ent.y;
   const int64_t b0 = s0 - f;
   const int64_t ns = g.ns, nb = g.nb;
   const bool mid = step_is_mid(d);
@@ -613,7 +615,7 @@ void launch_integrate_exact(const Dev &d, const Geo &g, const BinDesc *bins, int
   int blocks = 0;
   for (int k = 0; k < eb.n; ++k) {
     const BinDesc &b = bins[order[k]];
-    eb.list[k] = b.list;
+    eb.list[k] = b.entries;
     eb.count[k] = b.count;
     eb.width[k] = b.width > 0 ? b.width : b.maxn;
     eb.blk0[k] = blocks;
@@ -625,20 +627,18 @@ void launch_integrate_exact(const Dev &d, const Geo &g, const BinDesc *bins, int
                        eb);
 }
 
-void launch_integrate(const Dev &d, const Geo &g, const int32_t *bin_list,
-                      int bin_count, int bin_maxn, int precision, const Tune &t, bool mid,
-                      hipStream_t st) {
-  if (bin_count <= 0) return;
+void launch_integrate(const Dev &d, const Geo &g, const BinDesc &bin, int precision,
+                      const Tune &t, bool mid, hipStream_t st) {
+  if (bin.count <= 0) return;
   if (precision == SC_PREC_FP64) {
-    const BinDesc b = {bin_list, bin_count, bin_maxn, 0};
-    launch_integrate_exact(d, g, &b, 1, st);
+    launch_integrate_exact(d, g, &bin, 1, st);
     return;
   }
   // mixed precision: register-resident variants
-  if (launch_integrate_long(d, g, bin_list, bin_count, bin_maxn, precision, t.int_waves,
+  if (launch_integrate_long(d, g, bin.list, bin.count, bin.maxn, precision, t.int_waves,
                             t.int_layout, mid, st))
     return;
-  (void)launch_integrate_reg(d, g, bin_list, bin_count, bin_maxn, precision, t.int_waves, st);
+  (void)launch_integrate_reg(d, g, bin.list, bin.count, bin.maxn, precision, t.int_waves, st);
 }
 
 }  // namespace sc

@@ -193,6 +193,9 @@ constexpr int64_t kPairAlign = 512;  // range cuts: a multiple of every block si
 constexpr int kMaxBins = 6;
 struct BinDesc {
   const int32_t *list;  // filament indices of the bin (packed: lane table)
+  const int4 *entries;  // FP64: {filament, first site, sites, 0} of the listed
+                        // filaments, so that the sites can be loaded as soon
+                        // as the entry is there
   int count;            // filaments (packed: wavefronts)
   int maxn;             // 8, 16, 32, 64, 128 or 256 sites; 0: packed waves
   int width;            // packed: lane-group width of the waves (16/32/64);
@@ -203,7 +206,7 @@ struct BinDesc {
 struct ExactBins {
   int n;
   int32_t blk0[kMaxBins], count[kMaxBins], width[kMaxBins];
-  const int32_t *list[kMaxBins];
+  const int4 *list[kMaxBins];
 };
 
 // Grouped launches: one launch steps several independent systems (a batch
@@ -293,9 +296,8 @@ int64_t pair_blocks(const Geo &g, const Tune &t);
 void launch_pair_range(const Dev &d, const Geo &g, int precision, const Tune &t, hipStream_t st,
                        bool thermo, int64_t b_lo, int64_t b_hi);  // blocks of one pair launch
 // `mid`: the step is a midstep (odd step index)
-void launch_integrate(const Dev &d, const Geo &g, const int32_t *bin_list,
-                      int bin_count, int bin_maxn, int precision, const Tune &t, bool mid,
-                      hipStream_t st);
+void launch_integrate(const Dev &d, const Geo &g, const BinDesc &bin, int precision,
+                      const Tune &t, bool mid, hipStream_t st);
 // FP64: every bin in one launch
 void launch_integrate_exact(const Dev &d, const Geo &g, const BinDesc *bins, int n,
                             hipStream_t st);
