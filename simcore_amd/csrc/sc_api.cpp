@@ -1032,14 +1032,14 @@ size_t system_estimate_bytes(const sc_params *params, int32_t nf, int64_t ns, in
   const int64_t n_cells = n1d * n1d * n1d;
   const int64_t nb = ns - nf;
   auto R = [](int64_t n) { return Arena::round((size_t)(n > 0 ? n : 1)); };
-  size_t b = R(sizeof(Ctl)) + R(8 * sc::kDrSlots) + R(4 * (nf + 1)) + 2 * R(4 * (int64_t)nf) +
+  size_t b = R(sizeof(Ctl)) + R(8 * sc::kDrSlots) + R(sizeof(sc::RebuildBar)) + R(4 * (nf + 1)) + 2 * R(4 * (int64_t)nf) +
              R(64 * (int64_t)nf) +
              R(8 * (int64_t)nf) + R(4 * nb);
   b += 4 * R(24 * ns) + 2 * R(8 * ns);                    // r, rp, fr, dr0, acc, acc_prev
   const int64_t rec_bytes = params->precision == SC_PREC_MIXED ? 32 : 64;
   b += R(rec_bytes * nb) + 2 * R(24 * nb) + R(8 * nb);    // record, F, T (at most), tension
   const int64_t ncol = n1d * n1d, occ_words = (n1d + 31) / 32;
-  b += R(4 * nb) + R(4 * ncol) + R(4 * (ncol + 1)) + 2 * R(4 * nb);  // keys, columns, col_tmp/rank
+  b += R(4 * nb) + R(4 * ncol) + R(4 * (ncol + 1)) + R(8 * nb) + R(4 * nb);  // keys, columns, col_tmp, col_rank
   b += R(8 * n_cells) + R(4 * ncol * occ_words);                 // cell runs, occupancy
   b += R(2 * ncol * occ_words) + R(4 * ncol) + R(4 * nb);        // run tables
   b += 2 * R(4 * nb) + R(4 * nb) + R(4 * (nb + 1));  // sorted, skey, deg, inc_start
@@ -1219,6 +1219,8 @@ int sc_load_filaments(sc_handle h, int32_t nf, const int32_t *site_off,
   if ((rc = dalloc(h, &d.dr_slots, sc::kDrSlots, false))) return rc;
   HIPCHK(h, hipMemsetAsync(d.dr_slots, 0, sizeof(unsigned long long) * sc::kDrSlots,
                            h->stream));
+  if ((rc = dalloc(h, &d.bar, 1, false))) return rc;
+  HIPCHK(h, hipMemsetAsync(d.bar, 0, sizeof(sc::RebuildBar), h->stream));
   if ((rc = dalloc(h, &d.site_off, nf + 1, false))) return rc;
   if ((rc = dalloc(h, &d.noise_off, nf, false))) return rc;
   if ((rc = dalloc(h, &d.fil_caller, nf, false))) return rc;
@@ -2097,6 +2099,9 @@ int sc_checkpoint_load(sc_handle h, const void *buf, size_t size) {
     p += f.bytes;
   }
   if ((rc = write_ctl(h, hd.ctl))) return rc;
+  // (a run that ended in an error leaves its displacement maxima behind)
+  HIPCHK(h, hipMemsetAsync(h->d.dr_slots, 0, sizeof(unsigned long long) * sc::kDrSlots,
+                           h->stream));
   // cell membership of the saved state's last rebuild (used between
   // rebuilds by the crosslink partner search)
   sc::launch_cells_from_keys(h->d, h->g, h->stream);

@@ -81,12 +81,24 @@ struct Geo {
 // slots into Ctl::dr_bits and clears them.
 constexpr int kDrSlots = 256;
 
+// Counters of the one-launch rebuild stage (sc_kernels.hip), zero between
+// launches; one cache line per counter that several blocks add to.
+constexpr int kBars = 6, kBarGroups = 16;
+struct RebuildBar {
+  uint32_t arrived, parts, gone;
+  int32_t abort, err, overflow;  // for Ctl, when the launch ends
+  uint32_t pad[10];
+  uint32_t full[kBars][16];
+  uint32_t group[kBars][kBarGroups][16];
+};
+
 struct Dev {
   Ctl *ctl;
   int ahead;               // steps taken since the last commit of Ctl: 1 on an
                            // even step that follows its odd step without a
                            // commit between them, else 0
-  unsigned long long *dr_slots;  // kDrSlots, zero between steps
+  unsigned long long *dr_slots;  // kDrSlots, zero between runs of steps
+  RebuildBar *bar;
   // filaments
   int32_t *site_off;       // nf+1
   int32_t *noise_off;      // nf: site index the noise stream is keyed by
@@ -115,7 +127,7 @@ struct Dev {
   int32_t *col_count;      // n1d^2: column populations (zero between builds)
   int32_t *col_start;      // n1d^2 + 1: column starts in sorted
   int32_t *col_rank;       // nb: a bond's place in its column (build scratch)
-  int32_t *col_tmp;        // nb: bonds grouped by column, unordered
+  int64_t *col_tmp;        // nb: key << 32 | bond, grouped by column, unordered
   int32_t *sorted, *skey;  // nb: bonds in (key, bond) order, their keys
   int2 *cell_run;          // n_cells: [start, end) of an occupied cell
   uint32_t *cell_occ;      // n1d^2 * occ_words: bit z of column (x, y)

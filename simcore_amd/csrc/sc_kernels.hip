@@ -294,35 +294,38 @@ constexpr int kColScanBlock = 1024;
 constexpr int kColScanTile = 4 * kColScanBlock;
 constexpr int64_t kColScanMax = (int64_t)1 << 17;
 
-// sum of v over the block; `ws` holds one int per wavefront
-template <int BLOCK>
+// Sum of v over each SUB consecutive threads of a block; `ws` holds one int
+// per wavefront of the block.
+template <int SUB>
 __device__ __forceinline__ int block_sum(int v, int *ws) {
   for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
   if ((threadIdx.x & 63) == 0) ws[threadIdx.x >> 6] = v;
   __syncthreads();
+  const int w0 = (int)threadIdx.x / SUB * (SUB / 64);
   int t = 0;
 #pragma unroll
-  for (int i = 0; i < BLOCK / 64; ++i) t += ws[i];
+  for (int i = 0; i < SUB / 64; ++i) t += ws[w0 + i];
   __syncthreads();
   return t;
 }
 
-// exclusive scan of v over the block
-template <int BLOCK>
+// exclusive scan of v over each SUB consecutive threads
+template <int SUB>
 __device__ __forceinline__ int block_excl(int v, int *total, int *ws) {
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, w0 = (int)threadIdx.x / SUB * (SUB / 64);
+  const int w = ((int)threadIdx.x >> 6) - w0;
   int x = v;
 #pragma unroll
   for (int o = 1; o < 64; o <<= 1) {
     const int y = __shfl_up(x, o, 64);
     if (lane >= o) x += y;
   }
-  if (lane == 63) ws[w] = x;
+  if (lane == 63) ws[threadIdx.x >> 6] = x;
   __syncthreads();
   int base = 0, tot = 0;
 #pragma unroll
-  for (int i = 0; i < BLOCK / 64; ++i) {
-    const int t = ws[i];
+  for (int i = 0; i < SUB / 64; ++i) {
+    const int t = ws[w0 + i];
     if (i < w) base += t;
     tot += t;
   }
@@ -331,6 +334,7 @@ __device__ __forceinline__ int block_excl(int v, int *total, int *ws) {
   return base + x - v;
 }
 
+// (kColScanBlock threads)
 __device__ __forceinline__ void colscan_body(const Dev &d, int64_t ncol, int64_t tile) {
   __shared__ int ws[kColScanBlock / 64];
   const int64_t base = tile * kColScanTile;
@@ -384,7 +388,7 @@ static void launch_colscan(const Dev &d, int64_t ncol, int guard, hipStream_t st
 // n1d^3, so the scan that follows is small), with each bond's place in its
 // column.  Streaming passes loop over their range, so any grid size serves.
 // The column counts are aggregated per block tile first: each bond enters
-// its column into an LDS hash table (linear probing; a tile of kScanBlock
+// its column into an LDS hash table (linear probing; a tile of BLOCK
 // bonds has at most that many columns, so it always fits) and takes its
 // place among the tile's bonds of that column from an LDS counter; one
 // device-scope atomic per distinct column of the tile then hands out the
@@ -392,15 +396,24 @@ static void launch_colscan(const Dev &d, int64_t ncol, int guard, hipStream_t st
 // a few tens of columns, so the device-scope atomics (which on MI355X go
 // past the XCD's L2 to memory) drop by an order of magnitude.  A bond's
 // place is any unique slot of its column; the column sort orders them.
-__device__ __forceinline__ void keys_body(const Dev &d, const Geo &g, int64_t bid, int64_t nblk) {
-  __shared__ int32_t hcol[kScanBlock], hcnt[kScanBlock], hbase[kScanBlock];
+template <int BLOCK>
+struct KeysLds {
+  int32_t col[BLOCK], cnt[BLOCK], base[BLOCK];
+};
+
+template <int BLOCK>
+__device__ __forceinline__ void keys_body(const Dev &d, const Geo &g, int64_t bid, int64_t nblk,
+                                          KeysLds<BLOCK> &L) {
+  int32_t *hcol = L.col, *hcnt = L.cnt, *hbase = L.base;
+  constexpr int kHashShift = BLOCK == 1024 ? 22 : 24;  // hash bits: log2(BLOCK)
+  static_assert(BLOCK == 256 || BLOCK == 1024, "hash bits");
   const int t = threadIdx.x;
-  const int64_t ntiles = (g.nb + kScanBlock - 1) / kScanBlock;
+  const int64_t ntiles = (g.nb + BLOCK - 1) / BLOCK;
   for (int64_t tile = bid; tile < ntiles; tile += nblk) {
     hcol[t] = -1;
     hcnt[t] = 0;
     __syncthreads();
-    const int64_t b = tile * kScanBlock + t;
+    const int64_t b = tile * BLOCK + t;
     int32_t k = 0, slot = 0, local = 0;
     if (b < g.nb) {
       if (g.compact) {
@@ -410,11 +423,11 @@ __device__ __forceinline__ void keys_body(const Dev &d, const Geo &g, int64_t bi
         k = cell_key(g.n1d, rec[0], rec[1], rec[2]);
       }
       const int32_t c = k / g.n1d;
-      slot = (int32_t)(((uint32_t)c * 2654435761u) >> 24);  // 8 bits of a multiplicative hash
+      slot = (int32_t)(((uint32_t)c * 2654435761u) >> kHashShift);  // multiplicative hash
       for (;;) {
         const int32_t prev = atomicCAS(&hcol[slot], -1, c);
         if (prev == -1 || prev == c) break;
-        slot = (slot + 1) & (kScanBlock - 1);
+        slot = (slot + 1) & (BLOCK - 1);
       }
       local = atomicAdd(&hcnt[slot], 1);
     }
@@ -434,25 +447,26 @@ __device__ __forceinline__ void keys_body(const Dev &d, const Geo &g, int64_t bi
 // block that loads and stores a few words).  Every block folds the
 // displacement slots and takes the decision for itself from values that no
 // block of this launch changes; block 0 also stores it in Ctl for the
-// launches that follow.  The slots are cleared by the column scatter, after
-// every block has read them and before a full step fills them again.  Returns
+// launches that follow.  The slots need no clearing for the next full step:
+// the accumulators, hence their maximum, only grow until a rebuild zeroes
+// them, and the rebuild's column scatter clears the slots too.  Returns
 // whether the odd step rebuilds.
 __device__ __forceinline__ bool fold_commit(const Dev &d, double thr, bool first) {
-  static_assert(kDrSlots == kScanBlock, "one slot per thread");
-  __shared__ unsigned long long wmax[kScanBlock / 64];
+  static_assert(kDrSlots == 256, "one slot per thread of the first four wavefronts");
+  __shared__ unsigned long long wmax[4];
   __shared__ int off;
   Ctl *c = d.ctl;
-  unsigned long long m = d.dr_slots[threadIdx.x];
+  unsigned long long m = threadIdx.x < kDrSlots ? d.dr_slots[threadIdx.x] : 0ull;
   if (threadIdx.x == 0) off = c->abort;
   for (int o = 32; o > 0; o >>= 1) {
     const unsigned long long y = __shfl_xor(m, o, 64);
     m = y > m ? y : m;
   }
-  if ((threadIdx.x & 63) == 0) wmax[threadIdx.x >> 6] = m;
+  if ((threadIdx.x & 63) == 0 && threadIdx.x < kDrSlots) wmax[threadIdx.x >> 6] = m;
   __syncthreads();
   if (off) return false;
 #pragma unroll
-  for (int i = 0; i < kScanBlock / 64; ++i) m = wmax[i] > m ? wmax[i] : m;
+  for (int i = 0; i < 4; ++i) m = wmax[i] > m ? wmax[i] : m;
   const double drm = __longlong_as_double((long long)m);
   const bool lost = drm > 10000;  // include/simcore/species.hpp:114-118
   const bool rb = !lost && drm > thr;
@@ -477,7 +491,8 @@ __global__ __launch_bounds__(kScanBlock) void k_keys(Dev d, Geo g) {
   } else {
     if (guard_off(d.ctl, kGuardRebuild)) return;
   }
-  keys_body(d, g, blockIdx.x, gridDim.x);
+  __shared__ KeysLds<kScanBlock> L;
+  keys_body<kScanBlock>(d, g, blockIdx.x, gridDim.x, L);
 }
 
 // Column populations from the stored keys (cell list restore).
@@ -489,125 +504,154 @@ __global__ void k_key_count(Dev d, Geo g) {
 
 // Groups the bonds by column at the place the population count handed
 // each bond (order inside a column arbitrary; the rank sort orders it): a
-// pure scatter, no atomics.
+// pure scatter, no atomics.  The key travels with the bond, so the column sort
+// need not gather it.
 __device__ __forceinline__ void scatter_body(const Dev &d, const Geo &g, int64_t bid,
                                              int64_t nblk) {
   const int64_t stride = nblk * blockDim.x;
   for (int64_t b = bid * blockDim.x + threadIdx.x; b < g.nb; b += stride) {
-    const int32_t c = d.keys[b] / g.n1d;
-    d.col_tmp[d.col_start[c] + d.col_rank[b]] = (int32_t)b;
+    const int32_t k = d.keys[b];
+    d.col_tmp[d.col_start[k / g.n1d] + d.col_rank[b]] = ((int64_t)k << 32) | (uint32_t)b;
   }
 }
 
-// (the displacement slots of the step before are done with here, see
-// fold_commit; between steps they are zero anyway)
+// (of the steps before the rebuild, see fold_commit)
 __device__ __forceinline__ void clear_dr_slots(const Dev &d) {
   for (int i = threadIdx.x; i < kDrSlots; i += blockDim.x) d.dr_slots[i] = 0ull;
 }
 
 __global__ void k_scatter(Dev d, Geo g, int guard) {
-  if (blockIdx.x == 0) clear_dr_slots(d);
   if (guard_off(d.ctl, guard)) return;
+  if (blockIdx.x == 0) clear_dr_slots(d);
   scatter_body(d, g, blockIdx.x, gridDim.x);
 }
 
-// Each cell column sorted by (cell key, bond index): one wavefront per
-// column; an entry's place is the number of smaller (key, bond) pairs in
-// its column, counted against the column staged in LDS (a column holds a
-// few tens of bonds at the densities simulated; longer ones than the stage
-// count against global memory).  Members of a cell thus appear in bond
-// order, the order Cell::AddObj appends in (src/cell.cpp:5-8).  The pass
-// also writes the column's occupancy words (every word of the column, so
-// no clearing pass is needed) with each word's count of occupied cells
-// before it, and the column's run table: the first sorted entry of each
-// occupied cell in z order, at the column's own range of `cell_first`, and
-// the number of occupied cells.  The degree pass finds a cell's run from
-// its rank among the column's occupied cells (cell_run_of) in these small,
-// L2-resident arrays, which cut its HBM reads from 540 to 200 MB on the
-// uneven 1.6M-bond system; the cell-indexed runs (n1d^3 entries, mostly
-// empty, so every lookup is a random HBM line) serve the list pass's rare
-// lookups beyond a bond's run slab (measured faster there) and the
-// crosslink partner search.
-constexpr int kColStage = 256;
+// Each cell column sorted by (cell key, bond index): kColLanes lanes per
+// column; an entry's place is the number of smaller (key, bond) pairs in its
+// column, counted against the column staged in LDS (a column holds a few tens
+// of bonds at the densities simulated; longer ones than the stage count
+// against global memory).  Members of a cell thus appear in bond order, the
+// order Cell::AddObj appends in (src/cell.cpp:5-8).  The pass also writes the
+// column's occupancy words (every word of the column, so no clearing pass is
+// needed) with each word's count of occupied cells before it, and the column's
+// run table: the first sorted entry of each occupied cell in z order, at the
+// column's own range of `cell_first`, and the number of occupied cells.  The
+// degree pass finds a cell's run from its rank among the column's occupied
+// cells (cell_run_of) in these small, L2-resident arrays, which cut its HBM
+// reads from 540 to 200 MB on the uneven 1.6M-bond system; the cell-indexed
+// runs (n1d^3 entries, mostly empty, so every lookup is a random HBM line)
+// serve the list pass's rare lookups beyond a bond's run slab (measured faster
+// there) and the crosslink partner search.
+//
+// A column's lanes lie in one wavefront and share nothing with others, so the
+// pass has no block barrier.  Bound: the latency of a column's few loads.
+// Sixteen lanes keep 4 columns in flight per wavefront and most lanes busy at
+// 2-30 bonds a column.  Active: uneven 1.6M bonds 44 us, dense 620k 21 us (one
+// column per wavefront, keys gathered: 46 and 24.5); in the one-launch rebuild,
+// where a few hundred wavefronts serve all columns, 52k bonds gained 1.1 us a
+// step.
+constexpr int kColLanes = 16;
+constexpr int kColStage = 96;
+constexpr int kOccWords = 44;  // occ_words <= 41 (n1d^3 < 2^31)
 
-__device__ __forceinline__ int64_t kb_pair(const Dev &d, int32_t b) {
-  return ((int64_t)d.keys[b] << 32) | (uint32_t)b;
+template <int BLOCK>
+struct ColsortLds {
+  int64_t ks[BLOCK / kColLanes][kColStage];  // (key, bond) pairs as they come
+  int32_t kr[BLOCK / kColLanes][kColStage];  // the keys in order
+  uint32_t occ[BLOCK / kColLanes][kOccWords];
+};
+
+// LDS written by lanes of a wavefront is read by its other lanes
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// WPB wavefronts per block, each on its own column (its own LDS stage); the
-// blocks step over groups of WPB columns, so every wave of a block runs the
-// same number of rounds and meets the same barriers (a wave past the last
-// column idles through its round).
-template <int WPB>
+template <int BLOCK>
 __device__ __forceinline__ void colsort_body(const Dev &d, const Geo &g, int64_t bid,
-                                             int64_t nblk) {
-  __shared__ int64_t ks_w[WPB][kColStage], kr_w[WPB][kColStage];
-  __shared__ uint32_t occ_w[WPB][64];  // occ_words <= 41 (n1d^3 < 2^31)
-  const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  int64_t *ks = ks_w[wv], *kr = kr_w[wv];
-  uint32_t *occ = occ_w[wv];
+                                             int64_t nblk, ColsortLds<BLOCK> &L) {
+  constexpr int kCols = BLOCK / kColLanes;
+  const int col = threadIdx.x / kColLanes, lane = threadIdx.x % kColLanes;
+  const int shift = (threadIdx.x & 63) - lane;  // the group's lanes in a ballot
+  int64_t *ks = L.ks[col];
+  int32_t *kr = L.kr[col];
+  uint32_t *occ = L.occ[col];
   const int n = g.n1d, W = g.occ_words;
   const int64_t ncol = (int64_t)n * n;
-  const int64_t ngrp = (ncol + WPB - 1) / WPB;
+  const int64_t ngrp = (ncol + kCols - 1) / kCols;
   for (int64_t grp = bid; grp < ngrp; grp += nblk) {
-    const int64_t c = grp * WPB + wv;
+    const int64_t c = grp * kCols + col;
     const bool live = c < ncol;
     const int32_t s = live ? d.col_start[c] : 0, e = live ? d.col_start[c + 1] : 0, m = e - s;
     const bool staged = m <= kColStage;
-    if (lane < W) occ[lane] = 0u;
+    for (int w = lane; w < W; w += kColLanes) occ[w] = 0u;
     if (live && lane == 0) d.col_count[c] = 0;  // for the next build's count
+    // (padded to whole groups of four, which the count below reads together)
     if (staged)
-      for (int i = lane; i < m; i += 64) ks[i] = kb_pair(d, d.col_tmp[s + i]);
-    __syncthreads();
-    for (int i = lane; i < m; i += 64) {
-      const int64_t ki = staged ? ks[i] : kb_pair(d, d.col_tmp[s + i]);
+      for (int i = lane; i < ((m + 3) & ~3); i += kColLanes)
+        ks[i] = i < m ? d.col_tmp[s + i] : INT64_MAX;
+    wave_sync();
+    for (int i = lane; i < m; i += kColLanes) {
+      const int64_t ki = staged ? ks[i] : d.col_tmp[s + i];
       int32_t r = 0;
       if (staged) {
-        for (int j = 0; j < m; ++j) r += ks[j] < ki;
-        kr[r] = ki;
+        for (int j = 0; j < m; j += 4) {
+          const int64_t a = ks[j], b = ks[j + 1], x = ks[j + 2], y = ks[j + 3];
+          r += (a < ki) + (b < ki) + (x < ki) + (y < ki);
+        }
+        kr[r] = (int32_t)(ki >> 32);
       } else {
-        for (int j = 0; j < m; ++j) r += kb_pair(d, d.col_tmp[s + j]) < ki;
+        for (int j = 0; j < m; ++j) r += d.col_tmp[s + j] < ki;
       }
       d.sorted[s + r] = (int32_t)(uint32_t)ki;
       d.skey[s + r] = (int32_t)(ki >> 32);
     }
     // runs: staged columns read the sorted keys from LDS, long ones from
-    // global memory after a device-scope fence; each run start's rank among
-    // the column's run starts comes from a ballot per 64 entries
+    // global memory after a fence; each run start's rank among the column's
+    // run starts comes from a ballot per kColLanes entries
     if (!staged) __threadfence();
-    __syncthreads();
+    wave_sync();
     int32_t ncell = 0;
-    for (int base = 0; base < m; base += 64) {
-      const int i = base + lane;
+    // (the four columns of a wavefront take the longest one's rounds)
+    int rounds = (m + kColLanes - 1) / kColLanes;
+    for (int o = kColLanes; o < 64; o <<= 1) {
+      const int y = __shfl_xor(rounds, o, 64);
+      rounds = y > rounds ? y : rounds;
+    }
+    for (int q = 0; q < rounds; ++q) {
+      const int i = q * kColLanes + lane;
       int32_t k = -1;
       bool start = false;
       if (i < m) {
-        k = staged ? (int32_t)(kr[i] >> 32) : d.skey[s + i];
+        k = staged ? kr[i] : d.skey[s + i];
         const int32_t kp =
-            i == 0 ? -1 : (staged ? (int32_t)(kr[i - 1] >> 32) : d.skey[s + i - 1]);
+            i == 0 ? -1 : (staged ? kr[i - 1] : d.skey[s + i - 1]);
         start = k != kp;
       }
-      const unsigned long long bal = __ballot(start);
+      constexpr uint32_t kMask = (uint32_t)((1ull << kColLanes) - 1);
+      const uint32_t bal = (uint32_t)(__ballot(start) >> shift) & kMask;
       if (start) {
-        const int32_t rank = ncell + __popcll(bal & ((1ull << lane) - 1ull));
+        const int32_t rank = ncell + __popc(bal & ((1u << lane) - 1u));
         d.cell_first[s + rank] = s + i;
         int32_t j = i + 1;
-        while (j < m && (staged ? (int32_t)(kr[j] >> 32) : d.skey[s + j]) == k) ++j;
+        while (j < m && (staged ? kr[j] : d.skey[s + j]) == k) ++j;
         d.cell_run[k] = make_int2(s + i, s + j);
         const int z = k - (int32_t)c * n;
         atomicOr(&occ[z >> 5], 1u << (z & 31));
       }
-      ncell += __popcll(bal);
+      ncell += __popc(bal);
     }
-    __syncthreads();
-    if (live && lane < W) {
-      int pre = 0;
-      for (int w = 0; w < lane; ++w) pre += __popc(occ[w]);
-      d.cell_occ[c * W + lane] = occ[lane];
-      d.occ_pre[c * W + lane] = (uint16_t)pre;
-    }
+    wave_sync();
+    if (live)
+      for (int w = lane; w < W; w += kColLanes) {
+        int pre = 0;
+        for (int v = 0; v < w; ++v) pre += __popc(occ[v]);
+        d.cell_occ[c * W + w] = occ[w];
+        d.occ_pre[c * W + w] = (uint16_t)pre;
+      }
     if (live && lane == 0) d.col_ncell[c] = ncell;
-    __syncthreads();
+    wave_sync();
   }
 }
 
@@ -632,18 +676,18 @@ __device__ __forceinline__ int2 cell_run_key(const Dev &d, const Geo &g, int32_t
 }
 
 
-// four columns per 256-thread block: as many waves in flight as one
-// column per 64-thread block, a quarter of the workgroups (the launch on
-// the odd steps that do not rebuild costs less)
-constexpr int kColWaves = 4;
+constexpr int kColBlock = 256;
+constexpr int64_t kColBlocks = 1024;  // (blocks loop over the columns)
 
-__global__ __launch_bounds__(64 * kColWaves) void k_colsort(Dev d, Geo g, int guard) {
+__global__ __launch_bounds__(kColBlock) void k_colsort(Dev d, Geo g, int guard) {
   if (guard_off(d.ctl, guard)) return;
-  colsort_body<kColWaves>(d, g, blockIdx.x, gridDim.x);
+  __shared__ ColsortLds<kColBlock> L;
+  colsort_body<kColBlock>(d, g, blockIdx.x, gridDim.x, L);
 }
 
 static inline unsigned colsort_grid(int64_t ncol) {
-  return (unsigned)std::min<int64_t>((ncol + kColWaves - 1) / kColWaves, 8192 / kColWaves);
+  constexpr int kCols = kColBlock / kColLanes;
+  return (unsigned)std::min<int64_t>((ncol + kCols - 1) / kCols, kColBlocks);
 }
 
 // Coordinates of the q-th cell of the half-shell stencil of (x, y, z) in
@@ -816,9 +860,12 @@ __device__ __forceinline__ int64_t n_supers(int64_t nb) {
   return (nb + kPullGroup * kSuper - 1) / (kPullGroup * kSuper);
 }
 
-__device__ __forceinline__ void degsum_body(const Dev &d, const Geo &g, int64_t sup) {
-  __shared__ int ws[4];
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+// (each 256 threads of a block take a block of groups)
+template <int BLOCK>
+__device__ __forceinline__ void degsum_body(const Dev &d, const Geo &g, int64_t bid) {
+  __shared__ int ws[BLOCK / 64];
+  const int lane = threadIdx.x & 63, wv = (threadIdx.x >> 6) & 3;
+  const int64_t sup = bid * (BLOCK / 256) + threadIdx.x / 256;
   int32_t *gsum = d.scan_tmp + n_supers(g.nb);
   const int64_t ngrp = n_groups(g.nb);
   int all = 0;
@@ -835,14 +882,18 @@ __device__ __forceinline__ void degsum_body(const Dev &d, const Geo &g, int64_t 
     if (lane == 0 && grp < ngrp) gsum[grp] = s;
     all += s;
   }
-  if (lane == 0) ws[wv] = all;
+  if (lane == 0) ws[threadIdx.x >> 6] = all;
   __syncthreads();
-  if (threadIdx.x == 0) d.scan_tmp[sup] = ws[0] + ws[1] + ws[2] + ws[3];
+  if (threadIdx.x % 256 == 0 && sup < n_supers(g.nb)) {
+    const int w = threadIdx.x >> 6;
+    d.scan_tmp[sup] = ws[w] + ws[w + 1] + ws[w + 2] + ws[w + 3];
+  }
+  __syncthreads();
 }
 
 __global__ __launch_bounds__(256) void k_degsum(Dev d, Geo g) {
   if (guard_off(d.ctl, kGuardRebuild)) return;
-  degsum_body(d, g, blockIdx.x);
+  degsum_body<256>(d, g, blockIdx.x);
 }
 
 static inline unsigned degsum_blocks(int64_t nb) {
@@ -868,9 +919,19 @@ static inline unsigned degsum_blocks(int64_t nb) {
 // checks the capacity, commits the list length and restarts the
 // displacement bookkeeping (InteractionManager::ZeroDrTot -> Mesh/Object::
 // ZeroDrTot, src/interaction_manager.cpp:316-321, src/mesh.cpp:546-551).
+// Where a failed list pass reports to: Ctl's own words, or, while blocks of
+// the same launch may still read those, words that reach Ctl at its end.
+struct Failure {
+  int32_t *abort, *err, *overflow;
+};
+
+__device__ __forceinline__ Failure ctl_failure(const Dev &d) {
+  return {&d.ctl->abort, &d.ctl->err, &d.ctl->overflow};
+}
+
 __device__ __forceinline__ void pull_one(const Dev &d, const Geo &g, int32_t b,
                                          int32_t w, int32_t wend, int2 *stage,
-                                         int32_t base) {
+                                         int32_t base, const Failure &fail) {
   const int32_t k = d.keys[b];
   const Excl x = excl_of(d, g, b);
   const int32_t tag = (b & 63) << 2;
@@ -932,31 +993,44 @@ __device__ __forceinline__ void pull_one(const Dev &d, const Geo &g, int32_t b,
     }
   }
   if (w != wend) {  // degree and list disagree: never expected; fail the step
-    d.ctl->abort = 1;
-    d.ctl->err = SC_ERR_STATE;
+    *fail.abort = 1;
+    *fail.err = SC_ERR_STATE;
   }
 }
 
 constexpr int kPullStage = 512;
 
-// Each block takes every nblk-th group of kPullGroup bonds; the list range of
-// a group starts at the sum of the groups before it.  The total is 64-bit, so
-// a count that does not fit the lists is seen before anything is written.
-__device__ __forceinline__ void pull_body(const Dev &d, const Geo &g, int64_t bid, int64_t nblk) {
-  static_assert(kPullGroup == 256, "one bond per thread of a block");
-  __shared__ int64_t red[4];
-  __shared__ int ws[4];
-  __shared__ int2 stage[4][kPullStage];
-  const int t = threadIdx.x, wv = t >> 6, lane = t & 63;
-  const int64_t i0 = bid * 256 + t;
-  const int64_t stride = nblk * 256;
+// Each 256 threads of a block take every so-many-th group of kPullGroup
+// bonds; the list range of a group starts at the sum of the groups before it.
+// The total is 64-bit, so a count that does not fit the lists is seen before
+// anything is written.
+template <int BLOCK>
+struct PullLds {
+  int64_t red[BLOCK / 64];
+  int2 stage[BLOCK / 64][kPullStage];
+  int ws[BLOCK / 64];
+};
+
+template <int BLOCK>
+__device__ __forceinline__ void pull_body(const Dev &d, const Geo &g, int64_t bid, int64_t nblk,
+                                          const Failure &fail, PullLds<BLOCK> &L) {
+  static_assert(kPullGroup == 256, "one bond per thread");
+  constexpr int kSubs = BLOCK / 256;
+  int64_t *red = L.red;
+  int *ws = L.ws;
+  const int t = threadIdx.x % 256, sub = threadIdx.x / 256, wv = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63;
+  const int64_t i0 = bid * BLOCK + threadIdx.x;
+  const int64_t stride = nblk * BLOCK;
   const int64_t ngrp = n_groups(g.nb), nsup = n_supers(g.nb);
   int64_t part = 0;
-  for (int64_t i = t; i < nsup; i += 256) part += d.scan_tmp[i];
+  for (int64_t i = threadIdx.x; i < nsup; i += BLOCK) part += d.scan_tmp[i];
   for (int o = 32; o > 0; o >>= 1) part += __shfl_xor(part, o, 64);
   if (lane == 0) red[wv] = part;
   __syncthreads();
-  const int64_t total = red[0] + red[1] + red[2] + red[3];  // two per candidate
+  int64_t total = 0;  // two per candidate
+#pragma unroll
+  for (int i = 0; i < BLOCK / 64; ++i) total += red[i];
   const bool fits = total <= 2 * g.cap;
   if (i0 == 0) {
     d.ctl->nc_need = total / 2;
@@ -965,8 +1039,8 @@ __device__ __forceinline__ void pull_body(const Dev &d, const Geo &g, int64_t bi
       d.ctl->n_rebuilds += 1;
       d.inc_start[g.nb] = (int32_t)total;
     } else {
-      d.ctl->abort = 1;
-      d.ctl->overflow = 1;
+      *fail.abort = 1;
+      *fail.overflow = 1;
     }
   }
   if (!fits) return;
@@ -976,10 +1050,12 @@ __device__ __forceinline__ void pull_body(const Dev &d, const Geo &g, int64_t bi
   }
   // the incidence starts of the block's groups, before the walk over them (in
   // one loop with it they cost the walk 22 registers, two waves per SIMD)
-  for (int grp = (int)bid; grp < (int)ngrp; grp += (int)nblk) {
+  for (int grp0 = (int)bid * kSubs; grp0 < (int)ngrp; grp0 += (int)nblk * kSubs) {
+    const int grp = grp0 + sub;
     const int64_t b = (int64_t)grp * kPullGroup + t;
     const int sup = grp / kSuper;
-    int32_t before = sup * kSuper + t < grp ? d.scan_tmp[nsup + sup * kSuper + t] : 0;
+    int32_t before =
+        sup * kSuper + t < grp && grp < (int)ngrp ? d.scan_tmp[nsup + sup * kSuper + t] : 0;
     for (int i = t; i < sup; i += 256) before += d.scan_tmp[i];
     const int32_t base = block_sum<256>(before, ws);
     int gtot;
@@ -989,8 +1065,8 @@ __device__ __forceinline__ void pull_body(const Dev &d, const Geo &g, int64_t bi
   // each wavefront's 64 consecutive bonds have one contiguous list range:
   // written to LDS entry by entry, then copied out in coalesced stores
   // (ranges longer than the stage are written directly)
-  for (int64_t grp = bid; grp < ngrp; grp += nblk) {
-    const int64_t b = grp * kPullGroup + t;
+  for (int64_t grp0 = bid * kSubs; grp0 < ngrp; grp0 += nblk * kSubs) {
+    const int64_t b = (grp0 + sub) * kPullGroup + t;
     int32_t w = (int32_t)total, wend = w;
     if (b < g.nb) {
       w = d.inc_start[b];
@@ -998,17 +1074,176 @@ __device__ __forceinline__ void pull_body(const Dev &d, const Geo &g, int64_t bi
     }
     const int32_t base = __shfl(w, 0, 64), cnt = __shfl(wend, 63, 64) - base;
     const bool staged = cnt <= kPullStage;
-    if (b < g.nb) pull_one(d, g, (int32_t)b, w, wend, staged ? stage[wv] : nullptr, base);
+    if (b < g.nb) pull_one(d, g, (int32_t)b, w, wend, staged ? L.stage[wv] : nullptr, base, fail);
     __syncthreads();
     if (staged)
-      for (int i = lane; i < cnt; i += 64) d.inc[base + i] = stage[wv][i];
+      for (int i = lane; i < cnt; i += 64) d.inc[base + i] = L.stage[wv][i];
     __syncthreads();
   }
 }
 
 __global__ __launch_bounds__(256) void k_pull(Dev d, Geo g) {
   if (guard_off(d.ctl, kGuardRebuild)) return;
-  pull_body(d, g, blockIdx.x, gridDim.x);
+  __shared__ PullLds<256> L;
+  pull_body<256>(d, g, blockIdx.x, gridDim.x, ctl_failure(d), L);
+}
+
+// ---- the rebuild stage in one launch ----------------------------------------
+// Every launch costs 1.55 us also on a step that does not rebuild, so up to
+// kOneLaunchBonds one launch runs the seven passes, with a barrier between
+// them among its blocks.  A barrier never waits for a block that is not
+// running: the blocks that take part are those that have arrived when the
+// first of them closes the door -- when all have, or after kDoorTicks --
+// and a block that arrives later leaves at once.  The passes take their block
+// index and count from that, so any number of blocks (one, if need be) does
+// all the work.  Measured (device-scope release and acquire included): a
+// barrier 3.5 us among 64 blocks, 7 among 256, 12 among 512, against 1.55 us
+// for a kernel boundary; hence few, large blocks, and the launches for larger
+// systems, whose passes want more of them.  us a step, seven launches against
+// one: 1k bonds 25.7 / 22.4, FP64 1.2k 31.4 / 27.3, 52k 31.9 / 29.6, 62k with
+// stress sums 34.2 / 31.6, 101k 36.4 / 32.9; FP64 155k 55.3 / 56.0, so the
+// line is drawn at 128k.
+constexpr int kOneBlock = 1024;
+constexpr int64_t kOneLaunchBonds = 131072;
+
+static inline bool rebuild_in_one(const Geo &g) {
+  return g.nb <= kOneLaunchBonds && (int64_t)g.n1d * g.n1d <= kColScanMax;
+}
+
+// Blocks of the one launch: enough for 800 bonds each (64 or 128 blocks where
+// they were the best of 16 to 256 at 52k and 101k bonds), and in small sparse
+// systems for 64 columns each, whose sort is the longest pass there.
+static inline unsigned one_blocks(const Geo &g) {
+  const int64_t ncol = (int64_t)g.n1d * g.n1d;
+  const int64_t b = std::max<int64_t>((g.nb + 799) / 800, std::min<int64_t>((ncol + 63) / 64, 64));
+  return (unsigned)std::min<int64_t>(std::max<int64_t>(b, 1), 128);
+}
+
+constexpr uint32_t kDoorClosed = 0x80000000u;
+constexpr long long kDoorTicks = 2000;  // of the 100 MHz clock: 20 us
+
+__device__ __forceinline__ uint32_t bar_load(const uint32_t *p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ uint32_t bar_add(uint32_t *p) {
+  return __hip_atomic_fetch_add(p, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// All threads: enters the block; false when it came too late.  *rank and
+// *parts: its number among the blocks taking part, and how many those are.
+// `blocks`: those of the launch that belong to the system.
+__device__ __forceinline__ bool door_enter(RebuildBar *b, uint32_t blocks, int *rank,
+                                           int *parts) {
+  __shared__ uint32_t sr, sp;
+  if (threadIdx.x == 0) {
+    const uint32_t r = bar_add(&b->arrived);
+    uint32_t p = 0;
+    if (r == 0) {  // the first to arrive closes the door
+      const long long t0 = wall_clock64();
+      while (bar_load(&b->arrived) < blocks && wall_clock64() - t0 < kDoorTicks)
+        __builtin_amdgcn_s_sleep(1);
+      p = __hip_atomic_fetch_or(&b->arrived, kDoorClosed, __ATOMIC_RELAXED,
+                                __HIP_MEMORY_SCOPE_AGENT);
+      __hip_atomic_store(&b->parts, p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    } else if (!(r & kDoorClosed)) {
+      while ((p = bar_load(&b->parts)) == 0) __builtin_amdgcn_s_sleep(1);
+    }
+    sr = r;
+    sp = p;
+  }
+  __syncthreads();
+  *rank = (int)(sr & ~kDoorClosed);
+  *parts = (int)sp;
+  return !(sr & kDoorClosed);
+}
+
+// Barrier `k` of a launch among the `parts` blocks inside (all threads).  The
+// arrivals are counted in kBarGroups groups and the full groups in one word,
+// as atomics on one address serialise.
+__device__ __forceinline__ void bar_wait(RebuildBar *b, int k, int rank, int parts) {
+  __syncthreads();
+  if (parts > 1 && threadIdx.x == 0) {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+    const int grp = rank % kBarGroups;
+    const uint32_t size = (uint32_t)((parts - grp + kBarGroups - 1) / kBarGroups);
+    const uint32_t groups = (uint32_t)(parts < kBarGroups ? parts : kBarGroups);
+    if (bar_add(&b->group[k][grp][0]) + 1 == size) bar_add(&b->full[k][0]);
+    while (bar_load(&b->full[k][0]) < groups) __builtin_amdgcn_s_sleep(1);
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+  }
+  __syncthreads();
+}
+
+// Every block of the launch, last thing.  A block that comes late must still
+// find the rebuild decided as the others did, or it would leave uncounted; so
+// what the decision is taken from -- the displacement slots, Ctl's abort word
+// -- changes only here, by the block that leaves last, which also clears the
+// counters for the next launch (nobody looks at them any more).
+__device__ __forceinline__ void door_leave(const Dev &d, uint32_t blocks) {
+  __shared__ int last;
+  RebuildBar *b = d.bar;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+    last = bar_add(&b->gone) + 1 == blocks;
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+  }
+  __syncthreads();
+  if (!last) return;
+  clear_dr_slots(d);
+  uint32_t *count = &b->full[0][0];
+  constexpr int kCounts = (int)((sizeof(b->full) + sizeof(b->group)) / sizeof(uint32_t));
+  for (int i = threadIdx.x; i < kCounts; i += blockDim.x) count[i] = 0;
+  if (threadIdx.x != 0) return;
+  Ctl *c = d.ctl;
+  if (b->overflow) c->overflow = 1;
+  if (b->err) c->err = b->err;
+  if (b->abort) c->abort = 1;
+  b->overflow = b->err = b->abort = 0;
+  b->arrived = b->parts = b->gone = 0;
+}
+
+// the passes' stages, one after the other in the same memory
+union OneLds {
+  KeysLds<kOneBlock> keys;
+  ColsortLds<kOneBlock> col;
+  PullLds<kOneBlock> pull;
+};
+
+template <bool FOLD>
+__device__ __forceinline__ void rebuild_one_body(const Dev &d, const Geo &g, uint32_t blocks,
+                                                 bool first, OneLds &L) {
+  if (FOLD) {
+    if (!fold_commit(d, g.thr, first)) return;
+  } else {
+    if (guard_off(d.ctl, kGuardRebuild)) return;
+  }
+  RebuildBar *bar = d.bar;
+  int rank, parts;
+  if (door_enter(bar, blocks, &rank, &parts)) {
+    const int64_t ncol = (int64_t)g.n1d * g.n1d;
+    keys_body<kOneBlock>(d, g, rank, parts, L.keys);
+    bar_wait(bar, 0, rank, parts);
+    for (int64_t t = rank; t * kColScanTile < ncol; t += parts) colscan_body(d, ncol, t);
+    bar_wait(bar, 1, rank, parts);
+    scatter_body(d, g, rank, parts);
+    bar_wait(bar, 2, rank, parts);
+    colsort_body<kOneBlock>(d, g, rank, parts, L.col);
+    bar_wait(bar, 3, rank, parts);
+    deg_body(d, g, rank, parts);
+    bar_wait(bar, 4, rank, parts);
+    for (int64_t s = rank; s * (kOneBlock / 256) < n_supers(g.nb); s += parts)
+      degsum_body<kOneBlock>(d, g, s);
+    bar_wait(bar, 5, rank, parts);
+    pull_body<kOneBlock>(d, g, rank, parts, {&bar->abort, &bar->err, &bar->overflow}, L.pull);
+  }
+  door_leave(d, blocks);
+}
+
+template <bool FOLD>
+__global__ __launch_bounds__(kOneBlock) void k_rebuild_one(Dev d, Geo g) {
+  __shared__ OneLds L;
+  rebuild_one_body<FOLD>(d, g, gridDim.x, blockIdx.x == 0, L);
 }
 
 static inline unsigned nblocks(int64_t n, int bs) {
@@ -1021,6 +1256,7 @@ static inline unsigned sgrid(int64_t n) {
   return b < (unsigned)kStreamBlocks ? b : (unsigned)kStreamBlocks;
 }
 
+// Up to kOneLaunchBonds one launch (k_rebuild_one); above:
 // keys (+ column populations) -> column scan -> column scatter -> column
 // sort (+ runs, occupancy) -> degrees -> degree sums -> incidence lists
 // (+ incidence starts, capacity check, displacement restart): 7 launches,
@@ -1033,13 +1269,21 @@ constexpr unsigned kListBlocks = 2048;
 void launch_rebuild(const Dev &d, const Geo &g, bool fold, hipStream_t st) {
   const unsigned gs = sgrid(g.nb);
   const int64_t ncol = (int64_t)g.n1d * g.n1d;
+  if (rebuild_in_one(g)) {
+    const dim3 grid(one_blocks(g));
+    if (fold)
+      hipLaunchKernelGGL(k_rebuild_one<true>, grid, dim3(kOneBlock), 0, st, d, g);
+    else
+      hipLaunchKernelGGL(k_rebuild_one<false>, grid, dim3(kOneBlock), 0, st, d, g);
+    return;
+  }
   if (fold)
     hipLaunchKernelGGL(k_keys<true>, dim3(gs), dim3(kScanBlock), 0, st, d, g);
   else
     hipLaunchKernelGGL(k_keys<false>, dim3(gs), dim3(kScanBlock), 0, st, d, g);
   launch_colscan(d, ncol, kGuardRebuild, st);
   hipLaunchKernelGGL(k_scatter, dim3(gs), dim3(kScanBlock), 0, st, d, g, (int)kGuardRebuild);
-  hipLaunchKernelGGL(k_colsort, dim3(colsort_grid(ncol)), dim3(64 * kColWaves), 0, st, d, g,
+  hipLaunchKernelGGL(k_colsort, dim3(colsort_grid(ncol)), dim3(kColBlock), 0, st, d, g,
                      (int)kGuardRebuild);
   const unsigned gl = std::min(nblocks(g.nb, 256), kListBlocks);
   hipLaunchKernelGGL(k_deg, dim3(gl), dim3(256), 0, st, d, g);
@@ -1062,23 +1306,25 @@ __global__ __launch_bounds__(kScanBlock) void k_group_keys(const Member *__restr
   } else {
     if (guard_off(M.d[0].ctl, kGuardRebuild)) return;
   }
-  keys_body(M.d[0], M.g, blockIdx.x - b0, nblk);
+  __shared__ KeysLds<kScanBlock> L;
+  keys_body<kScanBlock>(M.d[0], M.g, blockIdx.x - b0, nblk, L);
 }
 
 __global__ void k_group_scatter(const Member *__restrict__ ms, GroupGrid gg) {
   int b0, nblk;
   const Member &M = ms[group_member(gg, blockIdx.x, &b0, &nblk)];
-  if ((int)blockIdx.x == b0) clear_dr_slots(M.d[0]);
   if (guard_off(M.d[0].ctl, kGuardRebuild)) return;
+  if ((int)blockIdx.x == b0) clear_dr_slots(M.d[0]);
   scatter_body(M.d[0], M.g, blockIdx.x - b0, nblk);
 }
 
-__global__ __launch_bounds__(64) void k_group_colsort(const Member *__restrict__ ms,
-                                                      GroupGrid gg) {
+__global__ __launch_bounds__(kColBlock) void k_group_colsort(const Member *__restrict__ ms,
+                                                             GroupGrid gg) {
   int b0, nblk;
   const Member &M = ms[group_member(gg, blockIdx.x, &b0, &nblk)];
   if (guard_off(M.d[0].ctl, kGuardRebuild)) return;
-  colsort_body<1>(M.d[0], M.g, blockIdx.x - b0, nblk);
+  __shared__ ColsortLds<kColBlock> L;
+  colsort_body<kColBlock>(M.d[0], M.g, blockIdx.x - b0, nblk, L);
 }
 
 __global__ __launch_bounds__(256) void k_group_deg(const Member *__restrict__ ms, GroupGrid gg) {
@@ -1092,7 +1338,8 @@ __global__ __launch_bounds__(256) void k_group_pull(const Member *__restrict__ m
   int b0, nblk;
   const Member &M = ms[group_member(gg, blockIdx.x, &b0, &nblk)];
   if (guard_off(M.d[0].ctl, kGuardRebuild)) return;
-  pull_body(M.d[0], M.g, blockIdx.x - b0, nblk);
+  __shared__ PullLds<256> L;
+  pull_body<256>(M.d[0], M.g, blockIdx.x - b0, nblk, ctl_failure(M.d[0]), L);
 }
 
 // the two-launch column scan, for batches with a member of more than
@@ -1129,7 +1376,16 @@ __global__ __launch_bounds__(256) void k_group_degsum(const Member *__restrict__
   int b0, nblk;
   const Member &M = ms[group_member(gg, blockIdx.x, &b0, &nblk)];
   if (guard_off(M.d[0].ctl, kGuardRebuild)) return;
-  degsum_body(M.d[0], M.g, blockIdx.x - b0);
+  degsum_body<256>(M.d[0], M.g, blockIdx.x - b0);
+}
+
+template <bool FOLD>
+__global__ __launch_bounds__(kOneBlock) void k_group_rebuild_one(const Member *__restrict__ ms,
+                                                                 GroupGrid gg) {
+  __shared__ OneLds L;
+  int b0, nblk;
+  const Member &M = ms[group_member(gg, blockIdx.x, &b0, &nblk)];
+  rebuild_one_body<FOLD>(M.d[0], M.g, nblk, (int)blockIdx.x == b0, L);
 }
 
 namespace {
@@ -1153,6 +1409,17 @@ unsigned scan_blocks(int64_t n) {
 
 void launch_group_rebuild(const Member *dm, const Member *hm, int n, bool fold, hipStream_t st) {
   if (n <= 0) return;
+  bool one = true;
+  for (int m = 0; m < n; ++m) one = one && rebuild_in_one(hm[m].g);
+  if (one) {
+    GroupGrid go;
+    const int32_t to = group_grid(go, hm, n, [](const Geo &g) { return one_blocks(g); });
+    if (fold)
+      hipLaunchKernelGGL(k_group_rebuild_one<true>, dim3(to), dim3(kOneBlock), 0, st, dm, go);
+    else
+      hipLaunchKernelGGL(k_group_rebuild_one<false>, dim3(to), dim3(kOneBlock), 0, st, dm, go);
+    return;
+  }
   GroupGrid gk, gcs, gsrt, gdeg, gds, gpl;
   const int32_t tk = group_grid(gk, hm, n, [](const Geo &g) { return sgrid(g.nb); });
   bool wide = false;
@@ -1162,7 +1429,7 @@ void launch_group_rebuild(const Member *dm, const Member *hm, int n, bool fold, 
     return wide ? scan_blocks(ncol) : colscan_tiles(ncol);
   });
   const int32_t tsrt = group_grid(gsrt, hm, n, [](const Geo &g) {
-    return (unsigned)std::min<int64_t>((int64_t)g.n1d * g.n1d, 8192);
+    return colsort_grid((int64_t)g.n1d * g.n1d);
   });
   const int32_t tdeg = group_grid(gdeg, hm, n, [](const Geo &g) {
     return std::min(nblocks(g.nb, 256), kListBlocks);
@@ -1182,7 +1449,7 @@ void launch_group_rebuild(const Member *dm, const Member *hm, int n, bool fold, 
     hipLaunchKernelGGL(k_group_colscan, dim3(tcs), dim3(kColScanBlock), 0, st, dm, gcs);
   }
   hipLaunchKernelGGL(k_group_scatter, dim3(tk), dim3(kScanBlock), 0, st, dm, gk);
-  hipLaunchKernelGGL(k_group_colsort, dim3(tsrt), dim3(64), 0, st, dm, gsrt);
+  hipLaunchKernelGGL(k_group_colsort, dim3(tsrt), dim3(kColBlock), 0, st, dm, gsrt);
   hipLaunchKernelGGL(k_group_deg, dim3(tdeg), dim3(256), 0, st, dm, gdeg);
   hipLaunchKernelGGL(k_group_degsum, dim3(tds), dim3(256), 0, st, dm, gds);
   hipLaunchKernelGGL(k_group_pull, dim3(tpl), dim3(256), 0, st, dm, gpl);
@@ -1204,7 +1471,7 @@ void launch_cells_from_keys(const Dev &d, const Geo &g, hipStream_t st) {
   hipLaunchKernelGGL(k_key_count, dim3(sgrid(g.nb)), dim3(256), 0, st, d, g);
   launch_colscan(d, ncol, 0, st);
   hipLaunchKernelGGL(k_scatter, dim3(sgrid(g.nb)), dim3(256), 0, st, d, g, 0);
-  hipLaunchKernelGGL(k_colsort, dim3(colsort_grid(ncol)), dim3(64 * kColWaves), 0, st, d, g, 0);
+  hipLaunchKernelGGL(k_colsort, dim3(colsort_grid(ncol)), dim3(kColBlock), 0, st, d, g, 0);
 }
 
 // Replays the displacement bookkeeping of the last full step after the host

@@ -62,6 +62,61 @@ def test_lists_at_launch_edges(n1d, nb, precision):
     s.close()
 
 
+def _cell_pairs(keys, n, site_off):
+    """Sorted pair codes (a * nb + b, a < b) of the bonds in adjacent cells,
+    neighbours along a filament left out, cell by cell."""
+    nb = len(keys)
+    order = np.argsort(keys, kind="stable")
+    ks = keys[order]
+    c = np.stack([ks // (n * n), ks // n % n, ks % n])
+    fil = np.repeat(np.arange(len(site_off) - 1), np.diff(site_off) - 1)
+    out = []
+    for dx in (-1, 0, 1):
+        for dy in (-1, 0, 1):
+            for dz in (-1, 0, 1):
+                m = [(c[0] + dx) % n, (c[1] + dy) % n, (c[2] + dz) % n]
+                kk = (m[0] * n + m[1]) * n + m[2]
+                lo, hi = np.searchsorted(ks, kk), np.searchsorted(ks, kk, side="right")
+                cnt = hi - lo
+                i = np.repeat(np.arange(nb), cnt)
+                j = np.arange(len(i)) - np.repeat(np.cumsum(cnt) - cnt, cnt) + np.repeat(lo, cnt)
+                a, b = order[i], order[j]
+                keep = (a < b) & ~((b - a == 1) & (fil[a] == fil[b]))
+                out.append(a[keep].astype(np.int64) * nb + b[keep])
+    return np.sort(np.concatenate(out))
+
+
+# 800 bonds a block of the one-launch rebuild, which serves 131072 bonds
+@pytest.mark.parametrize("nb", [799, 800, 801, 25599, 102401, 131071, 131072, 131073])
+def test_lists_of_one_and_several_launches(nb):
+    rng = np.random.default_rng(nb)
+    n1d = max(12, int(round((nb / 1.5) ** (1.0 / 3.0))))
+    p = sc.params_init(float(n1d), delta=1e-4, min_cell_length=2.0, seed=11)
+    lengths, left = [], nb
+    while left > 0:
+        k = min(left, int(rng.integers(2, 60)))
+        if left - k == 1:
+            k += 1
+        lengths.append(k + 1)
+        left -= k
+    u = rng.normal(size=(len(lengths), 3))
+    u /= np.linalg.norm(u, axis=1)[:, None]
+    start = rng.uniform(-n1d, n1d, (len(lengths), 3))
+    fil = make_filaments([start[f] + np.arange(n)[:, None] * u[f]
+                          for f, n in enumerate(lengths)])
+    assert fil.nb == nb
+    s = sc.FilamentSystem(p, fil, precision="mixed", use_graph=True, spatial_order=True)
+    assert s.counters()["n_cells_1d"] == n1d
+    for steps in (0, 41):  # the list of the load, then of rebuilds inside a run
+        s.step(steps)
+        a, b = s.candidates()
+        code = np.sort(np.minimum(a, b).astype(np.int64) * nb + np.maximum(a, b))
+        want = _cell_pairs(s.cell_keys().astype(np.int64), n1d, np.asarray(fil.site_off))
+        np.testing.assert_array_equal(code, want)
+    assert s.counters()["n_rebuilds"] > 1
+    s.close()
+
+
 def test_batch_with_a_wide_member():
     """A batch member with more columns than the one-launch scan takes, beside
     a small one: each as when stepped alone."""
