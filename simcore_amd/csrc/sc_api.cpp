@@ -1036,7 +1036,7 @@ size_t system_estimate_bytes(const sc_params *params, int32_t nf, int64_t ns, in
   const int64_t n_cells = n1d * n1d * n1d;
   const int64_t nb = ns - nf;
   auto R = [](int64_t n) { return Arena::round((size_t)(n > 0 ? n : 1)); };
-  size_t b = R(sizeof(Ctl)) + R(8 * sc::kDrSlots) + R(sizeof(sc::RebuildBar)) + R(4 * (nf + 1)) + 2 * R(4 * (int64_t)nf) +
+  size_t b = R(sizeof(Ctl)) + R(8 * sc::kDrSlots) + R(sizeof(sc::Door)) + R(4 * (nf + 1)) + 2 * R(4 * (int64_t)nf) +
              R(64 * (int64_t)nf) +
              R(8 * (int64_t)nf) + R(4 * nb);
   b += 4 * R(24 * ns) + 2 * R(8 * ns);                    // r, rp, fr, dr0, acc, acc_prev
@@ -1223,8 +1223,8 @@ int sc_load_filaments(sc_handle h, int32_t nf, const int32_t *site_off,
   if ((rc = dalloc(h, &d.dr_slots, sc::kDrSlots, false))) return rc;
   HIPCHK(h, hipMemsetAsync(d.dr_slots, 0, sizeof(unsigned long long) * sc::kDrSlots,
                            h->stream));
-  if ((rc = dalloc(h, &d.bar, 1, false))) return rc;
-  HIPCHK(h, hipMemsetAsync(d.bar, 0, sizeof(sc::RebuildBar), h->stream));
+  if ((rc = dalloc(h, &d.door, 1, false))) return rc;
+  HIPCHK(h, hipMemsetAsync(d.door, 0, sizeof(sc::Door), h->stream));
   if ((rc = dalloc(h, &d.site_off, nf + 1, false))) return rc;
   if ((rc = dalloc(h, &d.noise_off, nf, false))) return rc;
   if ((rc = dalloc(h, &d.fil_caller, nf, false))) return rc;

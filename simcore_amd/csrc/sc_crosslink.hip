@@ -14,6 +14,9 @@
 // (Ctl::xl_dirty), on the device, so the step stays graph-replayable.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
+#include "sc_block.h"
 #include "sc_internal.h"
 #include "sc_math.h"
 
@@ -83,7 +86,7 @@ __device__ __forceinline__ double unit_draw(uint32_t v) {
 // the scaled anchor points and each compute the same force and their own
 // torque.  A chain of loads, FP64 roots and divisions bounds it, so the lanes
 // halve it and small blocks spread it over the chip.
-// 20k crosslinks: 8.6 us with one lane each, 7.8 with two.
+// 50k crosslinks: 8.6 us with one lane each, 7.8 with two.
 constexpr int kXlBlock = 64;
 
 __global__ __launch_bounds__(kXlBlock) void k_xl_force(Dev d, Geo g) {
@@ -134,7 +137,7 @@ __global__ __launch_bounds__(kXlBlock) void k_xl_force(Dev d, Geo g) {
 // whoever finds it.  Few crosslinks come off in a step, so the launch lasts as
 // long as one search: 343-729 cells, a chain of loads, roots and divisions for
 // each bond in them: 35 us where one lane took 238
-// (20k crosslinks, 400k bonds, one coming off).
+// (50k crosslinks, 400k bonds, one coming off).
 __global__ __launch_bounds__(kXlBlock) void k_xl_events(Dev d, Geo g) {
   Ctl *ctl = d.ctl;
   if (ctl->abort) return;
@@ -232,50 +235,69 @@ __global__ __launch_bounds__(kXlBlock) void k_xl_events(Dev d, Geo g) {
   }
 }
 
-__device__ __forceinline__ bool xl_off(const Ctl *c) { return c->abort || !c->xl_dirty; }
+// Per-bond lists from the bindings, in one launch: count, chunk sums of the
+// counts, starts, fill, sort, with barriers between the passes.  On most steps
+// there is no event and the launch returns at once, so what counts is that it
+// is one and not six, 1.55 us each.  Blocks for 4096 bonds each, as many as
+// the barriers carry.  400k bonds, 50k crosslinks: 84.0 us a step with the six
+// launches, 80.0 with this one, which takes 44 us when there was an event.
+constexpr int kListBlock = 1024;
+constexpr int kXlListBlocks = 128;
 
-__global__ __launch_bounds__(256) void k_xl_count(Dev d, Geo g) {
-  if (xl_off(d.ctl)) return;
-  const int64_t x = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (x >= g.nx) return;
-  atomicAdd(&d.xdeg[d.xb[2 * x]], 1);
-  atomicAdd(&d.xdeg[d.xb[2 * x + 1]], 1);
-}
-
-// places the entries; xdeg returns to zero for the next rebuild
-__global__ __launch_bounds__(256) void k_xl_fill(Dev d, Geo g) {
-  if (xl_off(d.ctl)) return;
-  const int64_t x = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (x >= g.nx) return;
-  for (int a = 0; a < 2; ++a) {
-    const int32_t b = d.xb[2 * x + a];
-    const int32_t pos = d.xinc_start[b] + atomicSub(&d.xdeg[b], 1) - 1;
-    d.xinc[pos] = (int32_t)((x << 1) | a);
-  }
-}
-
-__global__ __launch_bounds__(256) void k_xl_sort(Dev d, Geo g) {
-  if (xl_off(d.ctl)) return;
-  const int64_t b = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (b >= g.nb) return;
-  const int32_t q0 = d.xinc_start[b], q1 = d.xinc_start[b + 1];
-  for (int32_t i = q0 + 1; i < q1; ++i) {
-    const int32_t v = d.xinc[i];
-    int32_t j = i - 1;
-    while (j >= q0 && d.xinc[j] > v) {
-      d.xinc[j + 1] = d.xinc[j];
-      --j;
+__global__ __launch_bounds__(kListBlock) void k_xl_lists(Dev d, Geo g) {
+  if (d.ctl->abort || !d.ctl->xl_dirty) return;
+  __shared__ int ws[kListBlock / 64];
+  int rank, parts;
+  if (door_enter(d.door, gridDim.x, &rank, &parts)) {
+    const int64_t t0 = (int64_t)rank * kListBlock + threadIdx.x, stride = (int64_t)parts * kListBlock;
+    // a block's bonds: a run of whole tiles
+    const int64_t tiles = (g.nb + kListBlock - 1) / kListBlock;
+    const int64_t b0 = tiles * rank / parts * kListBlock;
+    const int64_t b1 = std::min<int64_t>(tiles * (rank + 1) / parts * kListBlock, g.nb);
+    for (int64_t e = t0; e < 2 * g.nx; e += stride) atomicAdd(&d.xdeg[d.xb[e]], 1);
+    bar_wait(d.door, 0, rank, parts);
+    int s = 0;
+    for (int64_t b = b0 + threadIdx.x; b < b1; b += kListBlock) s += d.xdeg[b];
+    s = block_sum<kListBlock>(s, ws);
+    if (threadIdx.x == 0) d.scan_tmp[rank] = s;
+    bar_wait(d.door, 1, rank, parts);
+    int base = block_sum<kListBlock>((int)threadIdx.x < rank ? d.scan_tmp[threadIdx.x] : 0, ws);
+    for (int64_t c = b0; c < b1; c += kListBlock) {
+      const int64_t b = c + threadIdx.x;
+      int tot;
+      const int ex = block_excl<kListBlock>(b < b1 ? d.xdeg[b] : 0, &tot, ws);
+      if (b < b1) d.xinc_start[b] = base + ex;
+      base += tot;
     }
-    d.xinc[j + 1] = v;
+    if (rank == parts - 1 && threadIdx.x == 0) d.xinc_start[g.nb] = base;
+    bar_wait(d.door, 2, rank, parts);
+    // places the entries; xdeg returns to zero for the next rebuild
+    for (int64_t e = t0; e < 2 * g.nx; e += stride) {
+      const int32_t b = d.xb[e];
+      d.xinc[d.xinc_start[b] + atomicSub(&d.xdeg[b], 1) - 1] = (int32_t)e;
+    }
+    bar_wait(d.door, 3, rank, parts);
+    for (int64_t b = b0 + threadIdx.x; b < b1; b += kListBlock) {
+      const int32_t q0 = d.xinc_start[b], q1 = d.xinc_start[b + 1];
+      for (int32_t i = q0 + 1; i < q1; ++i) {
+        const int32_t v = d.xinc[i];
+        int32_t j = i - 1;
+        while (j >= q0 && d.xinc[j] > v) {
+          d.xinc[j + 1] = d.xinc[j];
+          --j;
+        }
+        d.xinc[j + 1] = v;
+      }
+    }
+  }
+  if (door_leave(d.door, gridDim.x)) {
+    if (threadIdx.x == 0) d.ctl->xl_dirty = 0;
+    door_reset(d.door);
   }
 }
 
-__global__ void k_xl_clean(Ctl *c) {
-  if (threadIdx.x == 0 && blockIdx.x == 0 && !c->abort) c->xl_dirty = 0;
-}
-
-inline dim3 grid_for(int64_t n, int block = 256) {
-  const int64_t b = (n + block - 1) / block;
+inline dim3 grid_for(int64_t n) {
+  const int64_t b = (n + kXlBlock - 1) / kXlBlock;
   return dim3((unsigned)(b > 0 ? b : 1));
 }
 
@@ -283,21 +305,18 @@ inline dim3 grid_for(int64_t n, int block = 256) {
 
 void launch_xlink_forces(const Dev &d, const Geo &g, hipStream_t st) {
   if (g.nx <= 0) return;
-  hipLaunchKernelGGL(k_xl_force, grid_for(2 * g.nx, kXlBlock), dim3(kXlBlock), 0, st, d, g);
+  hipLaunchKernelGGL(k_xl_force, grid_for(2 * g.nx), dim3(kXlBlock), 0, st, d, g);
 }
 
 void launch_xlink_events(const Dev &d, const Geo &g, hipStream_t st) {
   if (g.nx <= 0 || !(g.xpoff > 0)) return;
-  hipLaunchKernelGGL(k_xl_events, grid_for(g.nx, kXlBlock), dim3(kXlBlock), 0, st, d, g);
+  hipLaunchKernelGGL(k_xl_events, grid_for(g.nx), dim3(kXlBlock), 0, st, d, g);
 }
 
 void launch_xlink_lists(const Dev &d, const Geo &g, hipStream_t st) {
   if (g.nx <= 0) return;
-  hipLaunchKernelGGL(k_xl_count, grid_for(g.nx), dim3(256), 0, st, d, g);
-  launch_scan(d.xdeg, d.xinc_start, g.nb, d.scan_tmp, d.ctl, kGuardXlink, st);
-  hipLaunchKernelGGL(k_xl_fill, grid_for(g.nx), dim3(256), 0, st, d, g);
-  hipLaunchKernelGGL(k_xl_sort, grid_for(g.nb), dim3(256), 0, st, d, g);
-  hipLaunchKernelGGL(k_xl_clean, dim3(1), dim3(64), 0, st, d.ctl);
+  const int64_t blocks = std::min<int64_t>((g.nb + 4095) / 4096, kXlListBlocks);
+  hipLaunchKernelGGL(k_xl_lists, dim3((unsigned)blocks), dim3(kListBlock), 0, st, d, g);
 }
 
 }  // namespace sc

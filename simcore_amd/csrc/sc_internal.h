@@ -81,10 +81,10 @@ struct Geo {
 // slots into Ctl::dr_bits and clears them.
 constexpr int kDrSlots = 256;
 
-// Counters of the one-launch rebuild stage (sc_kernels.hip), zero between
+// Counters of the launches that run several passes (sc_block.h), zero between
 // launches; one cache line per counter that several blocks add to.
 constexpr int kBars = 6, kBarGroups = 16;
-struct RebuildBar {
+struct Door {
   uint32_t arrived, parts, gone;
   int32_t abort, err, overflow;  // for Ctl, when the launch ends
   uint32_t pad[10];
@@ -98,7 +98,7 @@ struct Dev {
                            // even step that follows its odd step without a
                            // commit between them, else 0
   unsigned long long *dr_slots;  // kDrSlots, zero between runs of steps
-  RebuildBar *bar;
+  Door *door;
   // filaments
   int32_t *site_off;       // nf+1
   int32_t *noise_off;      // nf: site index the noise stream is keyed by
@@ -285,7 +285,7 @@ constexpr int kStreamBlocks = 1024;
 constexpr int kScanTile = kScanBlock * kScanItems;
 constexpr int kPullGroup = 256;  // bonds whose lists a block of the list pass writes at a time
 
-enum Guard { kGuardStep = 0, kGuardRebuild = 1, kGuardXlink = 2 };
+enum Guard { kGuardStep = 0, kGuardRebuild = 1 };
 
 // Cell-list lookups.  Occupancy bit of cell (x, y, z); run of an occupied
 // cell (its members in bond order).

@@ -20,6 +20,7 @@
 
 #include <algorithm>
 
+#include "sc_block.h"
 #include "sc_internal.h"
 #include "sc_math.h"
 
@@ -148,7 +149,6 @@ __global__ void k_zero_i32(int32_t *p, int64_t n) {
 __device__ __forceinline__ bool guard_off(const Ctl *c, int guard) {
   if (!c) return false;
   if (c->abort) return true;
-  if (guard == kGuardXlink) return !c->xl_dirty;
   return guard == kGuardRebuild && !c->rebuild;
 }
 
@@ -260,8 +260,8 @@ __global__ __launch_bounds__(kScanBlock) void k_scan_down(const int32_t *in,
   scan_down_body(in, n, bsum, out, blockIdx.x, gridDim.x);
 }
 
-// entries of Dev::scan_tmp: tile sums of a two-launch scan over the columns
-// or the bonds, or the degree sums of the list pass
+// entries of Dev::scan_tmp: tile sums of a two-launch scan over the columns,
+// the degree sums of the list pass, or the crosslink lists' chunk sums
 int64_t scan_tmp_elems(int64_t ncol, int64_t nb) {
   const int64_t n = ncol > nb ? ncol : nb;
   const int64_t tiles = (n + kScanTile - 1) / kScanTile + 1;
@@ -293,46 +293,6 @@ void launch_scan(const int32_t *in, int32_t *out, int64_t n, int32_t *tmp,
 constexpr int kColScanBlock = 1024;
 constexpr int kColScanTile = 4 * kColScanBlock;
 constexpr int64_t kColScanMax = (int64_t)1 << 17;
-
-// Sum of v over each SUB consecutive threads of a block; `ws` holds one int
-// per wavefront of the block.
-template <int SUB>
-__device__ __forceinline__ int block_sum(int v, int *ws) {
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-  if ((threadIdx.x & 63) == 0) ws[threadIdx.x >> 6] = v;
-  __syncthreads();
-  const int w0 = (int)threadIdx.x / SUB * (SUB / 64);
-  int t = 0;
-#pragma unroll
-  for (int i = 0; i < SUB / 64; ++i) t += ws[w0 + i];
-  __syncthreads();
-  return t;
-}
-
-// exclusive scan of v over each SUB consecutive threads
-template <int SUB>
-__device__ __forceinline__ int block_excl(int v, int *total, int *ws) {
-  const int lane = threadIdx.x & 63, w0 = (int)threadIdx.x / SUB * (SUB / 64);
-  const int w = ((int)threadIdx.x >> 6) - w0;
-  int x = v;
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const int y = __shfl_up(x, o, 64);
-    if (lane >= o) x += y;
-  }
-  if (lane == 63) ws[threadIdx.x >> 6] = x;
-  __syncthreads();
-  int base = 0, tot = 0;
-#pragma unroll
-  for (int i = 0; i < SUB / 64; ++i) {
-    const int t = ws[w0 + i];
-    if (i < w) base += t;
-    tot += t;
-  }
-  __syncthreads();
-  *total = tot;
-  return base + x - v;
-}
 
 // (kColScanBlock threads)
 __device__ __forceinline__ void colscan_body(const Dev &d, int64_t ncol, int64_t tile) {
@@ -1091,16 +1051,10 @@ __global__ __launch_bounds__(256) void k_pull(Dev d, Geo g) {
 // ---- the rebuild stage in one launch ----------------------------------------
 // Every launch costs 1.55 us also on a step that does not rebuild, so up to
 // kOneLaunchBonds one launch runs the seven passes, with a barrier between
-// them among its blocks.  A barrier never waits for a block that is not
-// running: the blocks that take part are those that have arrived when the
-// first of them closes the door -- when all have, or after kDoorTicks --
-// and a block that arrives later leaves at once.  The passes take their block
-// index and count from that, so any number of blocks (one, if need be) does
-// all the work.  Measured (device-scope release and acquire included): a
-// barrier 3.5 us among 64 blocks, 7 among 256, 12 among 512, against 1.55 us
-// for a kernel boundary; hence few, large blocks, and the launches for larger
-// systems, whose passes want more of them.  us a step, seven launches against
-// one: 1k bonds 25.7 / 22.4, FP64 1.2k 31.4 / 27.3, 52k 31.9 / 29.6, 62k with
+// them among its blocks (sc_block.h): 3.5 us among 64 blocks, 7 among 256,
+// against 1.55 us for a kernel boundary; hence few, large blocks, and the
+// launches for larger systems, whose passes want more of them.  us a step,
+// seven launches against one: 1k bonds 25.7 / 22.4, FP64 1.2k 31.4 / 27.3, 52k 31.9 / 29.6, 62k with
 // stress sums 34.2 / 31.6, 101k 36.4 / 32.9; FP64 155k 55.3 / 56.0, so the
 // line is drawn at 128k.
 constexpr int kOneBlock = 1024;
@@ -1119,88 +1073,19 @@ static inline unsigned one_blocks(const Geo &g) {
   return (unsigned)std::min<int64_t>(std::max<int64_t>(b, 1), 128);
 }
 
-constexpr uint32_t kDoorClosed = 0x80000000u;
-constexpr long long kDoorTicks = 2000;  // of the 100 MHz clock: 20 us
-
-__device__ __forceinline__ uint32_t bar_load(const uint32_t *p) {
-  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ uint32_t bar_add(uint32_t *p) {
-  return __hip_atomic_fetch_add(p, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-// All threads: enters the block; false when it came too late.  *rank and
-// *parts: its number among the blocks taking part, and how many those are.
-// `blocks`: those of the launch that belong to the system.
-__device__ __forceinline__ bool door_enter(RebuildBar *b, uint32_t blocks, int *rank,
-                                           int *parts) {
-  __shared__ uint32_t sr, sp;
-  if (threadIdx.x == 0) {
-    const uint32_t r = bar_add(&b->arrived);
-    uint32_t p = 0;
-    if (r == 0) {  // the first to arrive closes the door
-      const long long t0 = wall_clock64();
-      while (bar_load(&b->arrived) < blocks && wall_clock64() - t0 < kDoorTicks)
-        __builtin_amdgcn_s_sleep(1);
-      p = __hip_atomic_fetch_or(&b->arrived, kDoorClosed, __ATOMIC_RELAXED,
-                                __HIP_MEMORY_SCOPE_AGENT);
-      __hip_atomic_store(&b->parts, p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    } else if (!(r & kDoorClosed)) {
-      while ((p = bar_load(&b->parts)) == 0) __builtin_amdgcn_s_sleep(1);
-    }
-    sr = r;
-    sp = p;
-  }
-  __syncthreads();
-  *rank = (int)(sr & ~kDoorClosed);
-  *parts = (int)sp;
-  return !(sr & kDoorClosed);
-}
-
-// Barrier `k` of a launch among the `parts` blocks inside (all threads).  The
-// arrivals are counted in kBarGroups groups and the full groups in one word,
-// as atomics on one address serialise.
-__device__ __forceinline__ void bar_wait(RebuildBar *b, int k, int rank, int parts) {
-  __syncthreads();
-  if (parts > 1 && threadIdx.x == 0) {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-    const int grp = rank % kBarGroups;
-    const uint32_t size = (uint32_t)((parts - grp + kBarGroups - 1) / kBarGroups);
-    const uint32_t groups = (uint32_t)(parts < kBarGroups ? parts : kBarGroups);
-    if (bar_add(&b->group[k][grp][0]) + 1 == size) bar_add(&b->full[k][0]);
-    while (bar_load(&b->full[k][0]) < groups) __builtin_amdgcn_s_sleep(1);
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-  }
-  __syncthreads();
-}
-
-// Every block of the launch, last thing.  A block that comes late must still
+// The block that leaves last: until then a block that comes late must still
 // find the rebuild decided as the others did, or it would leave uncounted; so
 // what the decision is taken from -- the displacement slots, Ctl's abort word
-// -- changes only here, by the block that leaves last, which also clears the
-// counters for the next launch (nobody looks at them any more).
-__device__ __forceinline__ void door_leave(const Dev &d, uint32_t blocks) {
-  __shared__ int last;
-  RebuildBar *b = d.bar;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-    last = bar_add(&b->gone) + 1 == blocks;
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-  }
-  __syncthreads();
-  if (!last) return;
+// -- changes only here.
+__device__ __forceinline__ void rebuild_one_end(const Dev &d) {
   clear_dr_slots(d);
-  uint32_t *count = &b->full[0][0];
-  constexpr int kCounts = (int)((sizeof(b->full) + sizeof(b->group)) / sizeof(uint32_t));
-  for (int i = threadIdx.x; i < kCounts; i += blockDim.x) count[i] = 0;
   if (threadIdx.x != 0) return;
+  Door *b = d.door;
   Ctl *c = d.ctl;
   if (b->overflow) c->overflow = 1;
   if (b->err) c->err = b->err;
   if (b->abort) c->abort = 1;
   b->overflow = b->err = b->abort = 0;
-  b->arrived = b->parts = b->gone = 0;
 }
 
 // the passes' stages, one after the other in the same memory
@@ -1218,26 +1103,29 @@ __device__ __forceinline__ void rebuild_one_body(const Dev &d, const Geo &g, uin
   } else {
     if (guard_off(d.ctl, kGuardRebuild)) return;
   }
-  RebuildBar *bar = d.bar;
+  Door *door = d.door;
   int rank, parts;
-  if (door_enter(bar, blocks, &rank, &parts)) {
+  if (door_enter(door, blocks, &rank, &parts)) {
     const int64_t ncol = (int64_t)g.n1d * g.n1d;
     keys_body<kOneBlock>(d, g, rank, parts, L.keys);
-    bar_wait(bar, 0, rank, parts);
+    bar_wait(door, 0, rank, parts);
     for (int64_t t = rank; t * kColScanTile < ncol; t += parts) colscan_body(d, ncol, t);
-    bar_wait(bar, 1, rank, parts);
+    bar_wait(door, 1, rank, parts);
     scatter_body(d, g, rank, parts);
-    bar_wait(bar, 2, rank, parts);
+    bar_wait(door, 2, rank, parts);
     colsort_body<kOneBlock>(d, g, rank, parts, L.col);
-    bar_wait(bar, 3, rank, parts);
+    bar_wait(door, 3, rank, parts);
     deg_body(d, g, rank, parts);
-    bar_wait(bar, 4, rank, parts);
+    bar_wait(door, 4, rank, parts);
     for (int64_t s = rank; s * (kOneBlock / 256) < n_supers(g.nb); s += parts)
       degsum_body<kOneBlock>(d, g, s);
-    bar_wait(bar, 5, rank, parts);
-    pull_body<kOneBlock>(d, g, rank, parts, {&bar->abort, &bar->err, &bar->overflow}, L.pull);
+    bar_wait(door, 5, rank, parts);
+    pull_body<kOneBlock>(d, g, rank, parts, {&door->abort, &door->err, &door->overflow}, L.pull);
   }
-  door_leave(d, blocks);
+  if (door_leave(door, blocks)) {
+    rebuild_one_end(d);
+    door_reset(door);
+  }
 }
 
 template <bool FOLD>
