@@ -956,7 +956,7 @@ int system_create(const sc_params *params, hipStream_t stream, Arena *arena,
   g.n1d = n1d;
   g.thr = 0.25 * cell_len * cell_len;
   g.n_cells = (int64_t)n1d * n1d * n1d;
-  g.occ_words = (n1d + 31) / 32;
+  g.occ_words = sc::occ_words_of(n1d);
   build_home_order(g);
   g.stoch = p.stoch_flag ? 1 : 0;
   g.seed = p.seed;
@@ -1033,7 +1033,6 @@ int system_batch_done(sc_handle h, const Ctl &c, int64_t target, int *done) {
 
 size_t system_estimate_bytes(const sc_params *params, int32_t nf, int64_t ns, int n_bins) {
   const int64_t n1d = cells_per_side(*params);
-  const int64_t n_cells = n1d * n1d * n1d;
   const int64_t nb = ns - nf;
   auto R = [](int64_t n) { return Arena::round((size_t)(n > 0 ? n : 1)); };
   size_t b = R(sizeof(Ctl)) + R(8 * sc::kDrSlots) + R(sizeof(sc::Door)) + R(4 * (nf + 1)) + 2 * R(4 * (int64_t)nf) +
@@ -1042,10 +1041,9 @@ size_t system_estimate_bytes(const sc_params *params, int32_t nf, int64_t ns, in
   b += 4 * R(24 * ns) + 2 * R(8 * ns);                    // r, rp, fr, dr0, acc, acc_prev
   const int64_t rec_bytes = params->precision == SC_PREC_MIXED ? 32 : 64;
   b += R(rec_bytes * nb) + 2 * R(24 * nb) + R(8 * nb);    // record, F, T (at most), tension
-  const int64_t ncol = n1d * n1d, occ_words = (n1d + 31) / 32;
+  const int64_t ncol = n1d * n1d, occ_words = occ_words_of(n1d);
   b += R(4 * nb) + R(4 * ncol) + R(4 * (ncol + 1)) + R(8 * nb) + R(4 * nb);  // keys, columns, col_tmp, col_rank
-  b += R(8 * n_cells) + R(4 * ncol * occ_words);                 // cell runs, occupancy
-  b += R(2 * ncol * occ_words) + R(4 * ncol) + R(4 * nb);        // run tables
+  b += R(8 * ncol * occ_words) + R(4 * (nb + 1));                // occupancy, cell starts
   b += 2 * R(4 * nb) + R(4 * nb) + R(4 * (nb + 1));  // sorted, skey, deg, inc_start
   b += R(8 * sc::kRunSlab * nb);                      // run slabs
   const int64_t tmp = scan_tmp_elems(ncol, nb);
@@ -1255,13 +1253,10 @@ int sc_load_filaments(sc_handle h, int32_t nf, const int32_t *site_off,
   if ((rc = dalloc(h, &d.col_start, ncol + 1, false))) return rc;
   if ((rc = dalloc(h, &d.col_tmp, nb, false))) return rc;
   if ((rc = dalloc(h, &d.col_rank, nb, false))) return rc;
-  if ((rc = dalloc(h, &d.cell_run, g.n_cells, false))) return rc;
   if ((rc = dalloc(h, &d.sorted, nb, false))) return rc;
   if ((rc = dalloc(h, &d.skey, nb, false))) return rc;
   if ((rc = dalloc(h, &d.cell_occ, ncol * g.occ_words, false))) return rc;
-  if ((rc = dalloc(h, &d.occ_pre, ncol * g.occ_words, false))) return rc;
-  if ((rc = dalloc(h, &d.col_ncell, ncol, false))) return rc;
-  if ((rc = dalloc(h, &d.cell_first, nb, false))) return rc;
+  if ((rc = dalloc(h, &d.cell_first, nb + 1, false))) return rc;
   if ((rc = dalloc(h, &d.deg, nb, false))) return rc;
   if ((rc = dalloc(h, &d.nrun, sc::kRunSlab * (size_t)nb, false))) return rc;
   if ((rc = dalloc(h, &d.inc_start, nb + 1, false))) return rc;
@@ -1316,7 +1311,7 @@ int sc_load_filaments(sc_handle h, int32_t nf, const int32_t *site_off,
   HIPCHK(h, hipMemsetAsync(d.bpote, 0, sizeof(double) * nb, h->stream));
   HIPCHK(h, hipMemsetAsync(d.stress_acc, 0, sizeof(double) * 6 * stress_slots(nb), h->stream));
   HIPCHK(h, hipMemsetAsync(d.col_count, 0, sizeof(int32_t) * ncol, h->stream));
-  HIPCHK(h, hipMemsetAsync(d.cell_occ, 0, sizeof(uint32_t) * ncol * g.occ_words, h->stream));
+  HIPCHK(h, hipMemsetAsync(d.cell_occ, 0, sizeof(int2) * ncol * g.occ_words, h->stream));
   HIPCHK(h, hipMemsetAsync(d.deg, 0, sizeof(int32_t) * nb, h->stream));
   Ctl c{};
   if ((rc = write_ctl(h, c))) return rc;

@@ -180,7 +180,7 @@ __global__ __launch_bounds__(kXlBlock) void k_xl_events(Dev d, Geo g) {
         const int X = ((cx + off0 + dx) % n + n) % n, Y = ((cy + off0 + dy) % n + n) % n;
         const int Z = ((cz + off0 + dz) % n + n) % n;
         if (!cell_occupied(d, g, X, Y, Z)) continue;  // empty cell
-        const int2 run = d.cell_run[(X * n + Y) * n + Z];
+        const int2 run = cell_run_of(d, g, X, Y, Z);
         for (int32_t j = run.x; j < run.y; ++j) {
           const int32_t b = d.sorted[j];
           if (b == bs) continue;

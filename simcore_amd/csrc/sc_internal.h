@@ -50,7 +50,7 @@ struct Geo {
   double delta;
   double thr;              // 0.25 * cell_len^2
   int n1d;
-  int occ_words;           // 32-bit occupancy words per cell column
+  int occ_words;           // words of a column in Dev::cell_occ
   int stoch;
   int compact;             // mixed precision: 32-byte bond records (sc_math.h)
   double inv_n1d;
@@ -73,6 +73,10 @@ struct Geo {
   // face: (x == 0 ? 0 : x == n-1 ? 2 : 1) * 6 + (y likewise) * 2 + (z > 0)
   uint64_t home_order[18];
 };
+
+// Words of a cell column's occupancy bits 0 to n1d + 1, of which any two
+// neighbours from (n1d - 1) / 32 down are read together.
+inline int occ_words_of(int64_t n1d) { return (int)((n1d - 1) / 32 + 2); }
 
 // Device pointers (a plain struct so it can be passed by value).
 // Per-wave maxima of the displacement accumulator go to kDrSlots slots
@@ -129,13 +133,16 @@ struct Dev {
   int32_t *col_rank;       // nb: a bond's place in its column (build scratch)
   int64_t *col_tmp;        // nb: key << 32 | bond, grouped by column, unordered
   int32_t *sorted, *skey;  // nb: bonds in (key, bond) order, their keys
-  int2 *cell_run;          // n_cells: [start, end) of an occupied cell
-  uint32_t *cell_occ;      // n1d^2 * occ_words: bit z of column (x, y)
-  uint16_t *occ_pre;       // n1d^2 * occ_words: occupied cells in the
-                           // column's words before this one
-  int32_t *col_ncell;      // n1d^2: occupied cells of each column
-  int32_t *cell_first;     // nb: per column, at its range of `sorted`, the
-                           // first entry of each occupied cell in z order
+  int2 *cell_occ;          // n1d^2 * occ_words, per column 32 cells a word:
+                           // {occupancy, index in cell_first of the run of
+                           // the word's first occupied cell}.  Cell z is bit
+                           // z + 1; bit 0 repeats cell n1d - 1 and bit
+                           // n1d + 1 cell 0, so two neighbouring words hold
+                           // any cell and the cells above and below it
+  int32_t *cell_first;     // nb + 1: per column, at its range of `sorted`, the
+                           // first entry of each occupied cell in z order,
+                           // then the column's end: a run ends where the
+                           // next begins
   // candidates: per bond, its incidences in candidate order (CSR over
   // inc_start), each with its own copy of the pair's sticky force -- both
   // owners compute the same bits, so the copies agree, and a bond's slot
@@ -287,11 +294,20 @@ constexpr int kPullGroup = 256;  // bonds whose lists a block of the list pass w
 
 enum Guard { kGuardStep = 0, kGuardRebuild = 1 };
 
-// Cell-list lookups.  Occupancy bit of cell (x, y, z); run of an occupied
-// cell (its members in bond order).
+// Cell-list lookups.  Occupancy of cell (x, y, z); run [start, end) in
+// `sorted` of an occupied cell (its members in bond order).
+__device__ __forceinline__ int2 cell_word(const Dev &d, const Geo &g, int x, int y, int z) {
+  return d.cell_occ[((int64_t)x * g.n1d + y) * g.occ_words + ((z + 1) >> 5)];
+}
 __device__ __forceinline__ bool cell_occupied(const Dev &d, const Geo &g, int x, int y, int z) {
-  const uint32_t w = d.cell_occ[((int64_t)x * g.n1d + y) * g.occ_words + (z >> 5)];
-  return (w >> (z & 31)) & 1u;
+  return ((uint32_t)cell_word(d, g, x, y, z).x >> ((z + 1) & 31)) & 1u;
+}
+__device__ __forceinline__ int2 cell_run_of(const Dev &d, const Geo &g, int x, int y, int z) {
+  const int2 w = cell_word(d, g, x, y, z);
+  int2 run;
+  __builtin_memcpy(&run, d.cell_first + w.y + __popc((uint32_t)w.x & ((1u << ((z + 1) & 31)) - 1u)),
+                   sizeof(run));
+  return run;
 }
 
 // Launchers (sc_kernels.hip).  All are asynchronous on `st`.

@@ -506,13 +506,13 @@ __global__ void k_scatter(Dev d, Geo g, int guard) {
 // A column's lanes lie in one wavefront and share nothing with others, so the
 // pass has no block barrier.  Bound: the latency of a column's few loads.
 // Sixteen lanes keep 4 columns in flight per wavefront and most lanes busy at
-// 2-30 bonds a column.  Active: uneven 1.6M bonds 44 us, dense 620k 21 us (one
-// column per wavefront, keys gathered: 46 and 24.5); in the one-launch rebuild,
+// 2-30 bonds a column.  Active: uneven 1.6M bonds 37 us, dense 620k 18 us (one
+// column per wavefront, keys gathered: 7 and 6 us more); in the one-launch rebuild,
 // where a few hundred wavefronts serve all columns, 52k bonds gained 1.1 us a
 // step.
 constexpr int kColLanes = 16;
 constexpr int kColStage = 96;
-constexpr int kOccWords = 44;  // occ_words <= 41 (n1d^3 < 2^31)
+constexpr int kOccWords = 44;  // occ_words <= 42 (n1d^3 < 2^31)
 
 template <int BLOCK>
 struct ColsortLds {
@@ -594,47 +594,35 @@ __device__ __forceinline__ void colsort_body(const Dev &d, const Geo &g, int64_t
       if (start) {
         const int32_t rank = ncell + __popc(bal & ((1u << lane) - 1u));
         d.cell_first[s + rank] = s + i;
-        int32_t j = i + 1;
-        while (j < m && (staged ? kr[j] : d.skey[s + j]) == k) ++j;
-        d.cell_run[k] = make_int2(s + i, s + j);
-        const int z = k - (int32_t)c * n;
-        atomicOr(&occ[z >> 5], 1u << (z & 31));
+        const int p = k - (int32_t)c * n + 1;
+        atomicOr(&occ[p >> 5], 1u << (p & 31));
       }
       ncell += __popc(bal);
     }
     wave_sync();
-    if (live)
+    if (live) {
+      // (the copies of the first and the last cell beyond the ends count for
+      // no run index)
+      const uint32_t below = (occ[n >> 5] >> (n & 31)) & 1u, above = (occ[0] >> 1) & 1u;
       for (int w = lane; w < W; w += kColLanes) {
-        int pre = 0;
-        for (int v = 0; v < w; ++v) pre += __popc(occ[v]);
-        d.cell_occ[c * W + w] = occ[w];
-        d.occ_pre[c * W + w] = (uint16_t)pre;
+        int at = s;
+        for (int v = 0; v < w; ++v) at += __popc(occ[v]);
+        uint32_t bits = occ[w];
+        if (w == 0) {
+          bits |= below;
+          at -= (int)below;
+        }
+        if (w == (n + 1) >> 5) bits |= above << ((n + 1) & 31);
+        d.cell_occ[c * W + w] = make_int2((int32_t)bits, at);
       }
-    if (live && lane == 0) d.col_ncell[c] = ncell;
+      // where the last run of the column ends (the first of the next column
+      // starts there if every bond is a run of its own)
+      if (lane == 0 && ncell < m) d.cell_first[s + ncell] = e;
+      if (lane == 0 && c == ncol - 1) d.cell_first[e] = e;
+    }
     wave_sync();
   }
 }
-
-// Run [start, end) in `sorted` of the occupied cell (x, y, z): its rank
-// among its column's occupied cells (the occupancy bits below z plus the
-// word's prefix count) indexes the column's run table.
-__device__ __forceinline__ int2 cell_run_of(const Dev &d, const Geo &g, int x, int y, int z) {
-  const int64_t c = (int64_t)x * g.n1d + y;
-  const int64_t wi = c * g.occ_words + (z >> 5);
-  const uint32_t word = d.cell_occ[wi];
-  const int32_t s0 = d.col_start[c];
-  const int32_t nc = d.col_ncell[c];
-  const int32_t rank = d.occ_pre[wi] + __popc(word & ((1u << (z & 31)) - 1u));
-  const int32_t a = d.cell_first[s0 + rank];
-  const int32_t b = rank + 1 < nc ? d.cell_first[s0 + rank + 1] : d.col_start[c + 1];
-  return make_int2(a, b);
-}
-
-__device__ __forceinline__ int2 cell_run_key(const Dev &d, const Geo &g, int32_t k) {
-  const int n = g.n1d;
-  return cell_run_of(d, g, k / (n * n), (k / n) % n, k % n);
-}
-
 
 constexpr int kColBlock = 256;
 constexpr int64_t kColBlocks = 1024;  // (blocks loop over the columns)
@@ -687,29 +675,36 @@ __device__ __forceinline__ void shell_cell(int n, int x, int y, int z, int q, in
   *zo = zp;
 }
 
-template <bool BACK>
-__device__ __forceinline__ int32_t shell_key(int n, int x, int y, int z, int q) {
-  int xp, yp, zp;
-  shell_cell<BACK>(n, x, y, z, q, &xp, &yp, &zp);
-  return ((int32_t)xp * n + yp) * n + zp;
-}
-
 // Occupancy of the 26 neighbours of cell (cx, cy, cz): bit q the half-shell
-// cell q, bit 13 + q the mirrored half-shell cell q.  The 26 reads are
-// independent and go out together (one round trip to L2, where the mask
-// lives), so the list passes then read the runs of the few occupied cells
-// only.
-__device__ __forceinline__ uint32_t shell_mask(const Dev &d, const Geo &g, int cx, int cy,
-                                               int cz) {
+// cell q, bit 13 + q the mirrored half-shell cell q; *own: the run of the cell
+// itself.  Nine independent loads, one for each column: two words of its
+// table hold the bits of cz - 1, cz and cz + 1, also across the periodic
+// faces.  (26 loads, one a cell, and three more for each run kept the load
+// units of k_deg 70% busy.  Active, 1.6M uneven bonds: k_deg 114 -> 103 us,
+// k_colsort 44 -> 37 without its table of runs by cell.)
+__device__ __forceinline__ uint32_t shell_mask(const Dev &d, const Geo &g, int cx, int cy, int cz,
+                                               int2 *own) {
   const int n = g.n1d;
+  const int xs[3] = {cx == 0 ? n - 1 : cx - 1, cx, cx == n - 1 ? 0 : cx + 1};
+  const int ys[3] = {cy == 0 ? n - 1 : cy - 1, cy, cy == n - 1 ? 0 : cy + 1};
   uint32_t m = 0;
 #pragma unroll
-  for (int q = 0; q < 13; ++q) {
-    int x, y, z;
-    shell_cell<false>(n, cx, cy, cz, q, &x, &y, &z);
-    m |= (uint32_t)cell_occupied(d, g, x, y, z) << q;
-    shell_cell<true>(n, cx, cy, cz, q, &x, &y, &z);
-    m |= (uint32_t)cell_occupied(d, g, x, y, z) << (13 + q);
+  for (int i = 0; i < 9; ++i) {
+    const int dx = i % 3 - 1, dy = i / 3 - 1;
+    const int64_t c = (int64_t)xs[dx + 1] * n + ys[dy + 1];
+    int4 w;  // {bits, index} of two words
+    __builtin_memcpy(&w, d.cell_occ + c * g.occ_words + (cz >> 5), sizeof(w));
+    const uint64_t bits = (uint32_t)w.x | (uint64_t)(uint32_t)w.z << 32;
+    const uint32_t v = (uint32_t)(bits >> (cz & 31));
+    m |= ((v >> 2) & 1u) << (4 + (dy + 1) * 3 + dx + 1);
+    m |= (v & 1u) << (17 + (1 - dy) * 3 + 1 - dx);
+    if (dy == 1 || (dy == 0 && dx == 1)) m |= ((v >> 1) & 1u) << (dy == 1 ? dx + 2 : 0);
+    if (dy == -1 || (dy == 0 && dx == -1)) m |= ((v >> 1) & 1u) << (13 + (dy == -1 ? 2 - dx : 0));
+    if (dx == 0 && dy == 0) {
+      const int p = (cz & 31) + 1;
+      const int at = p < 32 ? w.y + __popc((uint32_t)w.x & ((1u << p) - 1u)) : w.w;
+      __builtin_memcpy(own, d.cell_first + at, sizeof(*own));
+    }
   }
   return m;
 }
@@ -740,14 +735,14 @@ __device__ __forceinline__ Excl excl_of(const Dev &d, const Geo &g, int32_t b) {
 __device__ __forceinline__ void deg_one(const Dev &d, const Geo &g, int64_t p) {
   const int32_t k = d.skey[p];
   const int32_t b = d.sorted[p];
-  const int2 own = cell_run_key(d, g, k);
   const Excl x = excl_of(d, g, b);
   const int32_t klo = x.lo >= 0 ? d.keys[x.lo] : -1;
   const int32_t khi = x.hi >= 0 ? d.keys[x.hi] : -1;
-  int32_t deg = (own.y - own.x - 1) - (klo == k) - (khi == k);
   const int n = g.n1d;
   const int cx = k / (n * n), cy = (k / n) % n, cz = k % n;
-  const uint32_t m = shell_mask(d, g, cx, cy, cz);
+  int2 own;
+  const uint32_t m = shell_mask(d, g, cx, cy, cz, &own);
+  int32_t deg = (own.y - own.x - 1) - (klo == k) - (khi == k);
   // the bond's own run, those of its first kRunSlab - 2 occupied stencil
   // cells (in bit order) and the occupancy mask go to the bond's slab (64
   // bytes, one whole line, so the scattered stores waste nothing), where
@@ -917,7 +912,7 @@ __device__ __forceinline__ void pull_one(const Dev &d, const Geo &g, int32_t b,
   const int4 s0 = sl[0], s1 = sl[1], s2 = sl[2], s3 = sl[3];
   const int2 own = make_int2(s0.x, s0.y);
   const uint32_t m = (uint32_t)s3.z;
-  auto run_of = [&](int q, int32_t key) -> int2 {
+  auto run_of = [&](int q) -> int2 {
     const int idx = 1 + __popc(m & ((1u << q) - 1u));
     switch (idx) {
       case 1: return make_int2(s0.z, s0.w);
@@ -926,8 +921,14 @@ __device__ __forceinline__ void pull_one(const Dev &d, const Geo &g, int32_t b,
       case 4: return make_int2(s2.x, s2.y);
       case 5: return make_int2(s2.z, s2.w);
       case 6: return make_int2(s3.x, s3.y);
-      default: return d.cell_run[key];
+      default: break;
     }
+    int x, y, z;
+    if (q < 13)
+      shell_cell<false>(n, cx, cy, cz, q, &x, &y, &z);
+    else
+      shell_cell<true>(n, cx, cy, cz, q - 13, &x, &y, &z);
+    return cell_run_of(d, g, x, y, z);
   };
   uint64_t order = g.home_order[cls];
   for (int step = 0; step < 14; ++step, order >>= 4) {
@@ -943,12 +944,12 @@ __device__ __forceinline__ void pull_one(const Dev &d, const Geo &g, int32_t b,
       for (int32_t j = r + 1; j < own.y; ++j) put(d.sorted[j], 0);
       for (uint32_t mm = m & 0x1fffu; mm; mm &= mm - 1) {
         const int q = __ffs(mm) - 1;
-        const int2 rn = run_of(q, shell_key<false>(n, cx, cy, cz, q));
+        const int2 rn = run_of(q);
         for (int32_t j = rn.x; j < rn.y; ++j) put(d.sorted[j], 0);
       }
     } else if ((m >> (13 + c)) & 1u) {
       // mirrored half-shell cell c: b is obj2 of each of its members
-      const int2 rn = run_of(13 + c, shell_key<true>(n, cx, cy, cz, c));
+      const int2 rn = run_of(13 + c);
       for (int32_t j = rn.x; j < rn.y; ++j) put(d.sorted[j], 1);
     }
   }
@@ -1035,10 +1036,10 @@ __device__ __forceinline__ void pull_body(const Dev &d, const Geo &g, int64_t bi
     const int32_t base = __shfl(w, 0, 64), cnt = __shfl(wend, 63, 64) - base;
     const bool staged = cnt <= kPullStage;
     if (b < g.nb) pull_one(d, g, (int32_t)b, w, wend, staged ? L.stage[wv] : nullptr, base, fail);
-    __syncthreads();
+    wave_sync();
     if (staged)
       for (int i = lane; i < cnt; i += 64) d.inc[base + i] = L.stage[wv][i];
-    __syncthreads();
+    wave_sync();
   }
 }
 
