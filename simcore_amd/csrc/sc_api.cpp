@@ -639,13 +639,12 @@ void to_caller(const sc_system *h, const std::vector<int64_t> &map, const T *src
 // one stress slot, whatever launch shape is set while the sum accumulates.
 int64_t stress_slots(int64_t nb) { return nb / 64 + 2; }
 
-// Scratch between steps: the rebuild's run slabs (kRunSlab * 8 bytes per
-// bond), which only the launches between the degree and the list pass of one
+// Scratch between steps: the rebuild's run slabs (64 bytes per bond), which only the launches between the degree and the list pass of one
 // rebuild use.  Every filament has at least two bonds, so it holds three
 // FP64 components of every site, or six of every filament.
-double *idle_scratch(const sc_system *h) { return reinterpret_cast<double *>(h->d.nrun); }
+double *idle_scratch(const sc_system *h) { return reinterpret_cast<double *>(h->d.slab); }
 size_t idle_scratch_bytes(const sc_system *h) {
-  return sizeof(int2) * sc::kRunSlab * (size_t)h->g.nb;
+  return sizeof(int32_t) * sc::kSlabWords * (size_t)h->g.nb;
 }
 
 // Reordered or FP32 arrays of at least this many values are put into the
@@ -1045,7 +1044,7 @@ size_t system_estimate_bytes(const sc_params *params, int32_t nf, int64_t ns, in
   b += R(4 * nb) + R(4 * ncol) + R(4 * (ncol + 1)) + R(8 * nb) + R(4 * nb);  // keys, columns, col_tmp, col_rank
   b += R(8 * ncol * occ_words) + R(4 * (nb + 1));                // occupancy, cell starts
   b += 2 * R(4 * nb) + R(4 * nb) + R(4 * (nb + 1));  // sorted, skey, deg, inc_start
-  b += R(8 * sc::kRunSlab * nb);                      // run slabs
+  b += R(4 * sc::kSlabWords * nb);                    // run slabs
   const int64_t tmp = scan_tmp_elems(ncol, nb);
   b += R(4 * tmp);
   b += R(4 * (int64_t)nf) + (size_t)n_bins * Arena::kAlign;  // bin lists
@@ -1258,7 +1257,7 @@ int sc_load_filaments(sc_handle h, int32_t nf, const int32_t *site_off,
   if ((rc = dalloc(h, &d.cell_occ, ncol * g.occ_words, false))) return rc;
   if ((rc = dalloc(h, &d.cell_first, nb + 1, false))) return rc;
   if ((rc = dalloc(h, &d.deg, nb, false))) return rc;
-  if ((rc = dalloc(h, &d.nrun, sc::kRunSlab * (size_t)nb, false))) return rc;
+  if ((rc = dalloc(h, &d.slab, sc::kSlabWords * (size_t)nb, false))) return rc;
   if ((rc = dalloc(h, &d.inc_start, nb + 1, false))) return rc;
   int64_t tmp = sc::scan_tmp_elems(ncol, nb);
   if ((rc = dalloc(h, &d.scan_tmp, tmp, false))) return rc;

@@ -149,10 +149,8 @@ struct Dev {
   // traffic follows its list.  The candidate list itself is implicit (the
   // reference's order is recovered from the lists for the taps).
   int32_t *deg, *inc_start;
-  int2 *nrun;              // per bond, rebuild scratch: kRunSlab entries (own
-                           // cell's run, the first six occupied stencil
-                           // cells' runs, the stencil occupancy mask: bits
-                           // 0-12 half shell, 13-25 mirrored)
+  int32_t *slab;           // nb * kSlabWords, rebuild scratch: a bond's cell
+                           // runs in list order (k_deg)
   int2 *inc;               // {partner bond, role | written << 1 | (owner
                            // mod 64) << 2}: role 1 when the bond is obj2;
                            // written once the slot holds a force (a slot
@@ -205,7 +203,7 @@ struct Tune {
                          // integrator then runs beside the rest of the pass
 };
 constexpr int kMaxParts = 8;
-constexpr int kRunSlab = 8;  // cell runs kept per bond between the list passes
+constexpr int kSlabWords = 16;  // words per bond kept between the list passes
 constexpr int64_t kPairAlign = 512;  // range cuts: a multiple of every block size
 
 // Length bins of the integrator, as the step loop hands them over.
@@ -294,6 +292,15 @@ constexpr int kPullGroup = 256;  // bonds whose lists a block of the list pass w
 
 enum Guard { kGuardStep = 0, kGuardRebuild = 1 };
 
+// two words from a four-byte boundary in one load
+__device__ __forceinline__ int2 two_at(const int32_t *p) {
+  struct __attribute__((packed, aligned(4))) Two {
+    int32_t x, y;
+  };
+  const Two t = *reinterpret_cast<const Two *>(p);
+  return make_int2(t.x, t.y);
+}
+
 // Cell-list lookups.  Occupancy of cell (x, y, z); run [start, end) in
 // `sorted` of an occupied cell (its members in bond order).
 __device__ __forceinline__ int2 cell_word(const Dev &d, const Geo &g, int x, int y, int z) {
@@ -304,10 +311,7 @@ __device__ __forceinline__ bool cell_occupied(const Dev &d, const Geo &g, int x,
 }
 __device__ __forceinline__ int2 cell_run_of(const Dev &d, const Geo &g, int x, int y, int z) {
   const int2 w = cell_word(d, g, x, y, z);
-  int2 run;
-  __builtin_memcpy(&run, d.cell_first + w.y + __popc((uint32_t)w.x & ((1u << ((z + 1) & 31)) - 1u)),
-                   sizeof(run));
-  return run;
+  return two_at(d.cell_first + w.y + __popc((uint32_t)w.x & ((1u << ((z + 1) & 31)) - 1u)));
 }
 
 // Launchers (sc_kernels.hip).  All are asynchronous on `st`.

@@ -638,75 +638,51 @@ static inline unsigned colsort_grid(int64_t ncol) {
   return (unsigned)std::min<int64_t>((ncol + kCols - 1) / kCols, kColBlocks);
 }
 
-// Coordinates of the q-th cell of the half-shell stencil of (x, y, z) in
+// The 27 cells around (x, y, z) are numbered (dx + 1) + 3 (dy + 1) +
+// 9 (dz + 1): 13 is the cell itself, 14 + q the q-th cell of its half shell in
 // the order of CellList::AssignCellNeighbors (src/cell_list.cpp:206-262):
-// (x+1, y, z); (x-1..x+1, y+1, z); then (x-1..x+1, y-1..y+1, z+1), x
-// fastest.  BACK: the mirrored half shell, the 13 cells whose half shell
-// holds (x, y, z) (offsets negated).  Periodic wrap; with at least 3 cells
-// per side the 13 + 13 + 1 cells are distinct.
-template <bool BACK>
-__device__ __forceinline__ void shell_cell(int n, int x, int y, int z, int q, int *xo, int *yo,
-                                           int *zo) {
-  int dx, dy, dz;
-  if (q == 0) {
-    dx = 1;
-    dy = 0;
-    dz = 0;
-  } else if (q < 4) {
-    dx = q - 2;
-    dy = 1;
-    dz = 0;
-  } else {
-    dx = (q - 4) % 3 - 1;
-    dy = (q - 4) / 3 - 1;
-    dz = 1;
-  }
-  if (BACK) {
-    dx = -dx;
-    dy = -dy;
-    dz = -dz;
-  }
-  int xp = x + dx, yp = y + dy, zp = z + dz;
-  xp = xp < 0 ? n - 1 : (xp == n ? 0 : xp);
-  yp = yp < 0 ? n - 1 : (yp == n ? 0 : yp);
-  zp = zp < 0 ? n - 1 : (zp == n ? 0 : zp);
-  *xo = xp;
-  *yo = yp;
-  *zo = zp;
+// (x+1, y, z); (x-1..x+1, y+1, z); then (x-1..x+1, y-1..y+1, z+1), x fastest;
+// and 12 - q the q-th cell of the mirrored half shell, the 13 cells whose half
+// shell holds (x, y, z).  Periodic wrap; with at least 3 cells per side the 27
+// are distinct.
+constexpr int kOwnCell = 13;
+
+__device__ __forceinline__ void stencil_cell(int n, int x, int y, int z, int code, int *xo, int *yo,
+                                             int *zo) {
+  const int xp = x + code % 3 - 1, yp = y + code / 3 % 3 - 1, zp = z + code / 9 - 1;
+  *xo = xp < 0 ? n - 1 : (xp == n ? 0 : xp);
+  *yo = yp < 0 ? n - 1 : (yp == n ? 0 : yp);
+  *zo = zp < 0 ? n - 1 : (zp == n ? 0 : zp);
 }
 
-// Occupancy of the 26 neighbours of cell (cx, cy, cz): bit q the half-shell
-// cell q, bit 13 + q the mirrored half-shell cell q; *own: the run of the cell
-// itself.  Nine independent loads, one for each column: two words of its
-// table hold the bits of cz - 1, cz and cz + 1, also across the periodic
-// faces.  (26 loads, one a cell, and three more for each run kept the load
-// units of k_deg 70% busy.  Active, 1.6M uneven bonds: k_deg 114 -> 103 us,
-// k_colsort 44 -> 37 without its table of runs by cell.)
-__device__ __forceinline__ uint32_t shell_mask(const Dev &d, const Geo &g, int cx, int cy, int cz,
-                                               int2 *own) {
+// Occupancy of the 27 cells around (and with) cell (cx, cy, cz).  Nine independent loads, one for each column: two words
+// of its table hold the bits of cz - 1, cz and cz + 1, also across the
+// periodic faces.  (26 loads, one a cell, and three more for each run kept the
+// load units of k_deg 70% busy.  Active, 1.6M uneven bonds: k_deg 114 ->
+// 103 us, k_colsort 44 -> 37 without its table of runs by cell.)
+__device__ __forceinline__ uint32_t stencil_mask(const Dev &d, const Geo &g, int cx, int cy,
+                                                 int cz) {
   const int n = g.n1d;
   const int xs[3] = {cx == 0 ? n - 1 : cx - 1, cx, cx == n - 1 ? 0 : cx + 1};
   const int ys[3] = {cy == 0 ? n - 1 : cy - 1, cy, cy == n - 1 ? 0 : cy + 1};
   uint32_t m = 0;
 #pragma unroll
   for (int i = 0; i < 9; ++i) {
-    const int dx = i % 3 - 1, dy = i / 3 - 1;
-    const int64_t c = (int64_t)xs[dx + 1] * n + ys[dy + 1];
+    const int64_t c = (int64_t)xs[i % 3] * n + ys[i / 3];
     int4 w;  // {bits, index} of two words
     __builtin_memcpy(&w, d.cell_occ + c * g.occ_words + (cz >> 5), sizeof(w));
     const uint64_t bits = (uint32_t)w.x | (uint64_t)(uint32_t)w.z << 32;
     const uint32_t v = (uint32_t)(bits >> (cz & 31));
-    m |= ((v >> 2) & 1u) << (4 + (dy + 1) * 3 + dx + 1);
-    m |= (v & 1u) << (17 + (1 - dy) * 3 + 1 - dx);
-    if (dy == 1 || (dy == 0 && dx == 1)) m |= ((v >> 1) & 1u) << (dy == 1 ? dx + 2 : 0);
-    if (dy == -1 || (dy == 0 && dx == -1)) m |= ((v >> 1) & 1u) << (13 + (dy == -1 ? 2 - dx : 0));
-    if (dx == 0 && dy == 0) {
-      const int p = (cz & 31) + 1;
-      const int at = p < 32 ? w.y + __popc((uint32_t)w.x & ((1u << p) - 1u)) : w.w;
-      __builtin_memcpy(own, d.cell_first + at, sizeof(*own));
-    }
+    m |= ((v & 1u) << i) | (((v >> 1) & 1u) << (9 + i)) | (((v >> 2) & 1u) << (18 + i));
   }
   return m;
+}
+
+// Geo::home_order of a cell
+__device__ __forceinline__ uint64_t home_order_of(const Geo &g, int cx, int cy, int cz) {
+  const int n = g.n1d;
+  return g.home_order[(cx == 0 ? 0 : cx == n - 1 ? 2 : 1) * 6 +
+                      (cy == 0 ? 0 : cy == n - 1 ? 2 : 1) * 2 + (cz == 0 ? 0 : 1)];
 }
 
 // The bonds b-1 and b+1 when they share a site with b (Bond::HasNeighbor
@@ -728,10 +704,18 @@ __device__ __forceinline__ Excl excl_of(const Dev &d, const Geo &g, int32_t b) {
 // src/cell.cpp:14-70): the other members of its cell, the members of its 13
 // half-shell cells and of its 13 mirrored half-shell cells, less the
 // site-sharing neighbours among them.  One thread per sorted position (the
-// cell lookups of neighbouring threads then hit the same lines), no
-// atomics.  The stencil cells are recomputed per entry rather than held,
-// which keeps the register count (and so the occupancy) of this
-// latency-bound pass high.  The neighbour occupancy is kept for k_pull.
+// cell lookups of neighbouring threads then hit the same lines; in bond order
+// the pass took 133 us instead of 103 at 1.6M uneven bonds), no atomics.
+//
+// The runs go to the bond's slab in the order of its list, so the list pass,
+// which runs in bond order, only copies them: kSlabRuns starts, as many
+// lengths of a byte, and a word {runs | place of the own cell's run << 8 |
+// half-shell runs << 16}, 64 bytes, one whole line (the scattered stores waste
+// nothing).  Bonds with more runs (a mean of 4.5-5.2, at most 16 seen) or a
+// longer one are marked kSlabOver, and the list pass looks theirs up.
+constexpr int kSlabRuns = 12;
+constexpr int32_t kSlabOver = INT32_MIN;
+
 __device__ __forceinline__ void deg_one(const Dev &d, const Geo &g, int64_t p) {
   const int32_t k = d.skey[p];
   const int32_t b = d.sorted[p];
@@ -740,52 +724,61 @@ __device__ __forceinline__ void deg_one(const Dev &d, const Geo &g, int64_t p) {
   const int32_t khi = x.hi >= 0 ? d.keys[x.hi] : -1;
   const int n = g.n1d;
   const int cx = k / (n * n), cy = (k / n) % n, cz = k % n;
-  int2 own;
-  const uint32_t m = shell_mask(d, g, cx, cy, cz, &own);
-  int32_t deg = (own.y - own.x - 1) - (klo == k) - (khi == k);
-  // the bond's own run, those of its first kRunSlab - 2 occupied stencil
-  // cells (in bit order) and the occupancy mask go to the bond's slab (64
-  // bytes, one whole line, so the scattered stores waste nothing), where
-  // the list pass, which runs in bond order, reads them in coalesced loads
-  // without more dependent lookups
-  // (the first kRunSlab - 2 lookups are unrolled and independent, so they
-  // are in flight together; the slab is stored after them)
-  uint32_t mm = m;
-  int2 r[kRunSlab - 2];
-#pragma unroll
-  for (int i = 0; i < kRunSlab - 2; ++i) {
-    r[i] = make_int2(0, 0);
-    if (mm) {
-      const int q = __ffs(mm) - 1;
-      mm &= mm - 1;
-      int x, y, z;
-      if (q < 13)
-        shell_cell<false>(n, cx, cy, cz, q, &x, &y, &z);
-      else
-        shell_cell<true>(n, cx, cy, cz, q - 13, &x, &y, &z);
-      const int32_t kc = (x * n + y) * n + z;
-      r[i] = cell_run_of(d, g, x, y, z);
-      deg += (r[i].y - r[i].x) - (klo == kc) - (khi == kc);
+  const uint32_t m = stencil_mask(d, g, cx, cy, cz);
+  // the occupied cells in list order, 5 bits each
+  uint64_t seq = 0, order = home_order_of(g, cx, cy, cz);
+  int runs = 0, own_at = 0;
+  auto add = [&](int code) {
+    if (runs < kSlabRuns) seq |= (uint64_t)code << (5 * runs);
+    ++runs;
+  };
+  for (int step = 0; step < 14; ++step, order >>= 4) {
+    const int c = (int)(order & 15);
+    if (c == 13) {
+      own_at = runs;
+      add(kOwnCell);
+      for (uint32_t h = m >> 14; h; h &= h - 1) add(13 + __ffs(h));
+    } else if ((m >> (12 - c)) & 1u) {
+      add(12 - c);
     }
   }
-  for (; mm; mm &= mm - 1) {
-    const int q = __ffs(mm) - 1;
+  int32_t start[kSlabRuns], deg = -1;
+  uint32_t len[kSlabRuns];
+  bool over = runs > kSlabRuns;
+  auto run_of = [&](int code) {  // counts the run, too
     int x, y, z;
-    if (q < 13)
-      shell_cell<false>(n, cx, cy, cz, q, &x, &y, &z);
-    else
-      shell_cell<true>(n, cx, cy, cz, q - 13, &x, &y, &z);
+    stencil_cell(n, cx, cy, cz, code, &x, &y, &z);
+    const int2 r = cell_run_of(d, g, x, y, z);
     const int32_t kc = (x * n + y) * n + z;
-    const int2 rr = cell_run_of(d, g, x, y, z);
-    deg += (rr.y - rr.x) - (klo == kc) - (khi == kc);
+    deg += (r.y - r.x) - (klo == kc) - (khi == kc);
+    return r;
+  };
+#pragma unroll
+  for (int i = 0; i < kSlabRuns; ++i) {
+    start[i] = 0;
+    len[i] = 0;
+    if (i < runs) {
+      const int2 r = run_of((int)(seq >> (5 * i)) & 31);
+      start[i] = r.x;
+      len[i] = (uint32_t)(r.y - r.x);
+      over = over || r.y - r.x > 255;
+    }
+  }
+  if (runs > kSlabRuns) {  // all of them again
+    deg = -1;
+    for (uint32_t h = m; h; h &= h - 1) run_of(__ffs(h) - 1);
   }
   d.deg[b] = deg;
-  int4 *slab = reinterpret_cast<int4 *>(d.nrun + (int64_t)b * kRunSlab);
-  static_assert(kRunSlab == 8, "four int4 stores per slab");
-  slab[0] = make_int4(own.x, own.y, r[0].x, r[0].y);
-  slab[1] = make_int4(r[1].x, r[1].y, r[2].x, r[2].y);
-  slab[2] = make_int4(r[3].x, r[3].y, r[4].x, r[4].y);
-  slab[3] = make_int4(r[5].x, r[5].y, (int32_t)m, 0);
+  int4 *slab = reinterpret_cast<int4 *>(d.slab + (int64_t)b * kSlabWords);
+  static_assert(kSlabWords == 16 && kSlabRuns == 12, "four int4 stores per slab");
+  slab[0] = make_int4(start[0], start[1], start[2], start[3]);
+  slab[1] = make_int4(start[4], start[5], start[6], start[7]);
+  slab[2] = make_int4(start[8], start[9], start[10], start[11]);
+  auto four = [&](int i) {
+    return (int32_t)(len[i] | len[i + 1] << 8 | len[i + 2] << 16 | len[i + 3] << 24);
+  };
+  slab[3] = make_int4(four(0), four(4), four(8),
+                      over ? kSlabOver : runs | own_at << 8 | __popc(m >> 14) << 16);
 }
 
 // Grid-stride over the sorted positions: a capped grid keeps the launch
@@ -874,6 +867,12 @@ static inline unsigned degsum_blocks(int64_t nb) {
 // checks the capacity, commits the list length and restarts the
 // displacement bookkeeping (InteractionManager::ZeroDrTot -> Mesh/Object::
 // ZeroDrTot, src/interaction_manager.cpp:316-321, src/mesh.cpp:546-551).
+// k_deg leaves the runs in that order, so the pass copies them with their
+// first members loaded ahead.  When it walked the stencil itself, each cell a
+// branch and a load that waited, it was half the time on vector instructions
+// and half on loads, active: uneven 1.6M bonds 139 us, dense 620k 56; now 108
+// and 38, and k_deg 4 more.  Eight wavefronts a SIMD: 124 and 39 with the six
+// that 74 registers allow.
 // Where a failed list pass reports to: Ctl's own words, or, while blocks of
 // the same launch may still read those, words that reach Ctl at its end.
 struct Failure {
@@ -887,11 +886,10 @@ __device__ __forceinline__ Failure ctl_failure(const Dev &d) {
 __device__ __forceinline__ void pull_one(const Dev &d, const Geo &g, int32_t b,
                                          int32_t w, int32_t wend, int2 *stage,
                                          int32_t base, const Failure &fail) {
-  const int32_t k = d.keys[b];
   const Excl x = excl_of(d, g, b);
   const int32_t tag = (b & 63) << 2;
   auto put = [&](int32_t a, int role) {
-    if (a == x.lo || a == x.hi) return;
+    if (a == b || a == x.lo || a == x.hi) return;
     if (w < wend) {
       if (stage)
         stage[w - base] = make_int2(a, role | tag);
@@ -900,57 +898,55 @@ __device__ __forceinline__ void pull_one(const Dev &d, const Geo &g, int32_t b,
     }
     ++w;
   };
-  const int n = g.n1d;
-  const int cx = k / (n * n), cy = (k / n) % n, cz = k % n;
-  const int cls = (cx == 0 ? 0 : cx == n - 1 ? 2 : 1) * 6 +
-                  (cy == 0 ? 0 : cy == n - 1 ? 2 : 1) * 2 + (cz == 0 ? 0 : 1);
-  // the runs k_deg kept: own cell first, then the occupied stencil cells
-  // in bit order, and the occupancy mask of the 26 stencil cells; a run
-  // beyond the slab is looked up in the cell list
-  const int4 *sl = reinterpret_cast<const int4 *>(d.nrun + (int64_t)b * kRunSlab);
-  static_assert(kRunSlab == 8, "four int4 loads per slab");
+  const int4 *sl = reinterpret_cast<const int4 *>(d.slab + (int64_t)b * kSlabWords);
   const int4 s0 = sl[0], s1 = sl[1], s2 = sl[2], s3 = sl[3];
-  const int2 own = make_int2(s0.x, s0.y);
-  const uint32_t m = (uint32_t)s3.z;
-  auto run_of = [&](int q) -> int2 {
-    const int idx = 1 + __popc(m & ((1u << q) - 1u));
-    switch (idx) {
-      case 1: return make_int2(s0.z, s0.w);
-      case 2: return make_int2(s1.x, s1.y);
-      case 3: return make_int2(s1.z, s1.w);
-      case 4: return make_int2(s2.x, s2.y);
-      case 5: return make_int2(s2.z, s2.w);
-      case 6: return make_int2(s3.x, s3.y);
-      default: break;
-    }
-    int x, y, z;
-    if (q < 13)
-      shell_cell<false>(n, cx, cy, cz, q, &x, &y, &z);
-    else
-      shell_cell<true>(n, cx, cy, cz, q - 13, &x, &y, &z);
-    return cell_run_of(d, g, x, y, z);
-  };
-  uint64_t order = g.home_order[cls];
-  for (int step = 0; step < 14; ++step, order >>= 4) {
-    const int c = (int)(order & 15);
-    if (c == 13) {
-      // own cell (members in bond order): self pairs, then the rows of the
-      // half-shell blocks
-      // (a cell of one member holds b alone: no load needed)
-      int32_t r = own.x;
-      if (own.y - own.x > 1)
-        while (r < own.y && d.sorted[r] != b) ++r;
-      for (int32_t j = own.x; j < r; ++j) put(d.sorted[j], 1);
-      for (int32_t j = r + 1; j < own.y; ++j) put(d.sorted[j], 0);
-      for (uint32_t mm = m & 0x1fffu; mm; mm &= mm - 1) {
-        const int q = __ffs(mm) - 1;
-        const int2 rn = run_of(q);
-        for (int32_t j = rn.x; j < rn.y; ++j) put(d.sorted[j], 0);
+  if (s3.w != kSlabOver) {
+    const int32_t start[kSlabRuns] = {s0.x, s0.y, s0.z, s0.w, s1.x, s1.y,
+                                      s1.z, s1.w, s2.x, s2.y, s2.z, s2.w};
+    const uint32_t len[3] = {(uint32_t)s3.x, (uint32_t)s3.y, (uint32_t)s3.z};
+    const int runs = s3.w & 255, own = (s3.w >> 8) & 255, half = s3.w >> 16;
+    // the first member of every run (mostly its only one), in flight together
+    int32_t first[kSlabRuns];
+#pragma unroll
+    for (int i = 0; i < kSlabRuns; ++i)
+      if (i < runs) first[i] = d.sorted[start[i]];
+#pragma unroll
+    for (int i = 0; i < kSlabRuns; ++i) {
+      if (i < runs) {
+        // own cell: obj2 of the pairs with earlier members, obj1 of those
+        // with later ones; half shell: obj1; mirrored half shell: obj2
+        const int32_t pivot = i == own ? b : i > own && i <= own + half ? INT32_MIN : INT32_MAX;
+        put(first[i], first[i] < pivot);
+        const int l = (int)((len[i / 4] >> (8 * (i % 4))) & 255u);
+        for (int j = 1; j < l; ++j) {
+          const int32_t a = d.sorted[start[i] + j];
+          put(a, a < pivot);
+        }
       }
-    } else if ((m >> (13 + c)) & 1u) {
-      // mirrored half-shell cell c: b is obj2 of each of its members
-      const int2 rn = run_of(13 + c);
-      for (int32_t j = rn.x; j < rn.y; ++j) put(d.sorted[j], 1);
+    }
+  } else {
+    const int32_t k = d.keys[b];
+    const int n = g.n1d;
+    const int cx = k / (n * n), cy = (k / n) % n, cz = k % n;
+    const uint32_t m = stencil_mask(d, g, cx, cy, cz);
+    auto walk = [&](int code, int32_t pivot) {
+      int x, y, z;
+      stencil_cell(n, cx, cy, cz, code, &x, &y, &z);
+      const int2 r = cell_run_of(d, g, x, y, z);
+      for (int32_t j = r.x; j < r.y; ++j) {
+        const int32_t a = d.sorted[j];
+        put(a, a < pivot);
+      }
+    };
+    uint64_t order = home_order_of(g, cx, cy, cz);
+    for (int step = 0; step < 14; ++step, order >>= 4) {
+      const int c = (int)(order & 15);
+      if (c == 13) {
+        walk(kOwnCell, b);
+        for (uint32_t h = m >> 14; h; h &= h - 1) walk(13 + __ffs(h), INT32_MIN);
+      } else if ((m >> (12 - c)) & 1u) {
+        walk(12 - c, INT32_MAX);
+      }
     }
   }
   if (w != wend) {  // degree and list disagree: never expected; fail the step
@@ -1043,7 +1039,7 @@ __device__ __forceinline__ void pull_body(const Dev &d, const Geo &g, int64_t bi
   }
 }
 
-__global__ __launch_bounds__(256) void k_pull(Dev d, Geo g) {
+__global__ __launch_bounds__(256, 8) void k_pull(Dev d, Geo g) {
   if (guard_off(d.ctl, kGuardRebuild)) return;
   __shared__ PullLds<256> L;
   pull_body<256>(d, g, blockIdx.x, gridDim.x, ctl_failure(d), L);

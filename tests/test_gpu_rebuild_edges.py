@@ -6,6 +6,7 @@ import numpy as np
 import pytest
 
 import simcore_amd as sc
+from oracle.oracle_py import OracleSystem
 from tests.scenarios import make_filaments
 
 pytestmark = pytest.mark.gpu
@@ -114,6 +115,37 @@ def test_lists_of_one_and_several_launches(nb):
         want = _cell_pairs(s.cell_keys().astype(np.int64), n1d, np.asarray(fil.site_off))
         np.testing.assert_array_equal(code, want)
     assert s.counters()["n_rebuilds"] > 1
+    s.close()
+
+
+# cells around a bond: few, about the 12 that a bond's slab of runs holds, all
+# 27; `clump` bonds more in one cell, about the 255 that a slab's length holds
+@pytest.mark.parametrize("n1d, nb, clump", [(12, 300, 0), (12, 700, 0), (12, 1100, 0), (3, 600, 0),
+                                            (12, 400, 252), (12, 400, 254), (12, 400, 256),
+                                            (5, 800, 400)])
+def test_lists_at_the_edges_of_a_slab(n1d, nb, clump):
+    rng = np.random.default_rng(100 * n1d + nb + clump)
+    p = sc.params_init(float(n1d), delta=1e-4, min_cell_length=2.0, seed=11)
+    bonds = [rng.uniform(-n1d, n1d, 3) for _ in range(nb // 2)]  # two bonds each, straight
+    bonds += [1.0 + rng.uniform(-0.3, 0.3, 3) - n1d % 2 for _ in range(clump // 2)]
+    u = rng.normal(size=(len(bonds), 3))
+    u /= np.linalg.norm(u, axis=1)[:, None]
+    step = np.where(np.arange(len(bonds)) < nb // 2, 1.0, 0.1)
+    sites = [c + np.arange(-1, 2)[:, None] * w * s for c, w, s in zip(bonds, u, step)]
+    fil = make_filaments(sites)
+    s = sc.FilamentSystem(p, fil, precision="fp64")
+    a, b = s.candidates()
+    code = np.sort(np.minimum(a, b).astype(np.int64) * fil.nb + np.maximum(a, b))
+    keys = s.cell_keys().astype(np.int64)
+    if clump:
+        assert np.bincount(keys).max() >= clump - 2
+    np.testing.assert_array_equal(code, _cell_pairs(keys, n1d, np.asarray(fil.site_off)))
+    # the order of each list, by the sums it gives
+    ora = OracleSystem(p, fil)
+    s.step(2)
+    assert ora.step(2) == 0
+    for x, y in zip(s.bond_forces(), ora.bond_forces()):
+        np.testing.assert_array_equal(x, y)
     s.close()
 
 
