@@ -235,7 +235,7 @@ int sc_checkpoint_load(sc_handle h, const void *buf, size_t size);
  * any result except integrate_layout, which changes the rounding of the
  * mixed-precision integrator.
  *   pair_block          pair kernel threads per block, 64/128/256/512; 0
- *                       selects the load-balanced variant (one wave per 64
+ *                       selects the load-balanced variant (one wave per 16-64
  *                       bonds, incidences dealt evenly over its lanes), the
  *                       one a new handle uses
  *   pair_xcd            1: consecutive bond ranges on one XCD

@@ -635,9 +635,9 @@ void to_caller(const sc_system *h, const std::vector<int64_t> &map, const T *src
     for (int64_t i = 0; i < n; ++i) dst[k * n + map[i]] = src[k * n + i];
 }
 
-// Blocks of the pair pass at its smallest block size (64 bonds): each owns
+// Blocks of the pair pass at its smallest block size: each owns
 // one stress slot, whatever launch shape is set while the sum accumulates.
-int64_t stress_slots(int64_t nb) { return nb / 64 + 2; }
+int64_t stress_slots(int64_t nb) { return nb / sc::pair_bonds(nb, true) + 2; }
 
 // Scratch between steps: the rebuild's run slabs (64 bytes per bond), which only the launches between the degree and the list pass of one
 // rebuild use.  Every filament has at least two bonds, so it holds three
@@ -2180,7 +2180,7 @@ int sc_autotune(sc_handle h, int32_t steps, sc_tune_report *report) {
     }
   };
   // pair kernel: per-bond with 128/256/512 threads per block, or the
-  // balanced one-wave-per-64-bonds variant (block size not used)
+  // balanced one-wave-per-16-to-64-bonds variant (block size not used)
   const int blocks[] = {128, 256, 512, 0};
   for (int bs : blocks)
     for (int x = 0; x < 2; ++x) {

@@ -324,7 +324,7 @@ void launch_cells_from_keys(const Dev &d, const Geo &g, hipStream_t st);
 // `thermo`: also sum the pair stress and the bond energies (Geo::thermo)
 void launch_pair(const Dev &d, const Geo &g, int precision, const Tune &t,
                  hipStream_t st, bool thermo);
-int64_t pair_blocks(const Geo &g, const Tune &t);
+int pair_bonds(int64_t nb, bool thermo);
 void launch_pair_range(const Dev &d, const Geo &g, int precision, const Tune &t, hipStream_t st,
                        bool thermo, int64_t b_lo, int64_t b_hi);  // blocks of one pair launch
 // `mid`: the step is a midstep (odd step index)

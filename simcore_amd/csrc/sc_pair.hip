@@ -405,7 +405,7 @@ __global__ __launch_bounds__(512) void k_pair_fused(Dev d, Geo g, int xcd, int64
   if (THERMO) block_stress(d, S);
 }
 
-// Load-balanced variant: one wavefront per 64 bonds.  A bond's candidate
+// Load-balanced variant: one wavefront per G bonds (pair_bonds).  A bond's candidate
 // count varies (0 to ~10), and in the per-bond kernel a wave runs as long
 // as its busiest lane.  Here the wave's incidences (contiguous in the CSR)
 // are dealt out to the lanes in chunks of kChunk: each lane evaluates its
@@ -417,21 +417,21 @@ __global__ __launch_bounds__(512) void k_pair_fused(Dev d, Geo g, int xcd, int64
 // path's force shares are FP32 values and are staged as such.
 constexpr int kChunk = 128;
 
-template <bool MIXED, bool THERMO>
+template <bool MIXED, bool THERMO, int G>
 __device__ __forceinline__ void pair_bal_body(const Dev &d, const Geo &g, int64_t blk) {
   using FT = typename std::conditional<MIXED, float, double>::type;
-  __shared__ BondRec ownr[64];
+  __shared__ BondRec ownr[G];
   __shared__ FT cF[kChunk][3];
   __shared__ double cT[kChunk][3], cE[THERMO ? kChunk : 1];
-  __shared__ int32_t qs[65];
+  __shared__ int32_t qs[G + 1];
   if (d.ctl->abort) return;
   const int64_t nb = g.nb;
   const int lane = threadIdx.x;
-  const int64_t b0 = blk * 64;
+  const int64_t b0 = blk * G;
   const int64_t b = b0 + lane;
-  const bool valid = b < nb;
-  qs[lane] = d.inc_start[valid ? b : nb];
-  if (lane == 0) qs[64] = d.inc_start[b0 + 64 <= nb ? b0 + 64 : nb];
+  const bool valid = (G == 64 || lane < G) && b < nb;
+  if (lane <= G) qs[lane] = d.inc_start[b < nb ? b : nb];
+  if (G == 64 && lane == 0) qs[G] = d.inc_start[b0 + G <= nb ? b0 + G : nb];
   if (valid) ownr[lane] = load_rec<MIXED>(d.br, g, b);
   double F[3] = {0.0, 0.0, 0.0}, T[3] = {0.0, 0.0, 0.0}, E = 0.0;
   double S[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
@@ -446,14 +446,14 @@ __device__ __forceinline__ void pair_bal_body(const Dev &d, const Geo &g, int64_
     }
   }
   __syncthreads();
-  const int32_t Q0 = qs[0], Q1 = qs[64];
-  const int32_t my0 = qs[lane], my1 = qs[lane + 1];
+  const int32_t Q0 = qs[0], Q1 = qs[G];
+  const int32_t my0 = lane < G ? qs[lane] : Q1, my1 = lane < G ? qs[lane + 1] : Q1;
   for (int32_t cs = Q0; cs < Q1; cs += kChunk) {
     const int32_t ce = Q1 < cs + kChunk ? Q1 : cs + kChunk;
     for (int32_t q = cs + lane; q < ce; q += 64) {
       const int2 ent = d.inc[q];
       const BondRec oth = load_rec<MIXED>(d.br, g, ent.x);
-      const BondRec own = ownr[(ent.y >> 2) & 63];
+      const BondRec own = ownr[(ent.y >> 2) & (G - 1)];
       double fc[3], sc, rs, cf[3], ct[3];
       pair_slot<MIXED>(d, g, own, q, ent, oth, fc, &sc, &rs);
       const double sg = (ent.y & 1) ? -1.0 : 1.0;
@@ -484,25 +484,38 @@ __device__ __forceinline__ void pair_bal_body(const Dev &d, const Geo &g, int64_
   }
 }
 
-template <bool MIXED, bool THERMO>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5))) void k_pair_bal(Dev d, Geo g, int xcd,
-                                                                                           int64_t blk0) {
-  pair_bal_body<MIXED, THERMO>(d, g, blk0 + logical_block(xcd));
+template <bool MIXED, bool THERMO, int G>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(G == 64 ? 5 : 4)))
+void k_pair_bal(Dev d, Geo g, int xcd, int64_t blk0) {
+  pair_bal_body<MIXED, THERMO, G>(d, g, blk0 + logical_block(xcd));
 }
 
 // Ensemble batches: the balanced kernel over every member's bonds (mixed
 // precision, no stress sums); `par` 0 on odd steps, 1 on even ones.
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5))) void k_group_pair(
+template <int G>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(G == 64 ? 5 : 4)))
+void k_group_pair(
     const Member *__restrict__ ms, GroupGrid gg, int par) {
   int b0, nblk;
   const Member &M = ms[group_member(gg, blockIdx.x, &b0, &nblk)];
-  pair_bal_body<true, false>(M.d[par], M.g, blockIdx.x - b0);
+  pair_bal_body<true, false, G>(M.d[par], M.g, blockIdx.x - b0);
 }
 
-int64_t pair_blocks(const Geo &g, const Tune &t) {
-  const int bs = t.pair_bal ? 64 : t.pair_block;
-  const int64_t blocks = (g.nb + bs - 1) / bs;
-  return blocks > 0 ? blocks : 1;
+// Bonds of a wavefront of the balanced kernel.  A wavefront takes its bonds'
+// incidences (2 to 3 a bond) 64 at a time, each round a chain of loads and a
+// pair geometry, so with few bonds on the chip the pass lasts as long as one
+// wavefront's rounds: 16 bonds need one, 64 need two to four.  Once the chip
+// is full the owners' part, which 16 bonds leave to 16 lanes, counts instead.
+// us a step with 16 / 32 / 64 bonds, mixed: 1k bonds 17.8 / 19.1 / 21.4, 10k
+// 20.9 / 21.5 / 24.0, 31k 23.9 / 24.6 / 26.3, 62k 27.6 / 27.9 / 28.8, 102k
+// 35.4 / 33.0 / 34.1, 155k 43.1 / 41.3 / 41.6, 400k 90.1 / 81.8 / 80.1; FP64:
+// 1k 26.8 / 27.5 / 30.3, 31k 33.8 / 34.8 / 36.5, 62k 38.1 / 38.0 / 40.6, 102k
+// 46.7 / 45.5 / 47.5.  Stress sums add 36 shuffles a wavefront and a slot
+// each, hence 32 bonds at least: 62k bonds, 49 steps and the sums read, 1756 /
+// 1649 / 1745 us.
+int pair_bonds(int64_t nb, bool thermo) {
+  if (nb > 131072) return 64;
+  return nb > 65536 || thermo ? 32 : 16;
 }
 
 void launch_pair(const Dev &d, const Geo &g, int precision, const Tune &t, hipStream_t st,
@@ -514,7 +527,8 @@ void launch_pair(const Dev &d, const Geo &g, int precision, const Tune &t, hipSt
 // it is the last bond.
 void launch_pair_range(const Dev &d, const Geo &g, int precision, const Tune &t, hipStream_t st,
                        bool thermo, int64_t b_lo, int64_t b_hi) {
-  const int bs = t.pair_bal ? 64 : t.pair_block;
+  const int bal = pair_bonds(g.nb, thermo);
+  const int bs = t.pair_bal ? bal : t.pair_block;
   const int64_t blk0 = b_lo / bs;
   const int64_t nblk = (b_hi - b_lo + bs - 1) / bs;
   if (nblk <= 0) return;
@@ -531,23 +545,46 @@ void launch_pair_range(const Dev &d, const Geo &g, int precision, const Tune &t,
     else                                                                                       \
       hipLaunchKernelGGL((KERNEL<true, false>), grid, dim3(BS), 0, st, d, g, t.pair_xcd, blk0); \
   } while (0)
-  if (t.pair_bal)
-    SC_PAIR(k_pair_bal, 64);
-  else
+  if (!t.pair_bal)
     SC_PAIR(k_pair_fused, t.pair_block);
 #undef SC_PAIR
+#define SC_BAL(G)                                                                              \
+  do {                                                                                         \
+    if (bal == G && fp64 && thermo)                                                            \
+      hipLaunchKernelGGL((k_pair_bal<false, true, G>), grid, dim3(64), 0, st, d, g, t.pair_xcd, blk0); \
+    else if (bal == G && fp64)                                                                 \
+      hipLaunchKernelGGL((k_pair_bal<false, false, G>), grid, dim3(64), 0, st, d, g, t.pair_xcd, blk0); \
+    else if (bal == G && thermo)                                                               \
+      hipLaunchKernelGGL((k_pair_bal<true, true, G>), grid, dim3(64), 0, st, d, g, t.pair_xcd, blk0); \
+    else if (bal == G)                                                                         \
+      hipLaunchKernelGGL((k_pair_bal<true, false, G>), grid, dim3(64), 0, st, d, g, t.pair_xcd, blk0); \
+  } while (0)
+  if (t.pair_bal) {
+    SC_BAL(16);
+    SC_BAL(32);
+    SC_BAL(64);
+  }
+#undef SC_BAL
 }
 
 void launch_group_pair(const Member *dm, const Member *hm, int n, bool odd, hipStream_t st) {
   GroupGrid gg;
   int32_t t = 0;
+  int64_t nb = 0;
+  for (int m = 0; m < n; ++m) nb += hm[m].g.nb;
+  const int bal = pair_bonds(nb, false);
   for (int m = 0; m < n; ++m) {
     gg.off[m] = t;
-    t += (int32_t)((hm[m].g.nb + 63) / 64);
+    t += (int32_t)((hm[m].g.nb + bal - 1) / bal);
   }
   for (int m = n; m <= kMaxGroup; ++m) gg.off[m] = t;
   if (t <= 0) return;
-  hipLaunchKernelGGL(k_group_pair, dim3((unsigned)t), dim3(64), 0, st, dm, gg, odd ? 0 : 1);
+  if (bal == 16)
+    hipLaunchKernelGGL(k_group_pair<16>, dim3((unsigned)t), dim3(64), 0, st, dm, gg, odd ? 0 : 1);
+  else if (bal == 32)
+    hipLaunchKernelGGL(k_group_pair<32>, dim3((unsigned)t), dim3(64), 0, st, dm, gg, odd ? 0 : 1);
+  else
+    hipLaunchKernelGGL(k_group_pair<64>, dim3((unsigned)t), dim3(64), 0, st, dm, gg, odd ? 0 : 1);
 }
 
 }  // namespace sc
