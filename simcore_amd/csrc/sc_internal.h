@@ -87,7 +87,7 @@ constexpr int kDrSlots = 256;
 
 // Counters of the launches that run several passes (sc_block.h), zero between
 // launches; one cache line per counter that several blocks add to.
-constexpr int kBars = 6, kBarGroups = 16;
+constexpr int kBars = 5, kBarGroups = 16;
 struct Door {
   uint32_t arrived, parts, gone;
   int32_t abort, err, overflow;  // for Ctl, when the launch ends

@@ -294,17 +294,18 @@ constexpr int kColScanBlock = 1024;
 constexpr int kColScanTile = 4 * kColScanBlock;
 constexpr int64_t kColScanMax = (int64_t)1 << 17;
 
-// (kColScanBlock threads)
+// (BLOCK threads, a tile of 4 * BLOCK columns)
+template <int BLOCK>
 __device__ __forceinline__ void colscan_body(const Dev &d, int64_t ncol, int64_t tile) {
-  __shared__ int ws[kColScanBlock / 64];
-  const int64_t base = tile * kColScanTile;
+  __shared__ int ws[BLOCK / 64];
+  const int64_t base = tile * 4 * BLOCK;
   const int4 *in4 = reinterpret_cast<const int4 *>(d.col_count);
   int part = 0;
-  for (int64_t i = threadIdx.x; i < base / 4; i += kColScanBlock) {
+  for (int64_t i = threadIdx.x; i < base / 4; i += BLOCK) {
     const int4 v = in4[i];
     part += v.x + v.y + v.z + v.w;
   }
-  const int carry = block_sum<kColScanBlock>(part, ws);
+  const int carry = block_sum<BLOCK>(part, ws);
   const int64_t i0 = base + 4 * (int64_t)threadIdx.x;
   int v[4], s = 0;
 #pragma unroll
@@ -313,18 +314,18 @@ __device__ __forceinline__ void colscan_body(const Dev &d, int64_t ncol, int64_t
     s += v[k];
   }
   int tot;
-  int ex = carry + block_excl<kColScanBlock>(s, &tot, ws);
+  int ex = carry + block_excl<BLOCK>(s, &tot, ws);
 #pragma unroll
   for (int k = 0; k < 4; ++k) {
     if (i0 + k < ncol) d.col_start[i0 + k] = ex;
     ex += v[k];
   }
-  if (base + kColScanTile >= ncol && threadIdx.x == 0) d.col_start[ncol] = carry + tot;
+  if (base + 4 * BLOCK >= ncol && threadIdx.x == 0) d.col_start[ncol] = carry + tot;
 }
 
 __global__ __launch_bounds__(kColScanBlock) void k_colscan(Dev d, int64_t ncol, int guard) {
   if (guard_off(d.ctl, guard)) return;
-  colscan_body(d, ncol, blockIdx.x);
+  colscan_body<kColScanBlock>(d, ncol, blockIdx.x);
 }
 
 static inline unsigned colscan_tiles(int64_t ncol) {
@@ -365,8 +366,8 @@ template <int BLOCK>
 __device__ __forceinline__ void keys_body(const Dev &d, const Geo &g, int64_t bid, int64_t nblk,
                                           KeysLds<BLOCK> &L) {
   int32_t *hcol = L.col, *hcnt = L.cnt, *hbase = L.base;
-  constexpr int kHashShift = BLOCK == 1024 ? 22 : 24;  // hash bits: log2(BLOCK)
-  static_assert(BLOCK == 256 || BLOCK == 1024, "hash bits");
+  constexpr int kHashShift = BLOCK == 1024 ? 22 : BLOCK == 512 ? 23 : 24;  // hash bits: log2(BLOCK)
+  static_assert(BLOCK == 256 || BLOCK == 512 || BLOCK == 1024, "hash bits");
   const int t = threadIdx.x;
   const int64_t ntiles = (g.nb + BLOCK - 1) / BLOCK;
   for (int64_t tile = bid; tile < ntiles; tile += nblk) {
@@ -808,12 +809,9 @@ __device__ __forceinline__ int64_t n_supers(int64_t nb) {
   return (nb + kPullGroup * kSuper - 1) / (kPullGroup * kSuper);
 }
 
-// (each 256 threads of a block take a block of groups)
-template <int BLOCK>
-__device__ __forceinline__ void degsum_body(const Dev &d, const Geo &g, int64_t bid) {
-  __shared__ int ws[BLOCK / 64];
-  const int lane = threadIdx.x & 63, wv = (threadIdx.x >> 6) & 3;
-  const int64_t sup = bid * (BLOCK / 256) + threadIdx.x / 256;
+__device__ __forceinline__ void degsum_body(const Dev &d, const Geo &g, int64_t sup) {
+  __shared__ int ws[4];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   int32_t *gsum = d.scan_tmp + n_supers(g.nb);
   const int64_t ngrp = n_groups(g.nb);
   int all = 0;
@@ -830,18 +828,14 @@ __device__ __forceinline__ void degsum_body(const Dev &d, const Geo &g, int64_t 
     if (lane == 0 && grp < ngrp) gsum[grp] = s;
     all += s;
   }
-  if (lane == 0) ws[threadIdx.x >> 6] = all;
+  if (lane == 0) ws[wv] = all;
   __syncthreads();
-  if (threadIdx.x % 256 == 0 && sup < n_supers(g.nb)) {
-    const int w = threadIdx.x >> 6;
-    d.scan_tmp[sup] = ws[w] + ws[w + 1] + ws[w + 2] + ws[w + 3];
-  }
-  __syncthreads();
+  if (threadIdx.x == 0) d.scan_tmp[sup] = ws[0] + ws[1] + ws[2] + ws[3];
 }
 
 __global__ __launch_bounds__(256) void k_degsum(Dev d, Geo g) {
   if (guard_off(d.ctl, kGuardRebuild)) return;
-  degsum_body<256>(d, g, blockIdx.x);
+  degsum_body(d, g, blockIdx.x);
 }
 
 static inline unsigned degsum_blocks(int64_t nb) {
@@ -968,7 +962,7 @@ struct PullLds {
   int ws[BLOCK / 64];
 };
 
-template <int BLOCK>
+template <int BLOCK, bool SUMS>
 __device__ __forceinline__ void pull_body(const Dev &d, const Geo &g, int64_t bid, int64_t nblk,
                                           const Failure &fail, PullLds<BLOCK> &L) {
   static_assert(kPullGroup == 256, "one bond per thread");
@@ -981,7 +975,21 @@ __device__ __forceinline__ void pull_body(const Dev &d, const Geo &g, int64_t bi
   const int64_t stride = nblk * BLOCK;
   const int64_t ngrp = n_groups(g.nb), nsup = n_supers(g.nb);
   int64_t part = 0;
-  for (int64_t i = threadIdx.x; i < nsup; i += BLOCK) part += d.scan_tmp[i];
+  int32_t before = 0;  // (of no use unless the total fits)
+  if (SUMS) {
+    for (int64_t i = threadIdx.x; i < nsup; i += BLOCK) part += d.scan_tmp[i];
+  } else {
+    const int4 *deg4 = reinterpret_cast<const int4 *>(d.deg);
+    const int64_t first = bid * BLOCK / 4, n4 = g.nb / 4;
+    for (int64_t i = threadIdx.x; i < n4; i += BLOCK) {
+      const int4 v = deg4[i];
+      const int64_t four = (int64_t)v.x + v.y + v.z + v.w;
+      part += four;
+      if (i < first) before += (int32_t)four;
+    }
+    // (the last one to three bonds come before no block's first)
+    if (4 * n4 + threadIdx.x < g.nb) part += d.deg[4 * n4 + threadIdx.x];
+  }
   for (int o = 32; o > 0; o >>= 1) part += __shfl_xor(part, o, 64);
   if (lane == 0) red[wv] = part;
   __syncthreads();
@@ -1007,17 +1015,32 @@ __device__ __forceinline__ void pull_body(const Dev &d, const Geo &g, int64_t bi
   }
   // the incidence starts of the block's groups, before the walk over them (in
   // one loop with it they cost the walk 22 registers, two waves per SIMD)
-  for (int grp0 = (int)bid * kSubs; grp0 < (int)ngrp; grp0 += (int)nblk * kSubs) {
-    const int grp = grp0 + sub;
-    const int64_t b = (int64_t)grp * kPullGroup + t;
-    const int sup = grp / kSuper;
-    int32_t before =
-        sup * kSuper + t < grp && grp < (int)ngrp ? d.scan_tmp[nsup + sup * kSuper + t] : 0;
-    for (int i = t; i < sup; i += 256) before += d.scan_tmp[i];
-    const int32_t base = block_sum<256>(before, ws);
-    int gtot;
-    const int32_t w = base + block_excl<256>(b < g.nb ? d.deg[b] : 0, &gtot, ws);
-    if (b < g.nb) d.inc_start[b] = w;  // read back by the same thread below
+  if (SUMS) {
+    for (int grp0 = (int)bid * kSubs; grp0 < (int)ngrp; grp0 += (int)nblk * kSubs) {
+      const int grp = grp0 + sub;
+      const int64_t b = (int64_t)grp * kPullGroup + t;
+      const int sup = grp / kSuper;
+      int32_t ahead =
+          sup * kSuper + t < grp && grp < (int)ngrp ? d.scan_tmp[nsup + sup * kSuper + t] : 0;
+      for (int i = t; i < sup; i += 256) ahead += d.scan_tmp[i];
+      const int32_t base = block_sum<256>(ahead, ws);
+      int gtot;
+      const int32_t w = base + block_excl<256>(b < g.nb ? d.deg[b] : 0, &gtot, ws);
+      if (b < g.nb) d.inc_start[b] = w;  // read back by the same thread below
+    }
+  } else {
+    int32_t base = block_sum<BLOCK>(before, ws);
+    for (int64_t b0 = bid * BLOCK; b0 < g.nb; b0 += stride) {
+      const int64_t b = b0 + threadIdx.x;
+      int tot;
+      const int32_t w = base + block_excl<BLOCK>(b < g.nb ? d.deg[b] : 0, &tot, ws);
+      if (b < g.nb) d.inc_start[b] = w;
+      // (to the block's next bonds, if there are any)
+      int32_t skip = 0;
+      if (b0 + stride < g.nb)
+        for (int64_t i = b + BLOCK; i < b0 + stride; i += BLOCK) skip += d.deg[i];
+      base += tot + block_sum<BLOCK>(skip, ws);
+    }
   }
   // each wavefront's 64 consecutive bonds have one contiguous list range:
   // written to LDS entry by entry, then copied out in coalesced stores
@@ -1042,31 +1065,42 @@ __device__ __forceinline__ void pull_body(const Dev &d, const Geo &g, int64_t bi
 __global__ __launch_bounds__(256, 8) void k_pull(Dev d, Geo g) {
   if (guard_off(d.ctl, kGuardRebuild)) return;
   __shared__ PullLds<256> L;
-  pull_body<256>(d, g, blockIdx.x, gridDim.x, ctl_failure(d), L);
+  pull_body<256, true>(d, g, blockIdx.x, gridDim.x, ctl_failure(d), L);
 }
 
 // ---- the rebuild stage in one launch ----------------------------------------
 // Every launch costs 1.55 us also on a step that does not rebuild, so up to
-// kOneLaunchBonds one launch runs the seven passes, with a barrier between
-// them among its blocks (sc_block.h): 3.5 us among 64 blocks, 7 among 256,
-// against 1.55 us for a kernel boundary; hence few, large blocks, and the
-// launches for larger systems, whose passes want more of them.  us a step,
-// seven launches against one: 1k bonds 25.7 / 22.4, FP64 1.2k 31.4 / 27.3, 52k 31.9 / 29.6, 62k with
-// stress sums 34.2 / 31.6, 101k 36.4 / 32.9; FP64 155k 55.3 / 56.0, so the
-// line is drawn at 128k.
-constexpr int kOneBlock = 1024;
+// kOneLaunchBonds one launch runs the passes, with a barrier between them
+// among its blocks (sc_block.h): 3.5 us among 64 blocks, 7 among 256, against
+// 1.55 us for a kernel boundary; hence few, large blocks, and the launches for
+// larger systems, whose passes want more of them.  us a step, seven launches
+// against one: 1k bonds 25.7 / 22.4, FP64 1.2k 31.4 / 27.3, 52k 31.9 / 29.6,
+// 62k with stress sums 34.2 / 31.6, 101k 36.4 / 32.9; FP64 155k 55.3 / 56.0,
+// so the line is drawn at 128k.
+//
+// The list pass adds up the degrees itself: with few bonds that is less than
+// the pass of group sums and its barrier, 11 us of a rebuild of 85 at 52k
+// bonds (27.5 -> 27.1 us a step, 62k with stress sums 29.2 -> 28.9).
 constexpr int64_t kOneLaunchBonds = 131072;
 
 static inline bool rebuild_in_one(const Geo &g) {
   return g.nb <= kOneLaunchBonds && (int64_t)g.n1d * g.n1d <= kColScanMax;
 }
 
+// Threads of a block: the gathers of the degree and list passes keep a CU's
+// load units busy, so small systems spread their bonds over more CUs with
+// blocks of 512 until the barriers cost more.  512 against 1024, us a step: 1k
+// bonds 18.2 / 18.6, 10k 20.1 / 20.5, 31k 23.2 / 23.5, 62k 28.0 / 27.5, 102k
+// 34.3 / 32.7.
+constexpr int64_t kSmallBonds = 40960;
+
 // Blocks of the one launch: enough for 800 bonds each (64 or 128 blocks where
-// they were the best of 16 to 256 at 52k and 101k bonds), and in small sparse
-// systems for 64 columns each, whose sort is the longest pass there.
-static inline unsigned one_blocks(const Geo &g) {
-  const int64_t ncol = (int64_t)g.n1d * g.n1d;
-  const int64_t b = std::max<int64_t>((g.nb + 799) / 800, std::min<int64_t>((ncol + 63) / 64, 64));
+// they were the best of 16 to 256 at 52k and 101k bonds), 400 in blocks of
+// 512, and in small sparse systems for 64 columns each, whose sort is the
+// longest pass there.
+static inline unsigned one_blocks(const Geo &g, int block) {
+  const int64_t ncol = (int64_t)g.n1d * g.n1d, per = block == 512 ? 400 : 800;
+  const int64_t b = std::max<int64_t>((g.nb + per - 1) / per, std::min<int64_t>((ncol + 63) / 64, 64));
   return (unsigned)std::min<int64_t>(std::max<int64_t>(b, 1), 128);
 }
 
@@ -1086,15 +1120,16 @@ __device__ __forceinline__ void rebuild_one_end(const Dev &d) {
 }
 
 // the passes' stages, one after the other in the same memory
+template <int BLOCK>
 union OneLds {
-  KeysLds<kOneBlock> keys;
-  ColsortLds<kOneBlock> col;
-  PullLds<kOneBlock> pull;
+  KeysLds<BLOCK> keys;
+  ColsortLds<BLOCK> col;
+  PullLds<BLOCK> pull;
 };
 
-template <bool FOLD>
+template <int BLOCK, bool FOLD>
 __device__ __forceinline__ void rebuild_one_body(const Dev &d, const Geo &g, uint32_t blocks,
-                                                 bool first, OneLds &L) {
+                                                 bool first, OneLds<BLOCK> &L) {
   if (FOLD) {
     if (!fold_commit(d, g.thr, first)) return;
   } else {
@@ -1104,20 +1139,19 @@ __device__ __forceinline__ void rebuild_one_body(const Dev &d, const Geo &g, uin
   int rank, parts;
   if (door_enter(door, blocks, &rank, &parts)) {
     const int64_t ncol = (int64_t)g.n1d * g.n1d;
-    keys_body<kOneBlock>(d, g, rank, parts, L.keys);
+    keys_body<BLOCK>(d, g, rank, parts, L.keys);
     bar_wait(door, 0, rank, parts);
-    for (int64_t t = rank; t * kColScanTile < ncol; t += parts) colscan_body(d, ncol, t);
+    for (int64_t t = rank; t * 4 * BLOCK < ncol; t += parts)
+      colscan_body<BLOCK>(d, ncol, t);
     bar_wait(door, 1, rank, parts);
     scatter_body(d, g, rank, parts);
     bar_wait(door, 2, rank, parts);
-    colsort_body<kOneBlock>(d, g, rank, parts, L.col);
+    colsort_body<BLOCK>(d, g, rank, parts, L.col);
     bar_wait(door, 3, rank, parts);
     deg_body(d, g, rank, parts);
     bar_wait(door, 4, rank, parts);
-    for (int64_t s = rank; s * (kOneBlock / 256) < n_supers(g.nb); s += parts)
-      degsum_body<kOneBlock>(d, g, s);
-    bar_wait(door, 5, rank, parts);
-    pull_body<kOneBlock>(d, g, rank, parts, {&door->abort, &door->err, &door->overflow}, L.pull);
+    const Failure fail = {&door->abort, &door->err, &door->overflow};
+    pull_body<BLOCK, false>(d, g, rank, parts, fail, L.pull);
   }
   if (door_leave(door, blocks)) {
     rebuild_one_end(d);
@@ -1125,10 +1159,10 @@ __device__ __forceinline__ void rebuild_one_body(const Dev &d, const Geo &g, uin
   }
 }
 
-template <bool FOLD>
-__global__ __launch_bounds__(kOneBlock) void k_rebuild_one(Dev d, Geo g) {
-  __shared__ OneLds L;
-  rebuild_one_body<FOLD>(d, g, gridDim.x, blockIdx.x == 0, L);
+template <int BLOCK, bool FOLD>
+__global__ __launch_bounds__(BLOCK) void k_rebuild_one(Dev d, Geo g) {
+  __shared__ OneLds<BLOCK> L;
+  rebuild_one_body<BLOCK, FOLD>(d, g, gridDim.x, blockIdx.x == 0, L);
 }
 
 static inline unsigned nblocks(int64_t n, int bs) {
@@ -1155,11 +1189,15 @@ void launch_rebuild(const Dev &d, const Geo &g, bool fold, hipStream_t st) {
   const unsigned gs = sgrid(g.nb);
   const int64_t ncol = (int64_t)g.n1d * g.n1d;
   if (rebuild_in_one(g)) {
-    const dim3 grid(one_blocks(g));
-    if (fold)
-      hipLaunchKernelGGL(k_rebuild_one<true>, grid, dim3(kOneBlock), 0, st, d, g);
+    const dim3 grid(one_blocks(g, g.nb <= kSmallBonds ? 512 : 1024));
+    if (g.nb <= kSmallBonds && fold)
+      hipLaunchKernelGGL((k_rebuild_one<512, true>), grid, dim3(512), 0, st, d, g);
+    else if (g.nb <= kSmallBonds)
+      hipLaunchKernelGGL((k_rebuild_one<512, false>), grid, dim3(512), 0, st, d, g);
+    else if (fold)
+      hipLaunchKernelGGL((k_rebuild_one<1024, true>), grid, dim3(1024), 0, st, d, g);
     else
-      hipLaunchKernelGGL(k_rebuild_one<false>, grid, dim3(kOneBlock), 0, st, d, g);
+      hipLaunchKernelGGL((k_rebuild_one<1024, false>), grid, dim3(1024), 0, st, d, g);
     return;
   }
   if (fold)
@@ -1224,7 +1262,7 @@ __global__ __launch_bounds__(256) void k_group_pull(const Member *__restrict__ m
   const Member &M = ms[group_member(gg, blockIdx.x, &b0, &nblk)];
   if (guard_off(M.d[0].ctl, kGuardRebuild)) return;
   __shared__ PullLds<256> L;
-  pull_body<256>(M.d[0], M.g, blockIdx.x - b0, nblk, ctl_failure(M.d[0]), L);
+  pull_body<256, true>(M.d[0], M.g, blockIdx.x - b0, nblk, ctl_failure(M.d[0]), L);
 }
 
 // the two-launch column scan, for batches with a member of more than
@@ -1253,7 +1291,7 @@ __global__ __launch_bounds__(kColScanBlock) void k_group_colscan(const Member *_
   int b0, nblk;
   const Member &M = ms[group_member(gg, blockIdx.x, &b0, &nblk)];
   if (guard_off(M.d[0].ctl, kGuardRebuild)) return;
-  colscan_body(M.d[0], (int64_t)M.g.n1d * M.g.n1d, blockIdx.x - b0);
+  colscan_body<kColScanBlock>(M.d[0], (int64_t)M.g.n1d * M.g.n1d, blockIdx.x - b0);
 }
 
 __global__ __launch_bounds__(256) void k_group_degsum(const Member *__restrict__ ms,
@@ -1261,16 +1299,16 @@ __global__ __launch_bounds__(256) void k_group_degsum(const Member *__restrict__
   int b0, nblk;
   const Member &M = ms[group_member(gg, blockIdx.x, &b0, &nblk)];
   if (guard_off(M.d[0].ctl, kGuardRebuild)) return;
-  degsum_body<256>(M.d[0], M.g, blockIdx.x - b0);
+  degsum_body(M.d[0], M.g, blockIdx.x - b0);
 }
 
-template <bool FOLD>
-__global__ __launch_bounds__(kOneBlock) void k_group_rebuild_one(const Member *__restrict__ ms,
+template <int BLOCK, bool FOLD>
+__global__ __launch_bounds__(BLOCK) void k_group_rebuild_one(const Member *__restrict__ ms,
                                                                  GroupGrid gg) {
-  __shared__ OneLds L;
+  __shared__ OneLds<BLOCK> L;
   int b0, nblk;
   const Member &M = ms[group_member(gg, blockIdx.x, &b0, &nblk)];
-  rebuild_one_body<FOLD>(M.d[0], M.g, nblk, (int)blockIdx.x == b0, L);
+  rebuild_one_body<BLOCK, FOLD>(M.d[0], M.g, nblk, (int)blockIdx.x == b0, L);
 }
 
 namespace {
@@ -1295,14 +1333,24 @@ unsigned scan_blocks(int64_t n) {
 void launch_group_rebuild(const Member *dm, const Member *hm, int n, bool fold, hipStream_t st) {
   if (n <= 0) return;
   bool one = true;
-  for (int m = 0; m < n; ++m) one = one && rebuild_in_one(hm[m].g);
+  bool small = true;
+  for (int m = 0; m < n; ++m) {
+    one = one && rebuild_in_one(hm[m].g);
+    small = small && hm[m].g.nb <= kSmallBonds;
+  }
   if (one) {
     GroupGrid go;
-    const int32_t to = group_grid(go, hm, n, [](const Geo &g) { return one_blocks(g); });
-    if (fold)
-      hipLaunchKernelGGL(k_group_rebuild_one<true>, dim3(to), dim3(kOneBlock), 0, st, dm, go);
+    const int32_t to = group_grid(go, hm, n, [small](const Geo &g) {
+      return one_blocks(g, small ? 512 : 1024);
+    });
+    if (small && fold)
+      hipLaunchKernelGGL((k_group_rebuild_one<512, true>), dim3(to), dim3(512), 0, st, dm, go);
+    else if (small)
+      hipLaunchKernelGGL((k_group_rebuild_one<512, false>), dim3(to), dim3(512), 0, st, dm, go);
+    else if (fold)
+      hipLaunchKernelGGL((k_group_rebuild_one<1024, true>), dim3(to), dim3(1024), 0, st, dm, go);
     else
-      hipLaunchKernelGGL(k_group_rebuild_one<false>, dim3(to), dim3(kOneBlock), 0, st, dm, go);
+      hipLaunchKernelGGL((k_group_rebuild_one<1024, false>), dim3(to), dim3(1024), 0, st, dm, go);
     return;
   }
   GroupGrid gk, gcs, gsrt, gdeg, gds, gpl;

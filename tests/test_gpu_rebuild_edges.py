@@ -87,9 +87,9 @@ def _cell_pairs(keys, n, site_off):
     return np.sort(np.concatenate(out))
 
 
-# 800 bonds a block of the one-launch rebuild, which serves 131072 bonds
-@pytest.mark.parametrize("nb", [799, 800, 801, 25599, 102401, 131071, 131072, 131073])
-def test_lists_of_one_and_several_launches(nb):
+def _spread(nb):
+    """(params, filaments, cells a side): straight filaments with nb bonds in
+    all, anywhere in the box."""
     rng = np.random.default_rng(nb)
     n1d = max(12, int(round((nb / 1.5) ** (1.0 / 3.0))))
     p = sc.params_init(float(n1d), delta=1e-4, min_cell_length=2.0, seed=11)
@@ -105,6 +105,14 @@ def test_lists_of_one_and_several_launches(nb):
     start = rng.uniform(-n1d, n1d, (len(lengths), 3))
     fil = make_filaments([start[f] + np.arange(n)[:, None] * u[f]
                           for f, n in enumerate(lengths)])
+    return p, fil, n1d
+
+
+# 400 and 800 bonds a block of the one-launch rebuild, which has blocks of 512
+# threads up to 40960 bonds and serves 131072
+@pytest.mark.parametrize("nb", [799, 800, 801, 25599, 40960, 40961, 102401, 131071, 131072, 131073])
+def test_lists_of_one_and_several_launches(nb):
+    p, fil, n1d = _spread(nb)
     assert fil.nb == nb
     s = sc.FilamentSystem(p, fil, precision="mixed", use_graph=True, spatial_order=True)
     assert s.counters()["n_cells_1d"] == n1d
@@ -147,6 +155,27 @@ def test_lists_at_the_edges_of_a_slab(n1d, nb, clump):
     for x, y in zip(s.bond_forces(), ora.bond_forces()):
         np.testing.assert_array_equal(x, y)
     s.close()
+
+
+def test_batch_of_more_blocks_than_fit():
+    """The one-launch rebuild of 24 members asks for more blocks than the chip
+    holds, so members start their passes with some of theirs."""
+    p, fil, _ = _spread(40000)
+    seeds = list(range(1, 25))
+    ens = sc.Ensemble(hbm_budget=16 << 30, max_active=24, steps_per_launch=16, batch_size=24)
+    ids = []
+    for k in seeds:
+        p.seed = k
+        ids.append(ens.submit(p, fil, 41, precision="mixed"))
+    ens.drain(60)
+    for k in (1, 9, 17, 24):
+        p.seed = k
+        s = sc.FilamentSystem(p, fil, precision="mixed", use_graph=True)
+        s.step(41)
+        assert s.counters()["n_rebuilds"] > 1
+        np.testing.assert_array_equal(ens.result(ids[k - 1]), s.sites()[0])
+        s.close()
+    ens.close()
 
 
 def test_batch_with_a_wide_member():
