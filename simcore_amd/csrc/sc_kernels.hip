@@ -1075,13 +1075,14 @@ __global__ __launch_bounds__(256, 8) void k_pull(Dev d, Geo g) {
 // 1.55 us for a kernel boundary; hence few, large blocks, and the launches for
 // larger systems, whose passes want more of them.  us a step, seven launches
 // against one: 1k bonds 25.7 / 22.4, FP64 1.2k 31.4 / 27.3, 52k 31.9 / 29.6,
-// 62k with stress sums 34.2 / 31.6, 101k 36.4 / 32.9; FP64 155k 55.3 / 56.0,
-// so the line is drawn at 128k.
+// 62k with stress sums 34.2 / 31.6, 155k 41.6 / 39.4, FP64 155k 55.4 / 53.6,
+// FP64 uneven 230k 92.4 / 89.0, 232k 47.5 / 47.3, 372k 60.9 / 66.4.  Up to 256k
+// bonds every thread of 256 blocks has one bond.
 //
 // The list pass adds up the degrees itself: with few bonds that is less than
 // the pass of group sums and its barrier, 11 us of a rebuild of 85 at 52k
 // bonds (27.5 -> 27.1 us a step, 62k with stress sums 29.2 -> 28.9).
-constexpr int64_t kOneLaunchBonds = 131072;
+constexpr int64_t kOneLaunchBonds = 262144;
 
 static inline bool rebuild_in_one(const Geo &g) {
   return g.nb <= kOneLaunchBonds && (int64_t)g.n1d * g.n1d <= kColScanMax;
@@ -1094,14 +1095,14 @@ static inline bool rebuild_in_one(const Geo &g) {
 // 34.3 / 32.7.
 constexpr int64_t kSmallBonds = 40960;
 
-// Blocks of the one launch: enough for 800 bonds each (64 or 128 blocks where
-// they were the best of 16 to 256 at 52k and 101k bonds), 400 in blocks of
-// 512, and in small sparse systems for 64 columns each, whose sort is the
-// longest pass there.
+// Blocks of the one launch: enough for 800 bonds each (64 or 128 blocks were
+// the best of 16 to 256 at 52k and 101k bonds; at 155k 1200 bonds a block cost
+// 1.5 us a step more), 400 in blocks of 512, and in small sparse systems for
+// 64 columns each, whose sort is the longest pass there.
 static inline unsigned one_blocks(const Geo &g, int block) {
   const int64_t ncol = (int64_t)g.n1d * g.n1d, per = block == 512 ? 400 : 800;
   const int64_t b = std::max<int64_t>((g.nb + per - 1) / per, std::min<int64_t>((ncol + 63) / 64, 64));
-  return (unsigned)std::min<int64_t>(std::max<int64_t>(b, 1), 128);
+  return (unsigned)std::min<int64_t>(std::max<int64_t>(b, 1), 256);
 }
 
 // The block that leaves last: until then a block that comes late must still

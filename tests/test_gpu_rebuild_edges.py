@@ -109,8 +109,8 @@ def _spread(nb):
 
 
 # 400 and 800 bonds a block of the one-launch rebuild, which has blocks of 512
-# threads up to 40960 bonds and serves 131072
-@pytest.mark.parametrize("nb", [799, 800, 801, 25599, 40960, 40961, 102401, 131071, 131072, 131073])
+# threads up to 40960 bonds and serves 262144
+@pytest.mark.parametrize("nb", [799, 800, 801, 25599, 40960, 40961, 102401, 131073, 262143, 262144, 262145])
 def test_lists_of_one_and_several_launches(nb):
     p, fil, n1d = _spread(nb)
     assert fil.nb == nb
