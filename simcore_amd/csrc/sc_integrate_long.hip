@@ -548,16 +548,24 @@ __device__ __forceinline__ void long_body(const Dev &d, const Geo &g, bool facti
   // new r_prev), the stored ones on a full step
   const double delta = mid ? 0.5 * g.delta : g.delta;
   double rn[S][3], rnn[S][3], uo[S][3];
+  // (the loads of all of a lane's sites before the first use: one wait instead
+  // of one for each site.  Uneven 1.6M bonds 211.3 -> 207.2 us a step, 110k in
+  // filaments of 129-256 sites 31.3 -> 31.0; the random forces loaded ahead as
+  // well spill 16 registers more: 208.5)
+  double rp[S][3];
+#pragma unroll
+  for (int k = 0; k < S; ++k) {
+    for (int q = 0; q < 3; ++q) rp[k][q] = 0.0;
+    if (base + k < n) {
+      const int64_t si = s0 + base + k;
+      for (int q = 0; q < 3; ++q) rp[k][q] = mid ? d.r[q * ns + si] : d.rp[q * ns + si];
+    }
+  }
 #pragma unroll
   for (int k = 0; k < S; ++k) {
     const int i = base + k;
-    double rp[3] = {0.0, 0.0, 0.0};
-    if (i < n) {
-      const int64_t si = s0 + i;
-      for (int q = 0; q < 3; ++q) rp[q] = mid ? d.r[q * ns + si] : d.rp[q * ns + si];
-      if (mid)
-        for (int q = 0; q < 3; ++q) d.rp[q * ns + si] = rp[q];
-    }
+    if (mid && i < n)
+      for (int q = 0; q < 3; ++q) d.rp[q * ns + s0 + i] = rp[k][q];
     if (i == 0) {
       for (int q = 0; q < 3; ++q) fs[k][q] += T[k] * u[k][q];
     } else if (i == n - 1) {
@@ -567,8 +575,18 @@ __device__ __forceinline__ void long_body(const Dev &d, const Geo &g, bool facti
     }
     double mv[3];
     mob(igperp, dg, t[k], fs[k], mv);
-    for (int q = 0; q < 3; ++q) rn[k][q] = rp[q] + delta * mv[q];
+    for (int q = 0; q < 3; ++q) rn[k][q] = rp[k][q] + delta * mv[q];
   }
+  // (and those of the displacement bookkeeping at the end)
+  double acc0[S], dr0[S][3];
+  if (!mid)
+#pragma unroll
+    for (int k = 0; k < S; ++k) {
+      if (base + k >= n) continue;
+      const int64_t si = s0 + base + k;
+      acc0[k] = d.acc[si];
+      for (int q = 0; q < 3; ++q) dr0[k][q] = d.dr0[q * ns + si];
+    }
   // new bond lengths mm and unit vectors uo, kept for the bond records
   double mm[S];
   site_at3<W, S, 1>(rn, rnn, lane, gl, Gf);
@@ -676,12 +694,11 @@ __device__ __forceinline__ void long_body(const Dev &d, const Geo &g, bool facti
       bond_store(d, g, b0 + i, rn[k], rd, mm[k], uo[k]);
     }
     if (!mid) {
-      double a = d.acc[si], dr0[3];
-      for (int q = 0; q < 3; ++q) dr0[q] = d.dr0[q * ns + si];
+      double a = acc0[k];
       d.acc_prev[si] = a;
       for (int rep = 0; rep < 2; ++rep)
         for (int q = 0; q < 3; ++q) {
-          const double dd = rn[k][q] - dr0[q];
+          const double dd = rn[k][q] - dr0[k][q];
           a += dd * dd;
         }
       d.acc[si] = a;
