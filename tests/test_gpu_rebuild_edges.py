@@ -1,7 +1,7 @@
 """Candidate lists where the rebuild's launches change shape: numbers of cell
 columns at the edges of a scan tile (4096) and of the one-launch scan (2^17),
 numbers of bonds at the edges of the list pass's groups (256) and blocks of
-groups (8192).  Checked against a brute-force walk over all pairs."""
+groups (1024).  Checked against a brute-force walk over all pairs."""
 import numpy as np
 import pytest
 
@@ -48,7 +48,8 @@ def _brute(keys, n, site_off):
 
 
 @pytest.mark.parametrize("n1d, nb", [(63, 255), (64, 256), (65, 257), (90, 511), (91, 513),
-                                     (362, 300), (363, 300), (40, 8191), (40, 8192), (40, 8193)])
+                                     (362, 300), (363, 300), (40, 8191), (40, 8192), (40, 8193),
+                                     (363, 1023), (363, 1024), (363, 1025)])
 @pytest.mark.parametrize("precision", ["fp64", "mixed"])
 def test_lists_at_launch_edges(n1d, nb, precision):
     p, fil = _system(n1d, nb, n1d + nb)
