@@ -27,6 +27,7 @@
 
 #include "sc_internal.h"
 #include "sc_math.h"
+#include "sc_thomas.h"
 
 namespace sc {
 
@@ -35,8 +36,6 @@ namespace {
 constexpr int kExactBlock = 256;
 constexpr int kSlots = 288;    // site slots of a block: slices of odd stride
 constexpr int kMaxChains = 64;  // filaments of a block: one lane each in a chain
-constexpr int kAhead = 2;       // rows loaded ahead of a chain (120 registers, four
-                                // wavefronts per SIMD; 4 rows take 144)
 
 // Slice layout of filaments of at most w sites: the stride between slices
 // (odd, so that the chains' lanes, one per slice, hit different banks) and
@@ -46,111 +45,6 @@ __host__ __device__ __forceinline__ int exact_per_block(int w) {
   const int a = kExactBlock / w, b = kSlots / exact_stride(w);
   const int n = a < b ? a : b;
   return n < kMaxChains ? (n < 1 ? 1 : n) : kMaxChains;
-}
-
-// IEEE division of several numerators by one denominator: the refined
-// reciprocal is shared and each quotient rounds once more, which gives the
-// correctly rounded quotient (the steps of the hardware division sequence
-// without its operand scaling).  Valid for 2^-200 <= |den| <= 2^200 or 0 and
-// |num| = 0 or >= 2^-900; v_div_fixup supplies zeros, infinities and NaNs.
-// 81 clocks for two dependent quotients in a chain, against 138 for two IEEE
-// divisions as the compiler expands them (one wavefront, measured).
-__device__ __forceinline__ double shared_rcp(double den) {
-  double y = __builtin_amdgcn_rcp(den);
-  y = fma(y, fma(-den, y, 1.0), y);
-  return fma(y, fma(-den, y, 1.0), y);
-}
-__device__ __forceinline__ double shared_quot(double num, double den, double y) {
-  const double m = num * y;
-  return __builtin_amdgcn_div_fixup(fma(fma(-den, m, num), y, m), den, num);
-}
-// (the high word of |x|, doubled) - 1: zero is the largest value, so a
-// minimum over numerators ignores zeros
-__device__ __forceinline__ uint32_t magnitude(double x) {
-  return ((uint32_t)(__double_as_longlong(x) >> 32) << 1) - 1u;
-}
-constexpr uint32_t kTiny = (1023u - 900u) << 21;  // magnitude of 2^-900
-
-// Thomas with the reference's operation order on symmetric rows {diagonal,
-// right-hand side} and off-diagonals off[i] (rows i, i+1); the solution
-// replaces the right-hand side.  `rows` is the same for every lane: rows
-// past a filament's last are {1, 0} with off-diagonal 0, which solve to 0
-// and leave the others as they are, so no lane needs a branch.  The last row's
-// solution is the forward recursion's value there.  FAST: quotients by
-// shared_quot; returns false when a numerator was too small for it (the
-// caller then sets the rows up again and takes the plain divisions).
-template <bool FAST>
-__device__ __forceinline__ bool thomas_chain(int rows, double2 *row, const double *off) {
-  uint32_t least = ~0u;
-  double cp = 0.0, dp = 0.0, lo = 0.0;
-  double2 v[kAhead];
-  double c[kAhead];
-  auto load = [&](int i0) {
-#pragma unroll
-    for (int k = 0; k < kAhead; ++k) {
-      const int i = i0 + k < rows ? i0 + k : rows - 1;
-      v[k] = row[i];
-      c[k] = off[i];
-    }
-  };
-  auto step = [&](int i, const double2 &w, double o) {
-    const double den = w.x - lo * cp;  // (row 0: lo, cp and dp are 0)
-    const double num = w.y - lo * dp;
-    if (FAST) {
-      const double y = shared_rcp(den);
-      least = min(least, magnitude(num));
-      cp = shared_quot(o, den, y);
-      dp = shared_quot(num, den, y);
-    } else {
-      cp = o / den;
-      dp = num / den;
-    }
-    lo = o;
-    row[i] = make_double2(cp, dp);
-  };
-  load(0);
-  int i0 = 0;
-  for (; i0 + kAhead <= rows; i0 += kAhead) {
-    double2 w[kAhead];
-    double o[kAhead];
-#pragma unroll
-    for (int k = 0; k < kAhead; ++k) {
-      w[k] = v[k];
-      o[k] = c[k];
-    }
-    load(i0 + kAhead);
-#pragma unroll
-    for (int k = 0; k < kAhead; ++k) step(i0 + k, w[k], o[k]);
-  }
-#pragma unroll
-  for (int k = 0; k < kAhead; ++k)
-    if (i0 + k < rows) step(i0 + k, v[k], c[k]);
-  // back substitution, rows rows-2 .. 0
-  double x = dp;
-  auto loadb = [&](int j0) {
-#pragma unroll
-    for (int k = 0; k < kAhead; ++k) v[k] = row[j0 - k > 0 ? j0 - k : 0];
-  };
-  int j0 = rows - 2;
-  loadb(j0);
-  for (; j0 - kAhead + 1 >= 0; j0 -= kAhead) {
-    double2 w[kAhead];
-#pragma unroll
-    for (int k = 0; k < kAhead; ++k) w[k] = v[k];
-    loadb(j0 - kAhead);
-#pragma unroll
-    for (int k = 0; k < kAhead; ++k) {
-      x = w[k].y - w[k].x * x;
-      row[j0 - k].y = x;
-    }
-  }
-#pragma unroll
-  for (int k = 0; k < kAhead; ++k)
-    if (j0 - k >= 0) {
-      x = v[k].y - v[k].x * x;
-      row[j0 - k].y = x;
-    }
-  return !FAST || least >= kTiny;
 }
 
 // Metric determinants (src/filament.cpp:613-623) from the cosines cs[0..n-3]
@@ -277,7 +171,7 @@ __global__ __launch_bounds__(kExactBlock) void k_integrate_exact(Dev d, Geo g, E
   // the lane's row of a solve: row, unit row past the last, or none
   const bool slot = grp < per;
   const int row = grp * stride + i;
-  const bool sane = gpar > 0x1p-50 && gpar < 0x1p50 && gperp > 0x1p-50 && gperp < 0x1p50;
+  const bool sane = shared_frictions(gpar, gperp);
 
   // ---- loads -------------------------------------------------------------
   double rp_reg[3], fr[3] = {0.0, 0.0, 0.0}, u[3] = {0.0, 0.0, 0.0};
@@ -361,7 +255,7 @@ __global__ __launch_bounds__(kExactBlock) void k_integrate_exact(Dev d, Geo g, E
   auto set_row = [&](double diag, double rhs, double off) {
     P_[row] = make_double2(diag, rhs);
     C_[row] = off;
-    if (!sane || (off != 0.0 && dabs(off) < 0x1p-900)) slow = 1;
+    if (!sane || (off != 0.0 && dabs(off) < kLeastShared)) slow = 1;
   };
   double rhs = 0.0;
   if (draws && slot) {
