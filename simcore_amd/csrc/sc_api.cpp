@@ -11,6 +11,7 @@
 #include <vector>
 
 #include "sc_internal.h"
+#include "sc_limits.h"
 #include "sc_math.h"
 #include "sc_system.h"
 
@@ -258,21 +259,17 @@ void free_cand(sc_system *h) {
   h->cand_bytes = 0;
 }
 
-// Candidates are numbered in int32 and each incidence entry holds a
-// candidate index shifted left by one bit.
-constexpr int64_t kMaxCandidates = ((int64_t)1 << 30) - 1;
-
 // Initial candidate capacity: capacity_factor * bonds + 4096 (4 when the
 // factor is 0); a negative factor is an absolute capacity of -factor
 // candidates (tests of capacity growth use it).
 int64_t initial_capacity(const sc_params &p, int64_t nb) {
   if (p.capacity_factor < 0) return std::max<int64_t>(1, (int64_t)(-p.capacity_factor));
   const double cf = p.capacity_factor > 0 ? p.capacity_factor : 4.0;
-  return std::min<int64_t>((int64_t)(cf * nb) + 4096, kMaxCandidates);
+  return std::min<int64_t>((int64_t)(cf * nb) + 4096, sc::kMaxCandidates);
 }
 
 int alloc_cand(sc_system *h, int64_t cap) {
-  if (cap > kMaxCandidates)
+  if (cap > sc::kMaxCandidates)
     return fail(h, SC_ERR_NOMEM, "more than 2^30 - 1 candidate pairs (" + std::to_string(cap) +
                                      " asked for)");
   free_cand(h);
@@ -290,14 +287,6 @@ int alloc_cand(sc_system *h, int64_t cap) {
   }
   h->g.cap = cap;
   return SC_OK;
-}
-
-// Capacity after an overflow that asked for `need` candidates: doubled, or
-// need + 25% + 1024 if more, at most kMaxCandidates unless need itself is
-// larger (alloc_cand then refuses).
-int64_t grown_capacity(int64_t cap, int64_t need) {
-  const int64_t want = std::max<int64_t>(2 * cap, need + need / 4 + 1024);
-  return need > kMaxCandidates ? need : std::min(want, kMaxCandidates);
 }
 
 // Control-block transfers, ordered on the system's stream.
@@ -603,7 +592,7 @@ int initial_rebuild(sc_system *h) {
     HIPCHK(h, hipGetLastError());
     c = read_ctl(h);
     if (c.overflow) {
-      if ((rc = alloc_cand(h, grown_capacity(h->g.cap, c.nc_need)))) return rc;
+      if ((rc = alloc_cand(h, sc::grown_capacity(h->g.cap, c.nc_need)))) return rc;
       continue;
     }
     c.rebuild = 0;
@@ -1555,7 +1544,7 @@ int sc_step_poll(sc_handle h, int *done) {
     // the capacity check returned): grow the candidate buffers and run the
     // remaining steps again from there
     ++h->grow_rounds;
-    if ((rc = alloc_cand(h, grown_capacity(h->g.cap, c.nc_need)))) {
+    if ((rc = alloc_cand(h, sc::grown_capacity(h->g.cap, c.nc_need)))) {
       h->pending = false;
       return rc;
     }

@@ -22,6 +22,7 @@
 
 #include "sc_block.h"
 #include "sc_internal.h"
+#include "sc_limits.h"
 #include "sc_math.h"
 
 namespace sc {
@@ -813,23 +814,23 @@ __device__ __forceinline__ int64_t n_supers(int64_t nb) {
 }
 
 __device__ __forceinline__ void degsum_body(const Dev &d, const Geo &g, int64_t sup) {
-  __shared__ int ws[4];
+  __shared__ int64_t ws[4];
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   int32_t *gsum = d.scan_tmp + n_supers(g.nb);
   const int64_t ngrp = n_groups(g.nb);
   static_assert(kSuper == 4, "a group per wavefront");
   const int64_t grp = sup * kSuper + wv;
-  int all = 0;
+  int64_t all = 0;
 #pragma unroll
   for (int k = 0; k < kPullGroup / 64; ++k) {
     const int64_t b = grp * kPullGroup + lane + 64 * k;
     if (b < g.nb) all += d.deg[b];
   }
   for (int o = 32; o > 0; o >>= 1) all += __shfl_xor(all, o, 64);
-  if (lane == 0 && grp < ngrp) gsum[grp] = all;
+  if (lane == 0 && grp < ngrp) gsum[grp] = kept_length(all);
   if (lane == 0) ws[wv] = all;
   __syncthreads();
-  if (threadIdx.x == 0) d.scan_tmp[sup] = ws[0] + ws[1] + ws[2] + ws[3];
+  if (threadIdx.x == 0) d.scan_tmp[sup] = kept_length(ws[0] + ws[1] + ws[2] + ws[3]);
 }
 
 __global__ __launch_bounds__(256) void k_degsum(Dev d, Geo g) {
@@ -952,7 +953,8 @@ constexpr int kPullStage = 512;
 
 // Each 256 threads of a block take every so-many-th group of kPullGroup
 // bonds; the list range of a group starts at the sum of the groups before it.
-// The total is 64-bit, so a count that does not fit the lists is seen before
+// The total is 64-bit and its parts are cut off rather than wrapped
+// (kept_length), so a count that does not fit the lists is seen before
 // anything is written.
 template <int BLOCK>
 struct PullLds {
@@ -997,7 +999,7 @@ __device__ __forceinline__ void pull_body(const Dev &d, const Geo &g, int64_t bi
   for (int i = 0; i < BLOCK / 64; ++i) total += red[i];
   const bool fits = total <= 2 * g.cap;
   if (i0 == 0) {
-    d.ctl->nc_need = total / 2;
+    d.ctl->nc_need = candidates_of(total);
     if (fits) {
       d.ctl->nc = total / 2;
       d.ctl->n_rebuilds += 1;
