@@ -490,20 +490,14 @@ __global__ void k_scatter(Dev d, Geo g, int guard) {
 
 // Each cell column sorted by (cell key, bond index): kColLanes lanes per
 // column; an entry's place is the number of smaller (key, bond) pairs in its
-// column, counted against the column staged in LDS (a column holds a few tens
-// of bonds at the densities simulated; longer ones than the stage count
-// against global memory).  Members of a cell thus appear in bond order, the
-// order Cell::AddObj appends in (src/cell.cpp:5-8).  The pass also writes the
-// column's occupancy words (every word of the column, so no clearing pass is
-// needed) with each word's count of occupied cells before it, and the column's
-// run table: the first sorted entry of each occupied cell in z order, at the
-// column's own range of `cell_first`, and the number of occupied cells.  The
-// degree pass finds a cell's run from its rank among the column's occupied
-// cells (cell_run_of) in these small, L2-resident arrays, which cut its HBM
-// reads from 540 to 200 MB on the uneven 1.6M-bond system; the cell-indexed
-// runs (n1d^3 entries, mostly empty, so every lookup is a random HBM line)
-// serve the list pass's rare lookups beyond a bond's run slab (measured faster
-// there) and the crosslink partner search.
+// column, counted against the column staged in LDS.  Members of a cell thus
+// appear in bond order, the order Cell::AddObj appends in (src/cell.cpp:5-8).
+// The pass also writes the column's cell tables: the first sorted entry of
+// each occupied cell in z order, at the column's own range of `cell_first`,
+// and the column's words of `cell_occ` (every word, so no clearing pass is
+// needed), each the occupancy bits of 32 cells and where in `cell_first` the
+// first of them stands.  A cell's run is found from its rank among the word's
+// bits (cell_run_of) in these small, L2-resident arrays.
 //
 // A column's lanes lie in one wavefront and share nothing with others, so the
 // pass has no block barrier.  Bound: the latency of a column's few loads.
@@ -512,8 +506,16 @@ __global__ void k_scatter(Dev d, Geo g, int guard) {
 // column per wavefront, keys gathered: 7 and 6 us more); in the one-launch rebuild,
 // where a few hundred wavefronts serve all columns, 52k bonds gained 1.1 us a
 // step.
+//
+// A wavefront with a column of more than kColStage bonds (large cells, dense
+// systems, bundles along z) takes its four one after the other with all 64
+// lanes, in all of its LDS: the count is quadratic, and 16 lanes that read the
+// column from global memory for each bond took 126 us instead of 24 for 1600
+// columns of 90 bonds on average, 560 instead of 77 for 400 of 250, 2530
+// instead of 224 for a bundle along z of 256 of 470.
 constexpr int kColLanes = 16;
 constexpr int kColStage = 96;
+constexpr int kColOwn = 4;      // bonds a lane ranks at a time in a long column
 constexpr int kOccWords = 44;  // occ_words <= 42 (n1d^3 < 2^31)
 
 template <int BLOCK>
@@ -530,97 +532,165 @@ __device__ __forceinline__ void wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// Pairs [from, from + count) of the column at s, padded to whole groups of
+// four (which the counts below read together).
+template <int LANES>
+__device__ __forceinline__ void stage_pairs(const Dev &d, int32_t s, int32_t from, int32_t count,
+                                            int lane, int64_t *ks) {
+  for (int i = lane; i < ((count + 3) & ~3); i += LANES)
+    ks[i] = i < count ? d.col_tmp[s + from + i] : INT64_MAX;
+}
+
+// The sort of a column that its LANES lanes hold in LDS.
+template <int LANES>
+__device__ __forceinline__ void sort_short(const Dev &d, int32_t s, int32_t m, int lane,
+                                           int64_t *ks, int32_t *kr) {
+  stage_pairs<LANES>(d, s, 0, m, lane, ks);
+  wave_sync();
+  for (int i = lane; i < m; i += LANES) {
+    const int64_t ki = ks[i];
+    int32_t r = 0;
+    for (int j = 0; j < m; j += 4) {
+      const int64_t a = ks[j], b = ks[j + 1], x = ks[j + 2], y = ks[j + 3];
+      r += (a < ki) + (b < ki) + (x < ki) + (y < ki);
+    }
+    kr[r] = (int32_t)(ki >> 32);
+    d.sorted[s + r] = (int32_t)(uint32_t)ki;
+    d.skey[s + r] = (int32_t)(ki >> 32);
+  }
+}
+
+// The sort of a column of any length by a wavefront, kColOwn bonds a lane
+// against `stage` pairs at a time.
+__device__ __forceinline__ void sort_long(const Dev &d, int32_t s, int32_t m, int lane,
+                                          int64_t *ks, int32_t *kr, int32_t stage) {
+  for (int32_t i0 = 0; i0 < m; i0 += 64 * kColOwn) {
+    int64_t own[kColOwn];
+    int32_t r[kColOwn];
+#pragma unroll
+    for (int q = 0; q < kColOwn; ++q) {
+      const int32_t i = i0 + 64 * q + lane;
+      own[q] = i < m ? d.col_tmp[s + i] : 0;
+      r[q] = 0;
+    }
+    for (int32_t t0 = 0; t0 < m; t0 += stage) {
+      const int32_t count = m - t0 < stage ? m - t0 : stage;
+      if (i0 == 0 || m > stage) {  // (a column within the stage stays there)
+        wave_sync();
+        stage_pairs<64>(d, s, t0, count, lane, ks);
+        wave_sync();
+      }
+      for (int j = 0; j < count; j += 4) {
+        const int64_t a = ks[j], b = ks[j + 1], x = ks[j + 2], y = ks[j + 3];
+#pragma unroll
+        for (int q = 0; q < kColOwn; ++q)
+          r[q] += (a < own[q]) + (b < own[q]) + (x < own[q]) + (y < own[q]);
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < kColOwn; ++q)
+      if (i0 + 64 * q + lane < m) {
+        if (m <= stage) kr[r[q]] = (int32_t)(own[q] >> 32);
+        d.sorted[s + r[q]] = (int32_t)(uint32_t)own[q];
+        d.skey[s + r[q]] = (int32_t)(own[q] >> 32);
+      }
+  }
+  // (read back below from global memory when not in LDS)
+  if (m > stage) __threadfence();
+}
+
+// The cell tables of column c, bonds [s, s + m) of the sorted order; each run
+// start's rank among the column's run starts comes from a ballot per LANES
+// entries.  `held`: the sorted keys are in kr; `rounds` the same for all lanes
+// of the wavefront; `shift` the lanes' place in a ballot.
+template <int LANES>
+__device__ __forceinline__ void column_tables(const Dev &d, const Geo &g, int64_t c, bool live,
+                                              int32_t s, int32_t m, bool held, int rounds,
+                                              int lane, int shift, const int32_t *kr,
+                                              uint32_t *occ) {
+  const int n = g.n1d, W = g.occ_words;
+  const int64_t ncol = (int64_t)n * n;
+  const int32_t e = s + m;
+  int32_t ncell = 0;
+  for (int q = 0; q < rounds; ++q) {
+    const int i = q * LANES + lane;
+    int32_t k = -1;
+    bool start = false;
+    if (i < m) {
+      k = held ? kr[i] : d.skey[s + i];
+      const int32_t kp = i == 0 ? -1 : (held ? kr[i - 1] : d.skey[s + i - 1]);
+      start = k != kp;
+    }
+    unsigned long long bal = __ballot(start) >> shift;
+    if (LANES < 64) bal &= (1ull << (LANES & 63)) - 1;
+    if (start) {
+      const int32_t rank = ncell + __popcll(bal & ((1ull << lane) - 1ull));
+      d.cell_first[s + rank] = s + i;
+      const int p = k - (int32_t)c * n + 1;
+      atomicOr(&occ[p >> 5], 1u << (p & 31));
+    }
+    ncell += __popcll(bal);
+  }
+  wave_sync();
+  if (!live) return;
+  // (the copies of the first and the last cell beyond the ends count for no
+  // run index)
+  const uint32_t below = (occ[n >> 5] >> (n & 31)) & 1u, above = (occ[0] >> 1) & 1u;
+  for (int w = lane; w < W; w += LANES) {
+    int at = s;
+    for (int v = 0; v < w; ++v) at += __popc(occ[v]);
+    uint32_t bits = occ[w];
+    if (w == 0) {
+      bits |= below;
+      at -= (int)below;
+    }
+    if (w == (n + 1) >> 5) bits |= above << ((n + 1) & 31);
+    d.cell_occ[c * W + w] = make_int2((int32_t)bits, at);
+  }
+  // where the last run of the column ends (the first of the next column
+  // starts there if every bond is a run of its own)
+  if (lane == 0 && ncell < m) d.cell_first[s + ncell] = e;
+  if (lane == 0 && c == ncol - 1) d.cell_first[e] = e;
+}
+
 template <int BLOCK>
 __device__ __forceinline__ void colsort_body(const Dev &d, const Geo &g, int64_t bid,
                                              int64_t nblk, ColsortLds<BLOCK> &L) {
-  constexpr int kCols = BLOCK / kColLanes;
+  constexpr int kCols = BLOCK / kColLanes, kWaveCols = 64 / kColLanes;
   const int col = threadIdx.x / kColLanes, lane = threadIdx.x % kColLanes;
-  const int shift = (threadIdx.x & 63) - lane;  // the group's lanes in a ballot
-  int64_t *ks = L.ks[col];
-  int32_t *kr = L.kr[col];
-  uint32_t *occ = L.occ[col];
-  const int n = g.n1d, W = g.occ_words;
-  const int64_t ncol = (int64_t)n * n;
+  const int wlane = threadIdx.x & 63, col0 = col / kWaveCols * kWaveCols;
+  const int W = g.occ_words;
+  const int64_t ncol = (int64_t)g.n1d * g.n1d;
   const int64_t ngrp = (ncol + kCols - 1) / kCols;
   for (int64_t grp = bid; grp < ngrp; grp += nblk) {
     const int64_t c = grp * kCols + col;
     const bool live = c < ncol;
-    const int32_t s = live ? d.col_start[c] : 0, e = live ? d.col_start[c + 1] : 0, m = e - s;
-    const bool staged = m <= kColStage;
-    for (int w = lane; w < W; w += kColLanes) occ[w] = 0u;
+    const int32_t s = live ? d.col_start[c] : 0, m = live ? d.col_start[c + 1] - s : 0;
+    for (int w = lane; w < W; w += kColLanes) L.occ[col][w] = 0u;
     if (live && lane == 0) d.col_count[c] = 0;  // for the next build's count
-    // (padded to whole groups of four, which the count below reads together)
-    if (staged)
-      for (int i = lane; i < ((m + 3) & ~3); i += kColLanes)
-        ks[i] = i < m ? d.col_tmp[s + i] : INT64_MAX;
-    wave_sync();
-    for (int i = lane; i < m; i += kColLanes) {
-      const int64_t ki = staged ? ks[i] : d.col_tmp[s + i];
-      int32_t r = 0;
-      if (staged) {
-        for (int j = 0; j < m; j += 4) {
-          const int64_t a = ks[j], b = ks[j + 1], x = ks[j + 2], y = ks[j + 3];
-          r += (a < ki) + (b < ki) + (x < ki) + (y < ki);
-        }
-        kr[r] = (int32_t)(ki >> 32);
-      } else {
-        for (int j = 0; j < m; ++j) r += d.col_tmp[s + j] < ki;
-      }
-      d.sorted[s + r] = (int32_t)(uint32_t)ki;
-      d.skey[s + r] = (int32_t)(ki >> 32);
-    }
-    // runs: staged columns read the sorted keys from LDS, long ones from
-    // global memory after a fence; each run start's rank among the column's
-    // run starts comes from a ballot per kColLanes entries
-    if (!staged) __threadfence();
-    wave_sync();
-    int32_t ncell = 0;
-    // (the four columns of a wavefront take the longest one's rounds)
-    int rounds = (m + kColLanes - 1) / kColLanes;
+    int longest = m;
     for (int o = kColLanes; o < 64; o <<= 1) {
-      const int y = __shfl_xor(rounds, o, 64);
-      rounds = y > rounds ? y : rounds;
+      const int y = __shfl_xor(longest, o, 64);
+      longest = y > longest ? y : longest;
     }
-    for (int q = 0; q < rounds; ++q) {
-      const int i = q * kColLanes + lane;
-      int32_t k = -1;
-      bool start = false;
-      if (i < m) {
-        k = staged ? kr[i] : d.skey[s + i];
-        const int32_t kp =
-            i == 0 ? -1 : (staged ? kr[i - 1] : d.skey[s + i - 1]);
-        start = k != kp;
+    if (longest <= kColStage) {
+      sort_short<kColLanes>(d, s, m, lane, L.ks[col], L.kr[col]);
+      wave_sync();
+      // (the wavefront's columns take the longest one's rounds)
+      column_tables<kColLanes>(d, g, c, live, s, m, true, (longest + kColLanes - 1) / kColLanes,
+                               lane, wlane - lane, L.kr[col], L.occ[col]);
+    } else {
+      for (int k = 0; k < kWaveCols; ++k) {
+        const int64_t ck = grp * kCols + col0 + k;
+        const int32_t sk = __shfl(s, k * kColLanes, 64), mk = __shfl(m, k * kColLanes, 64);
+        wave_sync();
+        // (the four columns' stages are one piece of memory)
+        int32_t *kr = &L.kr[0][0] + col0 * kColStage;
+        sort_long(d, sk, mk, wlane, &L.ks[0][0] + col0 * kColStage, kr, kWaveCols * kColStage);
+        wave_sync();
+        column_tables<64>(d, g, ck, ck < ncol, sk, mk, mk <= kWaveCols * kColStage, (mk + 63) / 64,
+                          wlane, 0, kr, L.occ[col0 + k]);
       }
-      constexpr uint32_t kMask = (uint32_t)((1ull << kColLanes) - 1);
-      const uint32_t bal = (uint32_t)(__ballot(start) >> shift) & kMask;
-      if (start) {
-        const int32_t rank = ncell + __popc(bal & ((1u << lane) - 1u));
-        d.cell_first[s + rank] = s + i;
-        const int p = k - (int32_t)c * n + 1;
-        atomicOr(&occ[p >> 5], 1u << (p & 31));
-      }
-      ncell += __popc(bal);
-    }
-    wave_sync();
-    if (live) {
-      // (the copies of the first and the last cell beyond the ends count for
-      // no run index)
-      const uint32_t below = (occ[n >> 5] >> (n & 31)) & 1u, above = (occ[0] >> 1) & 1u;
-      for (int w = lane; w < W; w += kColLanes) {
-        int at = s;
-        for (int v = 0; v < w; ++v) at += __popc(occ[v]);
-        uint32_t bits = occ[w];
-        if (w == 0) {
-          bits |= below;
-          at -= (int)below;
-        }
-        if (w == (n + 1) >> 5) bits |= above << ((n + 1) & 31);
-        d.cell_occ[c * W + w] = make_int2((int32_t)bits, at);
-      }
-      // where the last run of the column ends (the first of the next column
-      // starts there if every bond is a run of its own)
-      if (lane == 0 && ncell < m) d.cell_first[s + ncell] = e;
-      if (lane == 0 && c == ncol - 1) d.cell_first[e] = e;
     }
     wave_sync();
   }
