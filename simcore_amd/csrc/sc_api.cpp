@@ -55,6 +55,7 @@ struct sc_system {
   int pack_waves = 0;
   int64_t pack_sites = 0;
   sc::Tune tune;
+  bool shape_given = false;  // tune is from sc_set_launch_shape or sc_autotune
   // graphs: [0] odd step (rebuild stage included), [1] even step (a rebuild
   // is only ever decided after a full step, i.e. at odd steps), [2] the
   // odd+even pair, [3] kGraphPairs such pairs (fewer graph boundaries on
@@ -301,6 +302,35 @@ int write_ctl(sc_system *h, const Ctl &c) {
   HIPCHK(h, hipMemcpyAsync(h->d.ctl, &c, sizeof(Ctl), hipMemcpyHostToDevice, h->stream));
   HIPCHK(h, hipStreamSynchronize(h->stream));
   return SC_OK;
+}
+
+// Mean length of a bond's list up to which the balanced pair kernel is the
+// faster one.  Its lanes evaluate 128 entries and then each bond's lane adds
+// up the bond's, so with long lists a few lanes add while the others wait;
+// the per-bond kernel has every lane at its own list, all of about the same
+// length, but needs enough bonds to fill the chip.  us a pass, balanced /
+// per bond with 256 threads, by mean length: 4k bonds 65: 100 / 130, 151: 222
+// / 260, 317: 425 / 424; 50k 64: 142 / 184, 100: 243 / 231; 100k 27: 111 / 144,
+// 52: 204 / 189, 103: 473 / 303; 200k 35: 209 / 214, 52: 359 / 317; 600k 50:
+// 717 / 806, 101: 1834 / 1580.  Just above 131072 bonds, where a wavefront
+// takes 64 of them, they are too few to fill the chip: at 150k equal at 19 and
+// 1.28 times the time at 32.  FP64's lines lie up to a fifth lower.
+double longest_balanced(int64_t nb) {
+  return nb <= 32768 ? 160.0 : nb <= 65536 ? 80.0 : nb <= 131072 ? 32.0 : nb < 200000 ? 16.0 : 40.0;
+}
+
+// The launch shape that depends on the lists, for a handle whose caller chose
+// none; the stream idle and ctl_host current.  It changes no result.  The
+// lists have to get a quarter shorter again before the shape changes back, so
+// that a system near the line does not capture its graphs anew each time.
+void fit_shape(sc_system *h) {
+  if (h->shape_given) return;
+  const double mean = 2.0 * (double)h->ctl_host->nc / (double)h->g.nb;
+  const double line = longest_balanced(h->g.nb) * (h->tune.pair_bal ? 1.0 : 0.75);
+  const int bal = mean <= line ? 1 : 0;
+  if (bal == h->tune.pair_bal) return;
+  h->tune.pair_bal = bal;
+  drop_graph(h);
 }
 
 // Points d.br / d.br_out at the records of the state after i_step steps.
@@ -1397,6 +1427,7 @@ int sc_load_filaments(sc_handle h, int32_t nf, const int32_t *site_off,
   HIPCHK(h, hipStreamSynchronize(h->stream));
   *h->ctl_host = read_ctl(h);
   h->i_step_host = h->ctl_host->i_step;
+  fit_shape(h);
   h->loaded = true;
   return SC_OK;
 }
@@ -1508,6 +1539,7 @@ int sc_step_async(sc_handle h, int32_t n_steps) {
                   "handle is in an error state");
     h->target = h->i_step_host;
     h->grow_rounds = 0;
+    fit_shape(h);
   }
   if (n_steps == 0) return SC_OK;
   const int64_t from = h->target;
@@ -2267,6 +2299,7 @@ int sc_autotune(sc_handle h, int32_t steps, sc_tune_report *report) {
   }
   // leave the system where it was, with the chosen shapes
   h->tune = rc ? start : best;
+  if (!rc) h->shape_given = true;
   drop_graph(h);
   h->g.xi_buf = xi_keep;
   h->g.thermo = thermo_keep;
@@ -2308,6 +2341,7 @@ int sc_set_launch_shape(sc_handle h, const sc_launch_shape *shape) {
   h->tune.int_streams = v.integrate_streams;
   h->tune.parts = v.pair_parts > 1 ? v.pair_parts : 1;
   h->tune.early_long = v.early_long;
+  h->shape_given = true;
   drop_graph(h);
   if (v.integrate_streams > 0 || v.pair_parts > 1 || v.early_long) return ensure_side_streams(h);
   return SC_OK;

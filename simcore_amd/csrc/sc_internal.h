@@ -183,10 +183,11 @@ struct Tune {
   int pair_block = 256;  // threads per block of the pair kernel
   int pair_xcd = 0;      // 1: consecutive bond ranges stay on one XCD
   // 1: incidences dealt evenly over a wave's lanes.  The default at every
-  // size and precision, because the per-bond walk lasts as long as a wave's
-  // longest list: us per step with pair_block 256 against balanced, 1k bonds
-  // 34.8 / 28.1, 52k 40.4 / 34.5, 620k 105.6 / 84.0, 1.6M uneven 273 / 221,
-  // crosslinked 412k 105 / 88; FP64 1.2k 41.5 / 35.4, 155k 76.2 / 65.7
+  // size and precision unless the lists are long (longest_balanced), because
+  // the per-bond walk lasts as long as a wave's longest list: us per step with
+  // pair_block 256 against balanced, 1k bonds 34.8 / 28.1, 52k 40.4 / 34.5,
+  // 620k 105.6 / 84.0, 1.6M uneven 273 / 221, crosslinked 412k 105 / 88; FP64
+  // 1.2k 41.5 / 35.4, 155k 76.2 / 65.7
   int pair_bal = 1;
   int int_waves = 1;     // waves per block of the register integrator
   int int_layout = 1;    // up to 64 sites: 0 one site per lane, 1 two (the
