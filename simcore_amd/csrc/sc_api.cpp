@@ -319,16 +319,18 @@ double longest_balanced(int64_t nb) {
   return nb <= 32768 ? 160.0 : nb <= 65536 ? 80.0 : nb <= 131072 ? 32.0 : nb < 200000 ? 16.0 : 40.0;
 }
 
-// The launch shape that depends on the lists, for a handle whose caller chose
-// none; the stream idle and ctl_host current.  It changes no result.  The
-// lists have to get a quarter shorter again before the shape changes back, so
-// that a system near the line does not capture its graphs anew each time.
-void fit_shape(sc_system *h) {
-  if (h->shape_given) return;
+// The launches that depend on the lists, the stream idle and ctl_host current:
+// the rebuild stage's, and the pair kernel's if the caller chose none.  They
+// change no result.  The lists have to get a quarter shorter again before a
+// choice changes back, so that a system near the line does not capture its
+// graphs anew each time.
+void fit_launches(sc_system *h) {
   const double mean = 2.0 * (double)h->ctl_host->nc / (double)h->g.nb;
-  const double line = longest_balanced(h->g.nb) * (h->tune.pair_bal ? 1.0 : 0.75);
-  const int bal = mean <= line ? 1 : 0;
-  if (bal == h->tune.pair_bal) return;
+  const int one = sc::rebuild_in_one(h->g, mean, h->g.one_launch != 0) ? 1 : 0;
+  int bal = h->tune.pair_bal;
+  if (!h->shape_given) bal = mean <= longest_balanced(h->g.nb) * (bal ? 1.0 : 0.75) ? 1 : 0;
+  if (one == h->g.one_launch && bal == h->tune.pair_bal) return;
+  h->g.one_launch = one;
   h->tune.pair_bal = bal;
   drop_graph(h);
 }
@@ -1016,6 +1018,7 @@ bool system_batchable(sc_handle h) {
 }
 
 void system_member(sc_handle h, Member *m) {
+  fit_launches(h);
   m->d[0] = h->d;
   m->d[0].br = h->rec[0];
   m->d[0].br_out = h->rec[1];
@@ -1422,12 +1425,13 @@ int sc_load_filaments(sc_handle h, int32_t nf, const int32_t *site_off,
   sc::launch_bond_init(d, g, h->p.precision, h->stream);
   HIPCHK(h, hipStreamSynchronize(h->stream));
   HIPCHK(h, hipGetLastError());
+  g.one_launch = sc::rebuild_in_one(g, 0.0, true) ? 1 : 0;  // (the lists are not known yet)
   if ((rc = initial_rebuild(h))) return rc;
   sc::launch_decide(d, g, h->stream);  // the decision for step 1
   HIPCHK(h, hipStreamSynchronize(h->stream));
   *h->ctl_host = read_ctl(h);
   h->i_step_host = h->ctl_host->i_step;
-  fit_shape(h);
+  fit_launches(h);
   h->loaded = true;
   return SC_OK;
 }
@@ -1539,7 +1543,7 @@ int sc_step_async(sc_handle h, int32_t n_steps) {
                   "handle is in an error state");
     h->target = h->i_step_host;
     h->grow_rounds = 0;
-    fit_shape(h);
+    fit_launches(h);
   }
   if (n_steps == 0) return SC_OK;
   const int64_t from = h->target;

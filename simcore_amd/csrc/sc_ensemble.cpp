@@ -240,7 +240,7 @@ int enqueue_batch(sc_ensemble e, Batch &B) {
   for (int j = 0; j < n; ++j) {
     const sc::Geo &g = B.hm[j].g;
     key.insert(key.end(), {g.nb, g.ns, (int64_t)g.n1d, (int64_t)B.hm[j].pack_waves,
-                           (int64_t)B.hm[j].n_long});
+                           (int64_t)B.hm[j].n_long, (int64_t)g.one_launch});
   }
   if (!B.gx[0] || key != B.gkey) {
     const double tcap = e->now();

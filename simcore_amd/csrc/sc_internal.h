@@ -51,6 +51,7 @@ struct Geo {
   double thr;              // 0.25 * cell_len^2
   int n1d;
   int occ_words;           // words of a column in Dev::cell_occ
+  int one_launch;          // the rebuild stage in one launch (rebuild_in_one)
   int stoch;
   int compact;             // mixed precision: 32-byte bond records (sc_math.h)
   double inv_n1d;
@@ -318,6 +319,9 @@ __device__ __forceinline__ int2 cell_run_of(const Dev &d, const Geo &g, int x, i
 // Launchers (sc_kernels.hip).  All are asynchronous on `st`.
 void launch_decide(const Dev &d, const Geo &g, hipStream_t st);
 void launch_commit(const Dev &d, const Geo &g, hipStream_t st);
+// Whether the rebuild stage of a system whose lists have `mean` entries a bond
+// belongs in one launch (Geo::one_launch); `now`: what it is at present.
+bool rebuild_in_one(const Geo &g, double mean, bool now);
 // `fold`: the odd step follows an even step that was not committed; the first
 // launch commits it and decides the rebuild
 void launch_rebuild(const Dev &d, const Geo &g, bool fold, hipStream_t st);

@@ -1140,24 +1140,27 @@ __global__ __launch_bounds__(256, 8) void k_pull(Dev d, Geo g) {
 }
 
 // ---- the rebuild stage in one launch ----------------------------------------
-// Every launch costs 1.55 us also on a step that does not rebuild, so up to
-// kOneLaunchBonds one launch runs the passes, with a barrier between them
-// among its blocks (sc_block.h): 3.5 us among 64 blocks, 7 among 256, against
-// 1.55 us for a kernel boundary; hence few, large blocks, and the launches for
-// larger systems, whose passes want more of them.  us a step, seven launches
-// against one: 1k bonds 25.7 / 22.4, FP64 1.2k 31.4 / 27.3, 52k 31.9 / 29.6,
-// 62k with stress sums 34.2 / 31.6, 155k 41.6 / 39.4, FP64 155k 55.4 / 53.6,
-// FP64 uneven 230k 92.4 / 89.0, 232k 47.5 / 47.3, 372k 60.9 / 66.4.  Up to 256k
-// bonds every thread of 256 blocks has one bond.
+// Every launch costs 1.55 us also on a step that does not rebuild, so one
+// launch runs the passes where it can, with a barrier between them among its
+// blocks (sc_block.h): 3.5 us among 64 blocks, 7 among 256, against 1.55 us for
+// a kernel boundary; hence few, large blocks.  The seven launches serve what
+// wants more of them.  us a step, seven launches against one:
+//   many bonds (up to 256k every thread of 256 blocks has one bond): 1k 25.7 /
+//     22.4, FP64 1.2k 31.4 / 27.3, 52k 31.9 / 29.6, 62k with stress sums 34.2 /
+//     31.6, 155k 41.6 / 39.4, FP64 155k 55.4 / 53.6, FP64 uneven 230k 92.4 /
+//     89.0, 232k 47.5 / 47.3, 372k 60.9 / 66.4;
+//   many columns, whose sort is the longest pass (a rebuild every eleventh
+//     step): 200^2 with 300 bonds 22.6 / 20.7, with 5000 25.3 / 24.6, 256^2
+//     23.0 / 22.3 and 25.5 / 26.2, 362^2 24.0 / 26.5 and 26.8 / 31.6;
+//   long lists, whose gathers want every CU (the same): 64k bonds with 30
+//     entries each 97.6 / 98.7, with 127 381 / 387, 150k with 18 139.5 / 141.4;
+//     16k (in blocks of 512) with 57 115.3 / 112.8, with 130 237.7 / 236.2.
 //
 // The list pass adds up the degrees itself: with few bonds that is less than
 // the pass of group sums and its barrier, 11 us of a rebuild of 85 at 52k
 // bonds (27.5 -> 27.1 us a step, 62k with stress sums 29.2 -> 28.9).
 constexpr int64_t kOneLaunchBonds = 262144;
-
-static inline bool rebuild_in_one(const Geo &g) {
-  return g.nb <= kOneLaunchBonds && (int64_t)g.n1d * g.n1d <= kColScanMax;
-}
+constexpr int64_t kOneLaunchColumns = (int64_t)1 << 16;
 
 // Threads of a block: the gathers of the degree and list passes keep a CU's
 // load units busy, so small systems spread their bonds over more CUs with
@@ -1165,6 +1168,12 @@ static inline bool rebuild_in_one(const Geo &g) {
 // bonds 18.2 / 18.6, 10k 20.1 / 20.5, 31k 23.2 / 23.5, 62k 28.0 / 27.5, 102k
 // 34.3 / 32.7.
 constexpr int64_t kSmallBonds = 40960;
+
+// (the lists have to get a quarter shorter again before one launch is back)
+bool rebuild_in_one(const Geo &g, double mean, bool now) {
+  const double line = (g.nb <= kSmallBonds ? 160.0 : 16.0) * (now ? 1.0 : 0.75);
+  return g.nb <= kOneLaunchBonds && (int64_t)g.n1d * g.n1d <= kOneLaunchColumns && mean <= line;
+}
 
 // Blocks of the one launch: enough for 800 bonds each (64 or 128 blocks were
 // the best of 16 to 256 at 52k and 101k bonds; at 155k 1200 bonds a block cost
@@ -1247,7 +1256,7 @@ static inline unsigned sgrid(int64_t n) {
   return b < (unsigned)kStreamBlocks ? b : (unsigned)kStreamBlocks;
 }
 
-// Up to kOneLaunchBonds one launch (k_rebuild_one); above:
+// One launch (k_rebuild_one) where rebuild_in_one says so; else
 // keys (+ column populations) -> column scan -> column scatter -> column
 // sort (+ runs, occupancy) -> degrees -> degree sums -> incidence lists
 // (+ incidence starts, capacity check, displacement restart): 7 launches,
@@ -1260,7 +1269,7 @@ constexpr unsigned kListBlocks = 2048;
 void launch_rebuild(const Dev &d, const Geo &g, bool fold, hipStream_t st) {
   const unsigned gs = sgrid(g.nb);
   const int64_t ncol = (int64_t)g.n1d * g.n1d;
-  if (rebuild_in_one(g)) {
+  if (g.one_launch) {
     const dim3 grid(one_blocks(g, g.nb <= kSmallBonds ? 512 : 1024));
     if (g.nb <= kSmallBonds && fold)
       hipLaunchKernelGGL((k_rebuild_one<512, true>), grid, dim3(512), 0, st, d, g);
@@ -1407,7 +1416,7 @@ void launch_group_rebuild(const Member *dm, const Member *hm, int n, bool fold, 
   bool one = true;
   bool small = true;
   for (int m = 0; m < n; ++m) {
-    one = one && rebuild_in_one(hm[m].g);
+    one = one && hm[m].g.one_launch;
     small = small && hm[m].g.nb <= kSmallBonds;
   }
   if (one) {
