@@ -645,8 +645,8 @@ void get3(double *dst, const double *src_dev, int64_t n) {
 }
 
 // storage-order array of `comp` components x n entries -> caller order
-template <typename T>
-void to_caller(const sc_system *h, const std::vector<int64_t> &map, const T *src, T *dst,
+template <typename S, typename T>
+void to_caller(const sc_system *h, const std::vector<int64_t> &map, const S *src, T *dst,
                int64_t n, int comp) {
   if (!h->reordered) {
     std::copy(src, src + comp * n, dst);
@@ -668,11 +668,17 @@ size_t idle_scratch_bytes(const sc_system *h) {
   return sizeof(int32_t) * sc::kSlabWords * (size_t)h->g.nb;
 }
 
-// Reordered or FP32 arrays of at least this many values are put into the
-// caller's order and precision by a kernel, whose launch costs a few
-// microseconds; below it the host's loop is cheaper (992 sites: 21 us on the
-// host; 1.66M sites: 13.5 ms on the host against the copy alone).
-constexpr int64_t kDeviceOrderMin = 16384;
+// Arrays of at least this many values are put into the caller's order and
+// precision by a kernel, whose launch and wait cost some 20 us; below it the
+// host's loop is cheaper.  us an array, host / device: reordered FP64 32k values
+// 30 / 35, 48k 39 / 41, 64k 51 / 44, 128k 94 / 68, 5M 13500 / 4500; reordered
+// FP32 96k 51 / 56, 192k 92 / 103, 300k 167 / 149; FP32 in the caller's order
+// 192k 61 / 101, 768k 263 / 351, 1.5M 670 / 674.
+int64_t device_order_min(bool reordered, bool f32) {
+  return !reordered ? 1 << 20 : f32 ? 196608 : 49152;
+}
+
+constexpr int64_t kStatsSplitMin = 16384;
 
 // device SoA site/bond array (storage order) -> caller-order FP64 host array,
 // the stream idle.  Arrays already in the caller's order and precision are
@@ -681,16 +687,17 @@ int fetch_mapped(sc_system *h, const void *dev, bool f32, double *out, int64_t n
                  bool sites) {
   const size_t count = (size_t)comp * n;
   if (h->reordered || f32) {
-    if ((int64_t)count < kDeviceOrderMin) {
-      std::vector<double> wide(count);
+    if ((int64_t)count < device_order_min(h->reordered, f32)) {
+      const std::vector<int64_t> &map = sites ? h->site_map : h->bond_map;
       if (f32) {
         std::vector<float> v32(count);
         HIPCHK(h, hipMemcpy(v32.data(), dev, sizeof(float) * count, hipMemcpyDeviceToHost));
-        wide.assign(v32.begin(), v32.end());
+        to_caller(h, map, v32.data(), out, n, comp);
       } else {
-        HIPCHK(h, hipMemcpy(wide.data(), dev, sizeof(double) * count, hipMemcpyDeviceToHost));
+        std::vector<double> v64(count);
+        HIPCHK(h, hipMemcpy(v64.data(), dev, sizeof(double) * count, hipMemcpyDeviceToHost));
+        to_caller(h, map, v64.data(), out, n, comp);
       }
-      to_caller(h, sites ? h->site_map : h->bond_map, wide.data(), out, n, comp);
       return SC_OK;
     }
     double *tmp = idle_scratch(h);
@@ -1929,9 +1936,20 @@ int sc_filament_stats(sc_handle h, double *e2e, double *com) {
     return fail(h, SC_ERR_STATE, "statistics scratch too small");
   HIPCHK(h, hipStreamSynchronize(h->stream));
   refresh_records(h);
-  // results in the caller's filament order, copied into the caller's memory
+  // results in the caller's filament order.  Two small copies take longer than
+  // one and the host's own (38.7 / 28.3 us with 50 filaments); large ones go
+  // straight into the caller's memory.
   sc::launch_filament_stats(h->d, h->g, e2e ? buf : nullptr, com ? buf + n : nullptr, h->stream);
   HIPCHK(h, hipGetLastError());
+  if (e2e && com && n < kStatsSplitMin) {
+    std::vector<double> both(2 * (size_t)n);
+    HIPCHK(h, hipMemcpyAsync(both.data(), buf, sizeof(double) * 2 * n, hipMemcpyDeviceToHost,
+                             h->stream));
+    HIPCHK(h, hipStreamSynchronize(h->stream));
+    std::copy(both.begin(), both.begin() + n, e2e);
+    std::copy(both.begin() + n, both.end(), com);
+    return SC_OK;
+  }
   if (e2e)
     HIPCHK(h, hipMemcpyAsync(e2e, buf, sizeof(double) * n, hipMemcpyDeviceToHost, h->stream));
   if (com)
@@ -1953,7 +1971,10 @@ int sc_theta_histogram(sc_handle h, int32_t n_bins, int32_t n_rows, int64_t *his
   unsigned long long *buf = reinterpret_cast<unsigned long long *>(idle_scratch(h));
   if (own) HIPCHK(h, hipMalloc(&buf, sizeof(unsigned long long) * n));
   std::vector<unsigned long long> host(n);
-  sc::launch_zero_i32(reinterpret_cast<int32_t *>(buf), 2 * (int64_t)n, h->stream);
+  if (own)
+    (void)hipMemsetAsync(buf, 0, sizeof(unsigned long long) * n, h->stream);
+  else
+    sc::launch_zero_i32(reinterpret_cast<int32_t *>(buf), 2 * (int64_t)n, h->stream);
   sc::launch_theta_hist(h->d, h->g, n_bins, n_rows, buf, h->stream);
   hipError_t e = hipGetLastError();
   if (e == hipSuccess)
