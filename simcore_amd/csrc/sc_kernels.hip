@@ -1185,6 +1185,16 @@ static inline unsigned one_blocks(const Geo &g, int block) {
   return (unsigned)std::min<int64_t>(std::max<int64_t>(b, 1), 256);
 }
 
+// Blocks of a batch up to which its members rebuild in one launch.  The chip
+// holds 256 of 1024 threads or 512 of 512 at once: with more, also a step on
+// which nobody rebuilds takes a round of blocks after the other (about 3 us
+// each), and members wait for blocks that find no room.  us a step of the
+// batch, seven launches / one, and the one's blocks: 16 x 10k bonds 87.5 / 79.6
+// with 576, 8 x 31k 88.5 / 85.4 with 624, 8 x 50k 102.9 / 95.7 with 496, 12 x
+// 50k 118.8 / 115.8 with 744, 8 x 40k 98.1 / 100.2 with 808, 24 x 50k 175 / 194
+// with 1488, 8 x 87k 126 / 156 with 872, 16 x 87k 193 / 285 with 1744.
+constexpr int32_t kBatchBlocks = 768;
+
 // The block that leaves last: until then a block that comes late must still
 // find the rebuild decided as the others did, or it would leave uncounted; so
 // what the decision is taken from -- the displacement slots, Ctl's abort word
@@ -1419,11 +1429,11 @@ void launch_group_rebuild(const Member *dm, const Member *hm, int n, bool fold, 
     one = one && hm[m].g.one_launch;
     small = small && hm[m].g.nb <= kSmallBonds;
   }
-  if (one) {
-    GroupGrid go;
-    const int32_t to = group_grid(go, hm, n, [small](const Geo &g) {
-      return one_blocks(g, small ? 512 : 1024);
-    });
+  GroupGrid go;
+  const int32_t to = group_grid(go, hm, n, [small](const Geo &g) {
+    return one_blocks(g, small ? 512 : 1024);
+  });
+  if (one && to <= kBatchBlocks) {
     if (small && fold)
       hipLaunchKernelGGL((k_group_rebuild_one<512, true>), dim3(to), dim3(512), 0, st, dm, go);
     else if (small)
