@@ -237,8 +237,8 @@ int sc_checkpoint_load(sc_handle h, const void *buf, size_t size);
  *   pair_block          pair kernel threads per block, 64/128/256/512; 0
  *                       selects the load-balanced variant (one wave per 16-64
  *                       bonds, incidences dealt evenly over its lanes).  A
- *                       handle that was given no shape uses 0, or 256 while
- *                       its lists are long
+ *                       handle that was given no shape says 0 and uses that
+ *                       variant, or blocks of 256 while its lists are long
  *   pair_xcd            1: consecutive bond ranges on one XCD
  *   integrate_waves     integrator waves per block, 1/2/4
  *   integrate_layout    filaments of up to 64 sites: one (0) or two (1)

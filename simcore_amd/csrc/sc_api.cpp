@@ -304,21 +304,6 @@ int write_ctl(sc_system *h, const Ctl &c) {
   return SC_OK;
 }
 
-// Mean length of a bond's list up to which the balanced pair kernel is the
-// faster one.  Its lanes evaluate 128 entries and then each bond's lane adds
-// up the bond's, so with long lists a few lanes add while the others wait;
-// the per-bond kernel has every lane at its own list, all of about the same
-// length, but needs enough bonds to fill the chip.  us a pass, balanced /
-// per bond with 256 threads, by mean length: 4k bonds 65: 100 / 130, 151: 222
-// / 260, 317: 425 / 424; 50k 64: 142 / 184, 100: 243 / 231; 100k 27: 111 / 144,
-// 52: 204 / 189, 103: 473 / 303; 200k 35: 209 / 214, 52: 359 / 317; 600k 50:
-// 717 / 806, 101: 1834 / 1580.  Just above 131072 bonds, where a wavefront
-// takes 64 of them, they are too few to fill the chip: at 150k equal at 19 and
-// 1.28 times the time at 32.  FP64's lines lie up to a fifth lower.
-double longest_balanced(int64_t nb) {
-  return nb <= 32768 ? 160.0 : nb <= 65536 ? 80.0 : nb <= 131072 ? 32.0 : nb < 200000 ? 16.0 : 40.0;
-}
-
 // The launches that depend on the lists, the stream idle and ctl_host current:
 // the rebuild stage's, and the pair kernel's if the caller chose none.  They
 // change no result.  The lists have to get a quarter shorter again before a
@@ -328,7 +313,7 @@ void fit_launches(sc_system *h) {
   const double mean = 2.0 * (double)h->ctl_host->nc / (double)h->g.nb;
   const int one = sc::rebuild_in_one(h->g, mean, h->g.one_launch != 0) ? 1 : 0;
   int bal = h->tune.pair_bal;
-  if (!h->shape_given) bal = mean <= longest_balanced(h->g.nb) * (bal ? 1.0 : 0.75) ? 1 : 0;
+  if (!h->shape_given) bal = sc::pair_balanced(h->g.nb, mean, bal != 0) ? 1 : 0;
   if (one == h->g.one_launch && bal == h->tune.pair_bal) return;
   h->g.one_launch = one;
   h->tune.pair_bal = bal;
@@ -2377,7 +2362,8 @@ int sc_get_launch_shape(sc_handle h, sc_launch_shape *shape) {
   if (rc) return rc;
   if (!shape) return fail(h, SC_ERR_ARG, "null launch shape");
   const sc::Tune &t = h->tune;
-  shape->pair_block = t.pair_bal ? 0 : t.pair_block;
+  // (0 also stands for the library's choice)
+  shape->pair_block = t.pair_bal || !h->shape_given ? 0 : t.pair_block;
   shape->pair_xcd = t.pair_xcd;
   shape->integrate_waves = t.int_waves;
   shape->integrate_layout = t.int_layout;

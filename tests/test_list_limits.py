@@ -1,6 +1,7 @@
 """Candidate lists that no capacity holds are refused: the sums of list
 lengths, kept in 32 bits per block of bonds, never come out as a total that
-fits, and the capacity asked for is then past the limit."""
+fits, and the capacity asked for is then past the limit.  And the length from which a handle without a caller's launch
+shape leaves the balanced pair kernel, and comes back to it."""
 import ctypes
 import os
 import subprocess
@@ -50,3 +51,13 @@ def test_limit_itself(lib):
     assert lib.grown_capacity(limit // 2, limit) == limit
     assert lib.candidates_of(lib.kept_length(2**40)) == limit + 1
     assert lib.grown_capacity(limit, limit + 1) == limit + 1
+
+
+@pytest.mark.parametrize("nb, line", [(2, 160), (32768, 160), (32769, 80), (65536, 80), (65537, 32),
+                                      (131072, 32), (131073, 16), (199999, 16), (200000, 40),
+                                      (2000000, 40)])
+def test_pair_kernel_by_length(lib, nb, line):
+    asked = lambda mean, now: lib.pair_balanced(ctypes.c_int64(nb), ctypes.c_double(mean), now)
+    assert asked(0.0, 0) and asked(0.0, 1)
+    assert asked(line, 1) and not asked(line * 1.001, 1)
+    assert asked(0.75 * line, 0) and not asked(0.75 * line * 1.001, 0)
