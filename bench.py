@@ -300,14 +300,27 @@ def pmc_summary(root, tag, copy_bytes):
                       "write_scale": out["WRITE_SIZE_scale"]}), flush=True)
 
 
+def pair_kernel(balanced, precision, nb):
+    """Name of the pair kernel without stress sums; the balanced one's last
+    argument is the bonds of a wavefront (pair_bonds in sc_pair.hip)."""
+    mixed = "true" if precision == "mixed" else "false"
+    if not balanced:
+        return f"k_pair_fused<{mixed}, false>"
+    bonds = 64 if nb > 131072 else 32 if nb > 65536 else 16
+    return f"k_pair_bal<{mixed}, false, {bonds}>"
+
+
 def measured_traffic(tag, kernel):
+    """Measured bytes of a launch of `kernel`, whose last template arguments
+    may be left out; None without a measurement."""
     path = os.path.join(ROOT, "profiles", f"traffic_{tag}.json")
     if not os.path.exists(path):
         return None
     with open(path) as fh:
         d = json.load(fh)
     for k, e in d.get("kernels", {}).items():
-        if k.endswith(kernel) and "traffic_bytes" in e:
+        name = k.split("::")[-1]
+        if (name == kernel or name.startswith(kernel[:-1] + ", ")) and "traffic_bytes" in e:
             return e["traffic_bytes"]
     return None
 
@@ -469,8 +482,7 @@ def main():
     log(f"[bench] profile: {json.dumps(prof)} nc={nc} pair back-to-back {pair_warm_ms:.5f} ms")
     balanced = int(dev.launch_shape()["pair_block"]) == 0
     tune_layout = int(dev.launch_shape()["integrate_layout"])
-    kname = ("k_pair_bal" if balanced else "k_pair_fused") + (
-        "<true, false>" if args.precision == "mixed" else "<false, false>")
+    kname = pair_kernel(balanced, args.precision, fil.nb)
     ttag = f"{TRAFFIC_TAG[args.workload]}_{args.precision}" if args.workload in TRAFFIC_TAG else None
     # the pair pass: the step's largest single kernel on the uneven-length
     # system and the kernel the HBM target names
