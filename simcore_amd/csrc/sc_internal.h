@@ -329,9 +329,11 @@ void launch_cells_from_keys(const Dev &d, const Geo &g, hipStream_t st);
 // `thermo`: also sum the pair stress and the bond energies (Geo::thermo)
 void launch_pair(const Dev &d, const Geo &g, int precision, const Tune &t,
                  hipStream_t st, bool thermo);
+// bonds of a wavefront of the balanced pair kernel
 int pair_bonds(int64_t nb, bool thermo);
+// the pair pass of bonds [b_lo, b_hi)
 void launch_pair_range(const Dev &d, const Geo &g, int precision, const Tune &t, hipStream_t st,
-                       bool thermo, int64_t b_lo, int64_t b_hi);  // blocks of one pair launch
+                       bool thermo, int64_t b_lo, int64_t b_hi);
 // `mid`: the step is a midstep (odd step index)
 void launch_integrate(const Dev &d, const Geo &g, const BinDesc &bin, int precision,
                       const Tune &t, bool mid, hipStream_t st);

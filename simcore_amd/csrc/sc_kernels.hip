@@ -1087,12 +1087,11 @@ __device__ __forceinline__ void pull_body(const Dev &d, const Geo &g, int64_t bi
   // the incidence starts of the block's groups, before the walk over them (in
   // one loop with it they cost the walk 22 registers, two waves per SIMD)
   if (SUMS) {
-    for (int grp0 = (int)bid * kSubs; grp0 < (int)ngrp; grp0 += (int)nblk * kSubs) {
-      const int grp = grp0 + sub;
+    static_assert(!SUMS || BLOCK == 256, "a group per block");
+    for (int grp = (int)bid; grp < (int)ngrp; grp += (int)nblk) {
       const int64_t b = (int64_t)grp * kPullGroup + t;
       const int sup = grp / kSuper;
-      int32_t ahead =
-          sup * kSuper + t < grp && grp < (int)ngrp ? d.scan_tmp[nsup + sup * kSuper + t] : 0;
+      int32_t ahead = sup * kSuper + t < grp ? d.scan_tmp[nsup + sup * kSuper + t] : 0;
       for (int i = t; i < sup; i += 256) ahead += d.scan_tmp[i];
       const int32_t base = block_sum<256>(ahead, ws);
       int gtot;
@@ -1308,8 +1307,9 @@ void launch_rebuild(const Dev &d, const Geo &g, bool fold, hipStream_t st) {
 
 // Ensemble batches: the launches of launch_rebuild, each over all members
 // (odd-step pointers: a rebuild only ever starts an odd step); a member
-// that does not rebuild returns at its guard.  Per member, the same grid as
-// its own launch.
+// that does not rebuild returns at its guard.  Threads of a block and bonds of
+// a wavefront follow from the whole batch, so a member's grid need not be that
+// of its own launch; no kernel's results depend on its grid.
 template <bool FOLD>
 __global__ __launch_bounds__(kScanBlock) void k_group_keys(const Member *__restrict__ ms,
                                                            GroupGrid gg) {
