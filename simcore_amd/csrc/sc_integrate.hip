@@ -18,9 +18,9 @@
 //
 // Bound: the latency of those chains (about 100 clocks a Thomas row, most of
 // it the division) and, for large systems, instruction issue.  Measured, full
-// step and midstep: 925 x 8 filaments of 8-256 sites (229k bonds) 58 and 69 us
+// step and midstep: 925 x 8 filaments of 8-256 sites (229k bonds) 52 and 64 us
 // where the six launches, one per bin, with chains branching and loading row
-// by row took 190 and 260; 5000 filaments of 32 sites 28 and 31 us (31, 40).
+// by row took 190 and 260; 5000 filaments of 32 sites 27 and 29 us (31, 40).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
